@@ -28,4 +28,29 @@ struct QkvArgs {
 // registers); returns PDM_ERR_UNSUPPORTED for other widths.
 int launch_qkv_stationary(const QkvArgs& a, int D, hipStream_t s);
 
+// Row projection (row_proj.hip): out = epilogue(bf16(RMSNorm(x)) . W^T) for fp32 rows (b, t) of D columns.  S tokens
+// (t < n_s) use W, NS token n_s + g uses W_ns[g].
+enum { ROWPROJ_QKV = 0, ROWPROJ_GELU = 1 };
+struct RowProjArgs {
+  const float* x;        // row (b, t) at x + b * in_bstride + t * D
+  int64_t in_bstride;
+  const float* norm_w;   // RMSNorm weight [D]
+  const uint16_t* W;     // [N, D]
+  const uint16_t* W_ns;  // [n_ns, N, D], or null when n_ns == 0
+  int B, n_s, n_ns, N;
+  // ROWPROJ_GELU: out row (b, t) at out + b * out_bstride + t * N; the normalised bf16 rows are also left in h (the
+  // layout of x)
+  uint16_t* h;
+  uint16_t* out;
+  int64_t out_bstride;
+  // ROWPROJ_QKV (N = 3D): as QkvArgs
+  uint16_t* q;
+  uint16_t* k;
+  uint16_t* vt;
+  int kv, q_len, kv_pad;
+  // filled by the launcher
+  int blocks_per_sample, tiles_per_token, wgs_s, wgs_ns, split_s, split_ns;
+};
+int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s);
+
 }  // namespace pdm

@@ -16,16 +16,14 @@
 // is not rounded to bf16 before the residual addition (at most half a bf16
 // ulp of the FFN output away from the autocast result).
 //
-// Launches per block: rmsnorm, QKV GEMM (writes Q tail rows, K, and V
-// transposed per head), attention, out-proj GEMM (+x tail -> z in y),
-// rmsnorm, FFN-up GEMM (+GELU), FFN-down GEMM (+z -> y).
+// Launches per block: Q/K/V projection with RMSNorm1 in front (Q tail rows, K, and V transposed per head), attention,
+// then either out-projection + FFN in one kernel (d_model 128 / 256) or out-projection GEMM (+x tail -> z in y),
+// FFN-up with RMSNorm2 in front (row_proj.hip), FFN-down GEMM (+z -> y).
 //
-// GEMM design: C[128x128] tiles of A[M,K] . W[N,K]^T (both K-contiguous, the
-// nn.Linear layout), 4 waves in a 2x2 arrangement, each wave 2x2
-// v_mfma_f32_32x32x16_bf16 tiles, K streamed in 64-wide slices through a
-// double-buffered LDS ring.  Rows are (sample, token) pairs; S-token rows use
-// the shared weight and NS-token rows the weight of their token, so one
-// launch covers the shared GEMM and the 16 per-token GEMMs.
+// GEMM design (out-projection, FFN-down of d_model 384 / 512): tiles of A[M,K] . W[N,K]^T (both K-contiguous, the
+// nn.Linear layout), each wave 2x2 v_mfma_f32_32x32x16_bf16 tiles, K streamed in 64-wide slices through LDS.  Rows are
+// (sample, token) pairs; S-token rows use the shared weight and NS-token rows the weight of their token, so one launch
+// covers the shared GEMM and the 16 per-token GEMMs.
 //
 // Attention design: one wave owns 32 queries of one (sample, head).  It
 // computes S^T = K Q^T so that each lane holds one query's scores; the
@@ -48,57 +46,9 @@
 namespace pdm {
 
 // ---------------------------------------------------------------------------
-// RMSNorm -> bf16 rows.  One wave per row, D = 64 * VPL.
-// out row r = bf16((x * rsqrt(mean(x^2) + eps)) * w), fp32 arithmetic in the
-// reference's order (onetrans.py:80-82).
-// ---------------------------------------------------------------------------
-template <int VPL>
-__global__ __launch_bounds__(256) void rmsnorm_bf16_kernel(const float* __restrict__ x, int64_t x_bstride,
-                                                           int T, int64_t rows, const float* __restrict__ w,
-                                                           uint16_t* __restrict__ out, float eps) {
-  constexpr int D = 64 * VPL;
-  const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (r >= rows) return;
-  const int64_t b = r / T;
-  const int t = (int)(r - b * T);
-  const float* xr = x + b * x_bstride + (int64_t)t * D + lane * VPL;
-  float v[VPL];
-  if constexpr (VPL % 4 == 0) {
-#pragma unroll
-    for (int i = 0; i < VPL / 4; ++i) {
-      const float4 f = reinterpret_cast<const float4*>(xr)[i];
-      v[4 * i] = f.x; v[4 * i + 1] = f.y; v[4 * i + 2] = f.z; v[4 * i + 3] = f.w;
-    }
-  } else if constexpr (VPL % 2 == 0) {
-#pragma unroll
-    for (int i = 0; i < VPL / 2; ++i) {
-      const float2 f = reinterpret_cast<const float2*>(xr)[i];
-      v[2 * i] = f.x; v[2 * i + 1] = f.y;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < VPL; ++i) v[i] = xr[i];
-  }
-  float ss = 0.0f;
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) ss += v[i] * v[i];
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) ss += __shfl_xor(ss, s, 64);
-  const float rms = 1.0f / sqrtf(ss / (float)D + eps);
-  uint16_t* o = out + r * D + lane * VPL;
-#pragma unroll
-  for (int i = 0; i < VPL; ++i) {
-    const float wv = w[lane * VPL + i];
-    const float n = v[i] * rms;
-    o[i] = (uint16_t)bf16_bits(n * wv);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Grouped GEMM  C = A . W^T  over (sample, token) rows.
 // ---------------------------------------------------------------------------
-enum { EPI_BF16 = 0, EPI_QKV = 1, EPI_RESID = 2, EPI_GELU = 3, EPI_BIAS_GELU = 4, EPI_BIAS_F32 = 5 };
+enum { EPI_BIAS_GELU = 0, EPI_BIAS_F32 = 1 };
 
 constexpr int GBM = 128, GBN = 128, GBK = 64, GPAD = 8;
 
@@ -116,61 +66,28 @@ struct GemmArgs {
   int n_tiles;  // ceil(N / GBN)
   int64_t total_blocks;
   // epilogue
-  void* out;            // EPI_BF16 / EPI_GELU: bf16 [B, T, N]; EPI_RESID: fp32 [B, T, N]
+  void* out;            // bf16 (EPI_BIAS_GELU) or fp32 [B, T, N]
   int64_t out_bstride;  // elements between samples of out
-  const float* res;     // EPI_RESID: residual fp32, row (b, t) at res + b * res_bstride + (t + res_toff) * N
+  const float* res;     // residual fp32, row (b, t) at res + b * res_bstride + (t + res_toff) * N
   int64_t res_bstride;
   int res_toff;
-  // EPI_QKV: N = 3D.  Q [B, q_len, D] (tokens t >= kv - q_len), K [B, kv, D], VT [B, H, 64, kv_pad]
-  uint16_t* q;
-  uint16_t* k;
-  uint16_t* vt;
-  int kv, q_len, kv_pad, D;  // kv_pad: V^T row stride
-  // row-stationary kernels: fp32 A rows normalised on load (RMSNorm weight norm_w), FFN weights
-  const float* A32;
-  const float* norm_w;
+  int D;
+  // the fused FFN
+  const float* norm_w;    // RMSNorm2 weight
   const uint16_t* W2;     // FFN-down [D, F] shared
   const uint16_t* W2_ns;  // [n_ns, D, F]
   const uint16_t* bias;   // EPI_BIAS_*: bf16 [N]
   const uint16_t* Wo;     // FFN with the out-projection in front: Wout [D, D], shared by every token
 };
 
-// Stores one GEMM output element (b, t, n) with the epilogue EPI.
+// Stores one output element (b, t, n) of a Linear with bias (one rounding after the bias, as autocast makes it): its
+// GELU in bf16, or the bf16 result as fp32 (the promotion of the token concat).
 template <int EPI>
 __device__ __forceinline__ void epilogue_store(const GemmArgs& a, int b, int t, int n, float v) {
-  if constexpr (EPI == EPI_BF16) {
-    reinterpret_cast<uint16_t*>(a.out)[(int64_t)b * a.out_bstride + (int64_t)t * a.N + n] =
-        (uint16_t)bf16_bits(v);
-  } else if constexpr (EPI == EPI_GELU) {
-    reinterpret_cast<uint16_t*>(a.out)[(int64_t)b * a.out_bstride + (int64_t)t * a.N + n] =
-        (uint16_t)bf16_bits(gelu_erf(bf16_round(v)));
-  } else if constexpr (EPI == EPI_BIAS_GELU) {
-    // autocast Linear with bias (one rounding after the bias), then GELU on the bf16 value, rounded to bf16
-    const float x = bf16_round(v + bf16_bits_to_f32(a.bias[n]));
-    reinterpret_cast<uint16_t*>(a.out)[(int64_t)b * a.out_bstride + (int64_t)t * a.N + n] =
-        (uint16_t)bf16_bits(gelu_erf(x));
-  } else if constexpr (EPI == EPI_BIAS_F32) {
-    // autocast Linear with bias, its bf16 result stored as fp32 (the promotion of the token concat)
-    reinterpret_cast<float*>(a.out)[(int64_t)b * a.out_bstride + (int64_t)t * a.N + n] =
-        bf16_round(v + bf16_bits_to_f32(a.bias[n]));
-  } else if constexpr (EPI == EPI_RESID) {
-    const float r = a.res[(int64_t)b * a.res_bstride + (int64_t)(t + a.res_toff) * a.N + n];
-    reinterpret_cast<float*>(a.out)[(int64_t)b * a.out_bstride + (int64_t)t * a.N + n] = bf16_round(v) + r;
-  } else {  // EPI_QKV
-    const uint16_t bits = (uint16_t)bf16_bits(v);
-    const int D = a.D;
-    if (n < D) {
-      const int tq = t - (a.kv - a.q_len);
-      if (tq >= 0) a.q[((int64_t)b * a.q_len + tq) * D + n] = bits;
-    } else if (n < 2 * D) {
-      a.k[((int64_t)b * a.kv + t) * D + (n - D)] = bits;
-    } else {
-      const int c = n - 2 * D;
-      const int h = c >> 6, d = c & 63;
-      const int H = D >> 6;
-      a.vt[(((int64_t)b * H + h) * 64 + d) * a.kv_pad + t] = bits;
-    }
-  }
+  const int64_t o = (int64_t)b * a.out_bstride + (int64_t)t * a.N + n;
+  const float x = bf16_round(v + bf16_bits_to_f32(a.bias[n]));
+  if constexpr (EPI == EPI_BIAS_GELU) reinterpret_cast<uint16_t*>(a.out)[o] = (uint16_t)bf16_bits(gelu_erf(x));
+  else reinterpret_cast<float*>(a.out)[o] = x;
 }
 
 // (sample, token) of row i of GEMM row tile mt, or b = -1 past the end.  Tiles
@@ -236,21 +153,13 @@ constexpr int kGemmStages = PDM_GEMM_STAGES;
 #ifndef PDM_GEMM_TM
 #define PDM_GEMM_TM 256
 #endif
-// PDM_GEMM_STAGED_EPI: the residual and GELU epilogues write 64-row slices of the tile through LDS as
-// 16-byte / 8-byte row segments
-#ifndef PDM_GEMM_STAGED_EPI
-#define PDM_GEMM_STAGED_EPI 1
-#endif
-
-template <int EPI, int TM>
+template <int TM>
 __global__ __launch_bounds__(TM * 2, kGemmStages == 1 ? (TM == GBM ? PDM_GEMM_WPS : 4) : 2) void gemm_kernel(GemmArgs a) {
   constexpr int NT = TM * 2;                 // threads: TM / 64 x 2 waves
   constexpr int RPP = NT / 8;                // tile rows per pass of 16-byte loads
   constexpr int PA = TM / RPP, PB = GBN / RPP;  // passes of the A and W tiles
-  // the A and W tiles; after the k loop the Q/K/V epilogue stages V^T (128 x 136 bf16 per 128 rows) in the
-  // same bytes
+  // the A and W tiles; after the k loop the epilogue stages its rows in the same bytes
   constexpr int kAElems = kGemmStages * TM * (GBK + GPAD), kBElems = kGemmStages * GBN * (GBK + GPAD);
-  static_assert(kAElems + kBElems >= GBN * (GBM + 8), "the V^T staging tile must fit in the A and W tiles");
   __shared__ __attribute__((aligned(16))) uint16_t sAB[kAElems + kBElems];
   uint16_t (*sA)[TM][GBK + GPAD] = reinterpret_cast<uint16_t (*)[TM][GBK + GPAD]>(sAB);
   uint16_t (*sB)[GBN][GBK + GPAD] = reinterpret_cast<uint16_t (*)[GBN][GBK + GPAD]>(sAB + kAElems);
@@ -273,15 +182,6 @@ __global__ __launch_bounds__(TM * 2, kGemmStages == 1 ? (TM == GBM ? PDM_GEMM_WP
   if (tid < TM) tile_row(a, mt, TM, tid, s_rb[tid], s_rt[tid]);
   if (mt >= a.tiles_s) W = a.W_ns + (int64_t)((mt - a.tiles_s) / a.tiles_b) * a.N * a.K;
   __syncthreads();
-
-  if constexpr (EPI == EPI_QKV) {
-    // Q columns of S-token rows outside the kept tail are never read: skip the tile
-    if (n0 < a.D) {
-      const int thr = a.kv - a.q_len;
-      const int need = (tid < TM && s_rb[tid] >= 0 && s_rt[tid] >= thr) ? 1 : 0;
-      if (!__syncthreads_or(need)) return;
-    }
-  }
 
   // global -> LDS assignment: 8 threads x 16 B per 64-element row slice, RPP rows per pass.  Rows are 32-bit
   // element offsets from the tile's first row (-1: no row), which launch_gemm bounds.
@@ -356,567 +256,40 @@ __global__ __launch_bounds__(TM * 2, kGemmStages == 1 ? (TM == GBM ? PDM_GEMM_WP
 
   // epilogue: acc[i][j][e] is row wm*64 + i*32 + (e/4)*8 + (lane/32)*4 + e%4, column n0 + wn*64 + j*32 + lane%32
   const int hf = lane >> 5;
-  if constexpr (EPI == EPI_QKV) {
-    if (n0 >= 2 * a.D) {
-      // a V tile (2 D is a multiple of 128): V^T rows (b, h, d) are contiguous in t, so the tile goes through
-      // LDS transposed, sT[column][row], and each thread stores 8 consecutive rows of one column (consecutive t
-      // of one sample) with one 16-byte store, or two 8-byte stores where t is a multiple of 4 but not of 8;
-      // 16 lanes cover the 128 rows of a column.  Runs of 8 rows that are not 8 consecutive tokens of one
-      // sample (sample boundaries, the NS groups, padding rows) store element by element.  The k loop ended
-      // with a barrier.  128 rows at a time (TM / 128 rounds).
-      constexpr int TS = GBM + 8;  // sT row stride (bf16)
-      uint16_t* sT = sAB;
-      const int H = a.D >> 6;
+  // 64 rows at a time through LDS (fp32, rows of 128 + 4): the two waves that hold them write their accumulators,
+  // then every thread finishes 4 consecutive outputs of a row with one 16-byte residual read and one 16-byte store.
+  // The k loop ended with a barrier.  N = d_model is a multiple of 128.
+  constexpr int OS = GBN + 4;  // sO row stride (floats)
+  static_assert((kAElems + kBElems) * 2 >= 64 * OS * 4, "the staging rows must fit in the A and W tiles");
+  float* sO = reinterpret_cast<float*>(sAB);
 #pragma unroll
-      for (int hv = 0; hv < TM / GBM; ++hv) {
-        if (wm / 2 == hv) {
+  for (int rr = 0; rr < TM / 64; ++rr) {
+    if (wm == rr) {
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-              for (int e = 0; e < 16; e += 2) {
-                const int row = (wm & 1) * 64 + i * 32 + (e >> 2) * 8 + hf * 4 + (e & 3);
-                const int col = wn * 64 + j * 32 + fr;
-                *reinterpret_cast<uint32_t*>(sT + col * TS + row) = pack_bf16x2(acc[i][j][e], acc[i][j][e + 1]);
-              }
-        }
-        __syncthreads();
-        static_assert(GBN * (GBM / 8) % NT == 0, "pieces per thread");
-#pragma unroll 1
-        for (int it = 0; it < GBN * (GBM / 8) / NT; ++it) {
-          const int idx = it * NT + tid;
-          const int col = idx >> 4, r0 = (idx & 15) * 8;
-          if (n0 + col >= a.N) continue;
-          const int c = n0 + col - 2 * a.D;
-          const int h = c >> 6, d = c & 63;
-          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(sT + col * TS + r0);
-          const int rr = hv * GBM + r0;
-          const int b = s_rb[rr], t = s_rt[rr];
-          if (b >= 0 && s_rb[rr + 7] == b && s_rt[rr + 7] == t + 7 && (t & 3) == 0 && (a.kv_pad & 7) == 0) {
-            uint16_t* dst = a.vt + (((int64_t)b * H + h) * 64 + d) * a.kv_pad + t;
-            if ((t & 7) == 0) {
-              *reinterpret_cast<u32x4_t*>(dst) = v;
-            } else {
-              *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{v[0], v[1]};
-              *reinterpret_cast<u32x2_t*>(dst + 4) = u32x2_t{v[2], v[3]};
-            }
-          } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const int be = s_rb[rr + e];
-              if (be >= 0)
-                a.vt[(((int64_t)be * H + h) * 64 + d) * a.kv_pad + s_rt[rr + e]] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
-            }
-          }
-        }
-        __syncthreads();  // sT is read before the next round writes it
-      }
-      return;
+          for (int e = 0; e < 16; ++e)
+            sO[(i * 32 + (e >> 2) * 8 + hf * 4 + (e & 3)) * OS + wn * 64 + j * 32 + fr] = acc[i][j][e];
     }
-  }
-#if PDM_GEMM_STAGED_EPI
-  if constexpr (EPI == EPI_RESID || EPI == EPI_GELU || EPI == EPI_QKV) {
-    // (the Q/K/V GEMM's V tiles returned above: here its tiles are all Q or all K columns, D being a multiple
-    // of 128)
-    if (n0 + GBN <= a.N && (a.N & 7) == 0) {
-      // 64 rows at a time through LDS (fp32, rows of 128 + 4): the two waves that hold them write their
-      // accumulators, then every thread finishes VPT consecutive outputs of a row: 4 fp32 with one 16-byte
-      // residual read and one 16-byte store, or 8 bf16 with one 16-byte store.  The k loop ended with a barrier.
-      constexpr int OS = GBN + 4;  // sO row stride (floats)
-      constexpr int VPT = EPI == EPI_RESID ? 4 : 8;
-      static_assert((kAElems + kBElems) * 2 >= 64 * OS * 4, "the staging rows must fit in the A and W tiles");
-      float* sO = reinterpret_cast<float*>(sAB);
-      // GELU: the table of gelu_lut after the staging rows, filled once here (published by the first round's
-      // barrier, only read afterwards)
-      constexpr bool kLut = EPI == EPI_GELU && (kAElems + kBElems) * 2 >= (64 * OS + GELU_T_N) * 4;
-      float* const sG = sO + 64 * OS;
-      if constexpr (kLut) gelu_table_fill(sG, tid, NT);
+    __syncthreads();
 #pragma unroll
-      for (int rr = 0; rr < TM / 64; ++rr) {
-        if (wm == rr) {
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-              for (int e = 0; e < 16; ++e)
-                sO[(i * 32 + (e >> 2) * 8 + hf * 4 + (e & 3)) * OS + wn * 64 + j * 32 + fr] = acc[i][j][e];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int it = 0; it < 64 * (GBN / VPT) / NT; ++it) {
-          const int idx = it * NT + tid;
-          const int rl = idx / (GBN / VPT), cv = idx % (GBN / VPT);
-          const int row = rr * 64 + rl;
-          const int b = s_rb[row];
-          if (b < 0) continue;
-          const int t = s_rt[row];
-          const int n = n0 + cv * VPT;
-          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(sO + rl * OS + cv * VPT);
-          if constexpr (EPI == EPI_RESID) {
-            const f32x4_t r = *reinterpret_cast<const f32x4_t*>(
-                a.res + (int64_t)b * a.res_bstride + (int64_t)(t + a.res_toff) * a.N + n);
-            *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + (int64_t)b * a.out_bstride +
-                                        (int64_t)t * a.N + n) =
-                f32x4_t{bf16_round(v[0]) + r[0], bf16_round(v[1]) + r[1], bf16_round(v[2]) + r[2],
-                        bf16_round(v[3]) + r[3]};
-          } else {
-            const f32x4_t v2 = *reinterpret_cast<const f32x4_t*>(sO + rl * OS + cv * VPT + 4);
-            uint16_t* dst;
-            u32x4_t w;
-            if constexpr (EPI == EPI_QKV) {
-              if (n < a.D) {
-                const int tq = t - (a.kv - a.q_len);
-                if (tq < 0) continue;  // Q of a row outside the kept tail is never read
-                dst = a.q + ((int64_t)b * a.q_len + tq) * a.D + n;
-              } else {
-                dst = a.k + ((int64_t)b * a.kv + t) * a.D + (n - a.D);
-              }
-              w = u32x4_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v2[0], v2[1]),
-                          pack_bf16x2(v2[2], v2[3])};
-            } else {
-              dst = reinterpret_cast<uint16_t*>(a.out) + (int64_t)b * a.out_bstride + (int64_t)t * a.N + n;
-              if constexpr (kLut) {
-                const float u8[8] = {v[0], v[1], v[2], v[3], v2[0], v2[1], v2[2], v2[3]};
-                uint32_t gw[4];
-                gelu_lut_pack<8>(sG, u8, gw);
-                w = u32x4_t{gw[0], gw[1], gw[2], gw[3]};
-              } else {
-                auto g2 = [](float x0, float x1) {
-                  return (uint32_t)bf16_bits(gelu_erf(bf16_round(x0))) |
-                         ((uint32_t)bf16_bits(gelu_erf(bf16_round(x1))) << 16);
-                };
-                w = u32x4_t{g2(v[0], v[1]), g2(v[2], v[3]), g2(v2[0], v2[1]), g2(v2[2], v2[3])};
-              }
-            }
-            *reinterpret_cast<u32x4_t*>(dst) = w;
-          }
-        }
-        __syncthreads();  // sO is read before the next round writes it
-      }
-      return;
-    }
-  }
-#endif
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int row = wm * 64 + i * 32 + (e >> 2) * 8 + hf * 4 + (e & 3);
+    for (int it = 0; it < 64 * (GBN / 4) / NT; ++it) {
+      const int idx = it * NT + tid;
+      const int rl = idx / (GBN / 4), cv = idx % (GBN / 4);
+      const int row = rr * 64 + rl;
       const int b = s_rb[row];
       if (b < 0) continue;
       const int t = s_rt[row];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = n0 + wn * 64 + j * 32 + fr;
-        if (n >= a.N) continue;
-        epilogue_store<EPI>(a, b, t, n, acc[i][j][e]);
-      }
+      const int n = n0 + cv * 4;
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(sO + rl * OS + cv * 4);
+      const f32x4_t r = *reinterpret_cast<const f32x4_t*>(
+          a.res + (int64_t)b * a.res_bstride + (int64_t)(t + a.res_toff) * a.N + n);
+      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + (int64_t)b * a.out_bstride + (int64_t)t * a.N + n) =
+          f32x4_t{bf16_round(v[0]) + r[0], bf16_round(v[1]) + r[1], bf16_round(v[2]) + r[2], bf16_round(v[3]) + r[3]};
     }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Row-stationary GEMM for K = d_model:  out[rows, N] = A[rows, D] . W[N, D]^T.
-//
-// Each wave keeps RB x 32 rows of A for the whole K = D in registers as MFMA
-// A fragments (lane l holds row l%32, k-slots (l/32)*8 .. +8 of every
-// 16-wide k step).  With NORM the rows are fp32 residual-stream rows,
-// normalised on load: a first pass takes the sum of squares (the two lanes of
-// a row each hold half of it), a second re-reads the row (an L2 hit), scales
-// it by rsqrt(mean + eps) and the RMSNorm weight in fp32 and rounds to bf16,
-// exactly the autocast path of the reference (onetrans.py:80-82).  The
-// weight streams global -> LDS (no register staging) through a double
-// buffer in chunks of 32 output columns; each weight fragment read from LDS
-// feeds RB MFMAs.
-// ---------------------------------------------------------------------------
-template <int D, int RB, bool NORM>
-__device__ __forceinline__ void load_row_fragments(const GemmArgs& a, const int* s_rb, const int* s_rt, int wave,
-                                                   int fr, int hf, u32x4_t (&af)[RB][D / 16]) {
-  constexpr int KS = D / 16;
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int row = wave * RB * 32 + rb * 32 + fr;
-    const int b = s_rb[row];
-    if (b < 0) {
-#pragma unroll
-      for (int s = 0; s < KS; ++s) af[rb][s] = u32x4_t{0, 0, 0, 0};
-      continue;
-    }
-    const int64_t base = (int64_t)b * a.a_bstride + (int64_t)s_rt[row] * D + hf * 8;
-    if constexpr (NORM) {
-      const float* xr = a.A32 + base;
-      float ss = 0.0f;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const f32x4_t v0 = *reinterpret_cast<const f32x4_t*>(xr + s * 16);
-        const f32x4_t v1 = *reinterpret_cast<const f32x4_t*>(xr + s * 16 + 4);
-        ss += v0.x * v0.x + v0.y * v0.y + v0.z * v0.z + v0.w * v0.w;
-        ss += v1.x * v1.x + v1.y * v1.y + v1.z * v1.z + v1.w * v1.w;
-      }
-      ss += __shfl_xor(ss, 32, 64);
-      const float rms = 1.0f / sqrtf(ss / (float)D + 1e-6f);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const f32x4_t v0 = *reinterpret_cast<const f32x4_t*>(xr + s * 16);
-        const f32x4_t v1 = *reinterpret_cast<const f32x4_t*>(xr + s * 16 + 4);
-        const f32x4_t w0 = *reinterpret_cast<const f32x4_t*>(a.norm_w + s * 16 + hf * 8);
-        const f32x4_t w1 = *reinterpret_cast<const f32x4_t*>(a.norm_w + s * 16 + hf * 8 + 4);
-        af[rb][s] = u32x4_t{pack_bf16x2((v0.x * rms) * w0.x, (v0.y * rms) * w0.y),
-                            pack_bf16x2((v0.z * rms) * w0.z, (v0.w * rms) * w0.w),
-                            pack_bf16x2((v1.x * rms) * w1.x, (v1.y * rms) * w1.y),
-                            pack_bf16x2((v1.z * rms) * w1.z, (v1.w * rms) * w1.w)};
-      }
-    } else {
-      const uint16_t* ar = reinterpret_cast<const uint16_t*>(a.A) + base;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) af[rb][s] = *reinterpret_cast<const u32x4_t*>(ar + s * 16);
-    }
-  }
-}
-
-// Weight chunks of 32 output columns x D.  Register path (the residual
-// epilogue, whose per-chunk residual loads must not wait for weight loads):
-// a double buffer of rows padded to a stride of 2*D + 16, loaded into
-// registers at the top of a chunk and written to LDS after its MFMAs.  DMA
-// path (the Q/K/V epilogue, whose chunks only store): a 4-stage ring filled by
-// LDS DMA three chunks ahead, rows of 2*D bytes with 16-byte piece v of row r
-// at slot v ^ (r & 15), the chunk loop unrolled by the ring depth.  Either way
-// the 32 rows of one fragment read hit distinct bank groups.
-// Q/K/V GEMM: weight ring depth and workgroups per CU
-#ifndef PDM_QKV_NST
-#define PDM_QKV_NST 4
-#endif
-#ifndef PDM_QKV_WPS
-#define PDM_QKV_WPS 2
-#endif
-template <int D, int RB, int EPI, bool NORM>
-__global__ __launch_bounds__(256, EPI == EPI_QKV ? PDM_QKV_WPS : 2) void rowgemm_kernel(GemmArgs a) {
-  constexpr int KS = D / 16;
-  constexpr int TROWS = 4 * RB * 32;
-  constexpr bool DMA = EPI == EPI_QKV;
-  constexpr int NST = DMA ? PDM_QKV_NST : 2;
-  constexpr int PF = NST - 1;
-  constexpr int CHUNK_BYTES = DMA ? 32 * 2 * D : 32 * w_stride<D>();
-  __shared__ __attribute__((aligned(16))) char sW[NST][CHUNK_BYTES];
-  __shared__ int s_rb[TROWS];
-  __shared__ int s_rt[TROWS];
-  // Q/K/V^T epilogue: each wave's 32 x 32 bf16 output tile goes through LDS (rows of 64 bytes at a stride of
-  // 80, so that the lanes' 8-byte writes of one row group hit distinct banks) and leaves as 16-byte pieces,
-  // four lanes per 64-byte row segment, instead of 8-byte pieces of 32 rows
-  constexpr int SST = 80;
-  // residual epilogue: fp32 tiles through LDS (rows of 128 bytes at a stride of 144), leaving as full
-  // 128-byte row segments, eight lanes per row; the residual is read in the same layout
-  constexpr int RST = 144;
-  __shared__ __attribute__((aligned(16))) char sStage[EPI == EPI_QKV ? 4 * 32 * SST : (EPI == EPI_RESID ? 4 * 32 * RST : 16)];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int fr = lane & 31, hf = lane >> 5;
-  const int mt = blockIdx.x;
-  for (int i = tid; i < TROWS; i += 256) tile_row(a, mt, TROWS, i, s_rb[i], s_rt[i]);
-  const uint16_t* W = mt < a.tiles_s ? a.W : a.W_ns + (int64_t)((mt - a.tiles_s) / a.tiles_b) * a.N * D;
-  __syncthreads();
-
-  int c0 = 0;
-  if constexpr (EPI == EPI_QKV) {
-    // Q columns are needed only for the kept tail tokens
-    int need = 0;
-    for (int i = tid; i < TROWS; i += 256) need |= (s_rb[i] >= 0 && s_rt[i] >= a.kv - a.q_len) ? 1 : 0;
-    if (!__syncthreads_or(need)) c0 = D / 32;
-  }
-  const int nchunks = a.N / 32;
-  constexpr int CPR = D / 8;          // 16-byte pieces per weight row
-  constexpr int WL = 32 * CPR / 256;  // 16-byte pieces per thread of a chunk
-  // register path
-  constexpr int RPP = 256 / CPR;      // chunk rows covered by one piece round
-  const int wr0 = tid / CPR, wp0 = tid - (tid / CPR) * CPR;
-  u32x4_t wr[DMA ? 1 : WL];
-  auto gload = [&](int c) {
-#pragma unroll
-    for (int p = 0; p < WL; ++p)
-      wr[p] = *reinterpret_cast<const u32x4_t*>(W + (int64_t)(c * 32 + p * RPP + wr0) * D + wp0 * 8);
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < WL; ++p)
-      *reinterpret_cast<u32x4_t*>(sW[buf] + (p * RPP + wr0) * w_stride<D>() + wp0 * 16) = wr[p];
-  };
-  // DMA path: LDS piece o of a stage is loaded by thread o mod 256 (round o / 256) from row o / CPR,
-  // logical piece (o mod CPR) ^ (row & 15)
-  uint32_t woff[WL];
-#pragma unroll
-  for (int p = 0; p < WL; ++p) {
-    const int o = p * 256 + tid, r = o / CPR;
-    woff[p] = (uint32_t)((r * D + (((o % CPR) ^ (r & 15)) << 3)) * 2);
-  }
-  auto dma = [&](int c, int stg) {
-    const uint64_t base = (uint64_t)(uintptr_t)W + (uint64_t)c * 32 * D * 2;
-#pragma unroll
-    for (int p = 0; p < WL; ++p) lds_dma16(base, woff[p], (uint32_t)(uintptr_t)(sW[stg] + (p * 256 + wave * 64) * 16));
-  };
-  auto wfrag = [&](const char* wb, int s) -> u32x4_t {
-    if constexpr (DMA)
-      return *reinterpret_cast<const u32x4_t*>(wb + fr * (2 * D) + (((2 * s + hf) ^ (fr & 15)) << 4));
-    else
-      return read_w_frag<D>(wb, fr, 2 * s + hf);
-  };
-  if constexpr (DMA) {
-#pragma unroll
-    for (int j = 0; j < PF; ++j) dma(min(c0 + j, nchunks - 1), j);
-  } else {
-    gload(c0);
-    sstore(0);
-  }
-
-  u32x4_t af[RB][KS];
-  load_row_fragments<D, RB, NORM>(a, s_rb, s_rt, wave, fr, hf, af);
-
-  // Two accumulator layouts, chosen per chunk so that every store writes 4 consecutive outputs:
-  //  rows on lanes (acc = W . A^T): lane fr holds row rb*32 + fr and columns c*32 + (e/4)*8 + hf*4 + e%4
-  //    (Q, K and the residual epilogue: outputs are row-major);
-  //  columns on lanes (acc = A . W^T): lane fr holds column c*32 + fr and rows rb*32 + (e/4)*8 + hf*4 + e%4
-  //    (V, stored transposed as V^T[b, h, d, token]: consecutive tokens are consecutive outputs).
-  // vgrp bit rb*4 + g: rows rb*32 + g*8 + hf*4 .. +3 of this wave are 4 consecutive tokens of one
-  // sample starting at a multiple of 4, so their V^T outputs form one aligned 8-byte store.
-  int vgrp = 0;
-  if constexpr (EPI == EPI_QKV) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int r0 = wave * RB * 32 + rb * 32 + g * 8 + hf * 4;
-        const int b0 = s_rb[r0], t0 = s_rt[r0];
-        bool ok = b0 >= 0 && (t0 & 3) == 0;
-#pragma unroll
-        for (int i = 1; i < 4; ++i) ok = ok && s_rb[r0 + i] == b0 && s_rt[r0 + i] == t0 + i;
-        vgrp |= ok ? 1 << (rb * 4 + g) : 0;
-      }
-  }
-  const int my_row = wave * RB * 32 + fr;  // + rb * 32: this lane's row in the rows-on-lanes layout
-
-  // Staged stores (RB == 1): lane l writes 16-byte piece (l & 3) of tile rows (l >> 2) and 16 + (l >> 2).
-  // Q and K rows of those tile rows (null: no row, or a Q row outside the kept tail); for V^T, vcontig says
-  // the wave's 32 rows are the consecutive tokens t0 .. t0 + 31 of one sample b0 with t0 a multiple of 8, so
-  // a tile row of V^T (one feature, 32 tokens) is one aligned 64-byte segment.
-  constexpr bool STAGE = EPI == EPI_QKV && RB == 1;
-  constexpr bool RSTAGE = EPI == EPI_RESID && RB == 1;
-  // residual staging: lane l handles piece (l & 7) (4 outputs) of tile rows (l >> 3) + 8i, i < 4
-  float* zrow[4] = {nullptr, nullptr, nullptr, nullptr};
-  const float* rrow[4] = {nullptr, nullptr, nullptr, nullptr};
-  if constexpr (RSTAGE) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = wave * 32 + i * 8 + (lane >> 3);
-      const int b = s_rb[r], t = s_rt[r];
-      if (b >= 0) {
-        zrow[i] = reinterpret_cast<float*>(a.out) + (int64_t)b * a.out_bstride + (int64_t)t * a.N + (lane & 7) * 4;
-        rrow[i] = a.res + (int64_t)b * a.res_bstride + (int64_t)(t + a.res_toff) * a.N + (lane & 7) * 4;
-      }
-    }
-  }
-  const int spiece = lane & 3;
-  uint16_t* qrow[2] = {nullptr, nullptr};
-  uint16_t* krow[2] = {nullptr, nullptr};
-  bool vcontig = false;
-  int vb0 = 0, vt0 = 0;
-  char* stage = sStage + (STAGE ? wave * 32 * SST : 0);
-  if constexpr (STAGE) {
-#pragma unroll
-    for (int i2 = 0; i2 < 2; ++i2) {
-      const int r = wave * 32 + i2 * 16 + (lane >> 2);
-      const int b = s_rb[r], t = s_rt[r];
-      if (b >= 0) {
-        krow[i2] = a.k + ((int64_t)b * a.kv + t) * a.D;
-        const int tq = t - (a.kv - a.q_len);
-        if (tq >= 0) qrow[i2] = a.q + ((int64_t)b * a.q_len + tq) * a.D;
-      }
-    }
-    vb0 = s_rb[wave * 32];
-    vt0 = s_rt[wave * 32];
-    // uniform over the wave: every group of 4 rows is contiguous (vgrp) and the groups continue each other
-    bool ok = vb0 >= 0 && (vt0 & 7) == 0 && s_rb[wave * 32 + 31] == vb0 && s_rt[wave * 32 + 31] == vt0 + 31;
-    vcontig = __builtin_amdgcn_readfirstlane(__all(ok && vgrp == 0xf) ? 1 : 0) != 0;
-  }
-
-  // chunk c with its weights at wb (the MFMAs, then after_mfma(), then the stores)
-  auto chunk = [&](int c, const char* wb, auto&& after_mfma) {
-    const bool cols_on_lanes = EPI == EPI_QKV && c * 32 >= 2 * a.D;
-    f32x4_t res[RB][4];
-    if constexpr (RSTAGE) {
-      // issue the residual loads before the MFMAs (in the staged layout)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        res[0][i] = rrow[i] ? *reinterpret_cast<const f32x4_t*>(rrow[i] + c * 32) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    } else if constexpr (EPI == EPI_RESID) {
-      // issue the residual loads before the MFMAs
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const int b = s_rb[my_row + rb * 32];
-        const float* rr = a.res + (int64_t)max(b, 0) * a.res_bstride +
-                          (int64_t)(s_rt[my_row + rb * 32] + a.res_toff) * a.N + c * 32 + hf * 4;
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          res[rb][g] = b >= 0 ? *reinterpret_cast<const f32x4_t*>(rr + g * 8) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-      }
-    }
-    f32x16_t acc[RB];
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[rb][e] = 0.0f;
-    if (cols_on_lanes) {
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const u32x4_t wf = wfrag(wb, s);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32x32x16(af[rb][s], wf, acc[rb]);
-      }
-      // (register path) the next chunk goes to LDS before this chunk's stores: its wait on the loads would
-      // otherwise also wait for the stores (vector memory completes in issue order)
-      after_mfma();
-      if (STAGE && vcontig) {
-        // tile row fr = feature c*32 + fr - 2D of V, columns = the wave's 32 tokens
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<u32x2_t*>(stage + fr * SST + (g * 8 + hf * 4) * 2) =
-              u32x2_t{pack_bf16x2(acc[0][4 * g], acc[0][4 * g + 1]), pack_bf16x2(acc[0][4 * g + 2], acc[0][4 * g + 3])};
-        const int64_t vbs = (int64_t)(a.D >> 6) * 64 * a.kv_pad;
-#pragma unroll
-        for (int i2 = 0; i2 < 2; ++i2) {
-          const int tr = i2 * 16 + (lane >> 2);
-          const int cv = c * 32 + tr - 2 * a.D;
-          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(stage + tr * SST + spiece * 16);
-          *reinterpret_cast<u32x4_t*>(a.vt + vb0 * vbs + ((int64_t)(cv >> 6) * 64 + (cv & 63)) * a.kv_pad + vt0 +
-                                      spiece * 8) = v;
-        }
-        return;
-      }
-      // V^T[b, h, d, token]: column cv = c*32 + fr - 2D of V is head cv / 64, d = cv % 64
-      const int cv = c * 32 + fr - 2 * a.D;
-      uint16_t* vrow = a.vt + ((int64_t)(cv >> 6) * 64 + (cv & 63)) * a.kv_pad;
-      const int64_t vbs = (int64_t)(a.D >> 6) * 64 * a.kv_pad;  // per sample
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int r0 = wave * RB * 32 + rb * 32 + g * 8 + hf * 4;
-          const float v[4] = {acc[rb][4 * g], acc[rb][4 * g + 1], acc[rb][4 * g + 2], acc[rb][4 * g + 3]};
-          if (vgrp & (1 << (rb * 4 + g))) {
-            *reinterpret_cast<u32x2_t*>(vrow + s_rb[r0] * vbs + s_rt[r0]) =
-                u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int b = s_rb[r0 + i];
-              if (b >= 0) vrow[b * vbs + s_rt[r0 + i]] = (uint16_t)bf16_bits(v[i]);
-            }
-          }
-        }
-    } else {
-#pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const u32x4_t wf = wfrag(wb, s);
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) acc[rb] = mfma32x32x16(wf, af[rb][s], acc[rb]);
-      }
-      after_mfma();
-      if constexpr (RSTAGE) {
-        // tile row fr = the lane's row: bf16-rounded outputs c*32 .. c*32 + 31 as fp32, then each lane adds the
-        // residual to its pieces and stores them
-        char* st = sStage + wave * 32 * RST;
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4_t*>(st + fr * RST + (g * 8 + hf * 4) * 4) =
-              f32x4_t{bf16_round(acc[0][4 * g]), bf16_round(acc[0][4 * g + 1]), bf16_round(acc[0][4 * g + 2]),
-                      bf16_round(acc[0][4 * g + 3])};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f32x4_t v = *reinterpret_cast<const f32x4_t*>(st + (i * 8 + (lane >> 3)) * RST + (lane & 7) * 16);
-          if (zrow[i])
-            *reinterpret_cast<f32x4_t*>(zrow[i] + c * 32) =
-                f32x4_t{v.x + res[0][i].x, v.y + res[0][i].y, v.z + res[0][i].z, v.w + res[0][i].w};
-        }
-        return;
-      }
-      if constexpr (STAGE) {
-        // every lane writes its row of the tile (rows without a token too: their pieces are not stored), then
-        // stores the pieces of its two tile rows: columns c*32 .. c*32 + 31 of Q or K
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<u32x2_t*>(stage + fr * SST + (g * 8 + hf * 4) * 2) =
-              u32x2_t{pack_bf16x2(acc[0][4 * g], acc[0][4 * g + 1]), pack_bf16x2(acc[0][4 * g + 2], acc[0][4 * g + 3])};
-        const bool isq = c * 32 < a.D;
-        const int col = (isq ? c * 32 : c * 32 - a.D) + spiece * 8;
-#pragma unroll
-        for (int i2 = 0; i2 < 2; ++i2) {
-          uint16_t* o = isq ? qrow[i2] : krow[i2];
-          const u32x4_t v = *reinterpret_cast<const u32x4_t*>(stage + (i2 * 16 + (lane >> 2)) * SST + spiece * 16);
-          if (o) *reinterpret_cast<u32x4_t*>(o + col) = v;
-        }
-        return;
-      }
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const int b = s_rb[my_row + rb * 32];
-        if (b < 0) continue;
-        const int t = s_rt[my_row + rb * 32];
-        const int col = c * 32 + hf * 4;  // + g * 8
-        if constexpr (EPI == EPI_RESID) {
-          float* o = reinterpret_cast<float*>(a.out) + (int64_t)b * a.out_bstride + (int64_t)t * a.N + col;
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<f32x4_t*>(o + g * 8) =
-                f32x4_t{bf16_round(acc[rb][4 * g]) + res[rb][g].x, bf16_round(acc[rb][4 * g + 1]) + res[rb][g].y,
-                        bf16_round(acc[rb][4 * g + 2]) + res[rb][g].z, bf16_round(acc[rb][4 * g + 3]) + res[rb][g].w};
-        } else if constexpr (EPI == EPI_QKV) {
-          uint16_t* o;
-          if (col < a.D) {  // Q: kept tail tokens only
-            const int tq = t - (a.kv - a.q_len);
-            if (tq < 0) continue;
-            o = a.q + ((int64_t)b * a.q_len + tq) * a.D + col;
-          } else {
-            o = a.k + ((int64_t)b * a.kv + t) * a.D + (col - a.D);
-          }
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<u32x2_t*>(o + g * 8) = u32x2_t{pack_bf16x2(acc[rb][4 * g], acc[rb][4 * g + 1]),
-                                                             pack_bf16x2(acc[rb][4 * g + 2], acc[rb][4 * g + 3])};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            epilogue_store<EPI>(a, b, t, col + (e >> 2) * 8 + (e & 3), acc[rb][e]);
-        }
-      }
-    }
-  };
-  if constexpr (DMA) {
-    // before the barrier of chunk c: every DMA but the (PF - 1) * WL pieces issued for chunks c + 1 ..
-    // c + PF - 1 has landed, whatever number of stores came between (vector memory completes in issue order)
-    constexpr unsigned kWait = 0x0F70u | (unsigned)((PF - 1) * WL);
-    static_assert((PF - 1) * WL < 16, "vmcnt immediate");
-    for (int cb = c0; cb < nchunks; cb += NST) {
-#pragma unroll
-      for (int k = 0; k < NST; ++k) {
-        const int c = cb + k;
-        if (c >= nchunks) break;
-        __builtin_amdgcn_s_waitcnt(kWait);
-        __syncthreads();  // chunk c is in LDS; every wave is done with chunk c - 1, whose stage is refilled
-        // unconditional (past the end it reloads the last chunk into the freed stage, read by no later chunk)
-        dma(min(c + PF, nchunks - 1), (k + PF) % NST);
-        chunk(c, sW[k], [] {});
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // no DMA may land in LDS after the workgroup ends
-  } else {
-    for (int c = c0; c < nchunks; ++c) {
-      const int buf = (c - c0) & 1;
-      __syncthreads();  // chunk c is in LDS; every wave is done with chunk c - 1
-      const bool more = c + 1 < nchunks;
-      if (more) gload(c + 1);
-      chunk(c, sW[buf], [&] { if (more) sstore(buf ^ 1); });
-    }
+    __syncthreads();  // sO is read before the next round writes it
   }
 }
 
@@ -968,7 +341,7 @@ __global__ __launch_bounds__(256, EPI == EPI_QKV ? PDM_QKV_WPS : 2) void rowgemm
 #define PDM_FFN_UP16 1
 #endif
 
-template <int D, int RB, int NW, int NST, int WPS, bool OPROJ>
+template <int D, int RB, int NW, int NST, int WPS>
 __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
   static_assert(!PDM_FFN_UP16 || RB == 1, "the 16x16x32 FFN-up assumes one row block per wave");
   constexpr int NT = NW * 64;                // threads
@@ -986,20 +359,19 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
   __shared__ int s_rb[TROWS];
   __shared__ int s_rt[TROWS];
   __shared__ float sGelu[GELU_T_N];
-  __shared__ __attribute__((aligned(16))) float sNw[OPROJ ? D : 4];  // RMSNorm2 weight
+  __shared__ __attribute__((aligned(16))) float sNw[D];  // RMSNorm2 weight
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   gelu_table_fill(sGelu, tid, NT);
-  if constexpr (OPROJ)
-    for (int i = tid; i < D; i += NT) sNw[i] = a.norm_w[i];
+  for (int i = tid; i < D; i += NT) sNw[i] = a.norm_w[i];
   const int F = a.N;
   const uint16_t* W1 = a.W;
   const uint16_t* W2 = a.W2;
-  // OPROJ: the O fragments of a tile's rows, the out-projection's B operand: lane (fr, hf) holds row
+  // the O fragments of a tile's rows, the out-projection's B operand: lane (fr, hf) holds row
   // wave * 32 + fr, columns 16 s + hf * 8 .. + 8 of 64-column chunk kc
   constexpr int DWO = D / 64;
-  u32x4_t ofr[OPROJ ? DWO : 1][4];
+  u32x4_t ofr[DWO][4];
   auto load_o = [&](int mt_, int fr_, int hf_) {
     int b, t;
     tile_row(a, mt_, TROWS, wave * 32 + fr_, b, t);
@@ -1079,7 +451,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
   __syncthreads();
   u32x4_t hfr[RB][KS];
   f32x16_t y[RB][DB];
-  if constexpr (OPROJ) {
+  {
     static_assert(RB == 1 && NST == 2, "the out-projection prologue assumes one row block and a 2-stage ring");
     constexpr int DW = D / 64;  // Wout chunks of 64 columns, each D rows x 128 bytes = one ring stage
     static_assert(DW % NST == 0, "FFN chunk c must keep stage c % NST");
@@ -1191,17 +563,6 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
       const uint32_t r1 = (uint32_t)__shfl_xor((int)(hf ? a1 : b1), 32, 64);
       hfr[0][s] = hf ? u32x4_t{r0, r1, b0, b1} : u32x4_t{a0, a1, r0, r1};
     }
-  } else {
-#pragma unroll
-    for (int c = 0; c < PF; ++c)
-      if (c < nchunks) dma(c, c);
-    load_row_fragments<D, RB, true>(a, s_rb, s_rt, wave, fr, hf, hfr);
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) y[rb][db][e] = 0.0f;
   }
 
 #if PDM_FFN_UP16
@@ -1355,18 +716,14 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
   }
 
   // Epilogue.  y[rb][db][e] is output d = db*32 + (e/4)*8 + hf*4 + e%4 of row wave*RB*32 + rb*32 + fr.
-  // OPROJ: y already holds z + FFN (the FFN-down accumulated on top of z).  Otherwise y = z + bf16(FFN) with
-  // z the residual rows read here.  The values go through LDS (the weight ring is free now) SEG outputs at
-  // a time, so that y is written (and z read) as whole row segments of SEG outputs, with non-temporal stores
-  // (y is streamed to memory; the next kernel reads it from there).  The z segments of the first two
-  // passes are requested before the last DMA is awaited, each later pass's when the pass two before it is
-  // done, so the passes do not wait for memory one after another.
+  // y already holds z + FFN (the FFN-down accumulated on top of z).  The values go through LDS (the weight ring is
+  // free now) SEG outputs at a time, so that y is written as whole row segments of SEG outputs, with non-temporal
+  // stores (y is streamed to memory; the next kernel reads it from there).
   constexpr int SEG = NW * RB * 32 * (64 * 4 + 16) <= RING_BYTES ? 64 : 32;  // outputs per pass
   constexpr int SROW = SEG * 4 + 16;       // LDS row stride (bytes), padded against bank conflicts
   constexpr int NQ = D / SEG;              // passes
   constexpr int EK = RB * 32 * (SEG / 4) / 64;  // 16-byte pieces per lane and pass
   static_assert(NW * RB * 32 * SROW <= RING_BYTES, "epilogue staging must fit the weight ring");
-  const float* zsrc = a.res;
   int64_t eoff[EK];  // piece k of this lane: its row's output offset + its 4 columns (pass 0), or -1
 #pragma unroll
   for (int k = 0; k < EK; ++k) {
@@ -1376,16 +733,6 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
     const int b = s_rb[row];
     eoff[k] = b < 0 ? -1 : (int64_t)b * a.out_bstride + (int64_t)s_rt[row] * D + c4 * 4;
   }
-  f32x4_t zv[OPROJ ? 1 : 2][EK];
-  auto zload = [&](int q) {
-    if constexpr (!OPROJ) {
-#pragma unroll
-      for (int k = 0; k < EK; ++k)
-        zv[q & 1][k] = *reinterpret_cast<const f32x4_t*>(zsrc + (eoff[k] < 0 ? 0 : eoff[k] + q * SEG));
-    }
-  };
-  zload(0);
-  if (NQ > 1) zload(1);
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // the last DMA must land before the ring is reused
   __syncthreads();
   char* stage = sRing + wave * (RB * 32 * SROW);
@@ -1398,10 +745,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
         const int db = q * (SEG / 32) + db2;
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4_t*>(stage + (rb * 32 + fr) * SROW + (db2 * 32 + g * 8 + hf * 4) * 4) = OPROJ ?
-              f32x4_t{y[rb][db][4 * g], y[rb][db][4 * g + 1], y[rb][db][4 * g + 2], y[rb][db][4 * g + 3]} :
-              f32x4_t{bf16_round(y[rb][db][4 * g]), bf16_round(y[rb][db][4 * g + 1]),
-                      bf16_round(y[rb][db][4 * g + 2]), bf16_round(y[rb][db][4 * g + 3])};
+          *reinterpret_cast<f32x4_t*>(stage + (rb * 32 + fr) * SROW + (db2 * 32 + g * 8 + hf * 4) * 4) =
+              f32x4_t{y[rb][db][4 * g], y[rb][db][4 * g + 1], y[rb][db][4 * g + 2], y[rb][db][4 * g + 3]};
       }
     // each wave reads back only its own tile; a wave's LDS accesses execute in order, so no barrier
 #pragma unroll
@@ -1409,12 +754,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
       const int piece = k * 64 + lane;
       const int r = piece / (SEG / 4), c4 = piece - (piece / (SEG / 4)) * (SEG / 4);
       const f32x4_t v = *reinterpret_cast<const f32x4_t*>(stage + r * SROW + c4 * 16);
-      const f32x4_t z = OPROJ ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : zv[q & 1][k];
       if (eoff[k] >= 0)
-        __builtin_nontemporal_store(OPROJ ? v : f32x4_t{z.x + v.x, z.y + v.y, z.z + v.z, z.w + v.w},
-                                    reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + eoff[k] + q * SEG));
+        __builtin_nontemporal_store(v, reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + eoff[k] + q * SEG));
     }
-    if (q + 2 < NQ) zload(q + 2);
   }
   }  // row tiles
 }
@@ -2020,7 +1362,6 @@ static void gemm_tiles(GemmArgs& g) {
   g.total_blocks = ((int64_t)g.tiles_s + (int64_t)g.n_ns * g.tiles_b) * g.n_tiles;
 }
 
-template <int EPI>
 static int launch_gemm(GemmArgs& g, hipStream_t s) {
   constexpr int TM = PDM_GEMM_TM;
   g.tiles_s = (int)(((int64_t)g.B * g.n_s + TM - 1) / TM);
@@ -2032,7 +1373,7 @@ static int launch_gemm(GemmArgs& g, hipStream_t s) {
   // 32-bit element offsets of a tile's A rows from its first row, and of the weight rows
   PDM_CHECK_ARG((int64_t)TM * g.a_bstride + g.a_bstride < (int64_t(1) << 31), "GEMM rows too far apart");
   PDM_CHECK_ARG((int64_t)g.N * g.K < (int64_t(1) << 31), "GEMM weight too large");
-  hipLaunchKernelGGL((gemm_kernel<EPI, TM>), dim3((unsigned)g.total_blocks), dim3(TM * 2), 0, s, g);
+  hipLaunchKernelGGL((gemm_kernel<TM>), dim3((unsigned)g.total_blocks), dim3(TM * 2), 0, s, g);
   PDM_CHECK_LAUNCH();
   return PDM_OK;
 }
@@ -2042,22 +1383,6 @@ static int64_t row_tiles(GemmArgs& g, int rows_per_tile) {
   g.tiles_s = (int)(((int64_t)g.B * g.n_s + rows_per_tile - 1) / rows_per_tile);
   g.tiles_b = (g.B + rows_per_tile - 1) / rows_per_tile;
   return (int64_t)g.tiles_s + (int64_t)g.n_ns * g.tiles_b;
-}
-
-template <int EPI, bool NORM>
-static int launch_rowgemm(GemmArgs& g, int D, hipStream_t s) {
-  // the residual epilogue keeps 16 loaded residual values per row block in registers: one row block per wave
-#ifndef PDM_QKV_RB
-#define PDM_QKV_RB 1
-#endif
-  constexpr int RB = EPI == EPI_RESID ? 1 : PDM_QKV_RB;
-  const int64_t tiles = row_tiles(g, 4 * RB * 32);
-  if (tiles == 0) return PDM_OK;
-  PDM_CHECK_ARG(tiles < (int64_t(1) << 31), "GEMM grid too large");
-  if (D == 256) hipLaunchKernelGGL((rowgemm_kernel<256, RB, EPI, NORM>), dim3((unsigned)tiles), dim3(256), 0, s, g);
-  else hipLaunchKernelGGL((rowgemm_kernel<128, RB, EPI, NORM>), dim3((unsigned)tiles), dim3(256), 0, s, g);
-  PDM_CHECK_LAUNCH();
-  return PDM_OK;
 }
 
 // FFN launch shape: RB * 32 rows per wave, NW waves per workgroup, an NST-stage
@@ -2078,15 +1403,10 @@ static int launch_rowgemm(GemmArgs& g, int D, hipStream_t s) {
 #ifndef PDM_FFN_WPS
 #define PDM_FFN_WPS 2
 #endif
-// the out-projection runs in the FFN kernel (1) or as its own GEMM in front of it (0)
-#ifndef PDM_FFN_OPROJ
-#define PDM_FFN_OPROJ 1
-#endif
 // The FFN grid is persistent (WPS workgroups per CU walk the row tiles; 0: one workgroup per tile).
 #ifndef PDM_FFN_PERSIST
 #define PDM_FFN_PERSIST 1
 #endif
-template <bool OPROJ>
 static int launch_ffn(GemmArgs& g, int D, hipStream_t s) {
   constexpr int RB = PDM_FFN_RB, NW = PDM_FFN_NW, NST = PDM_FFN_NST, WPS = PDM_FFN_WPS;
   const int64_t tiles = row_tiles(g, NW * RB * 32);
@@ -2105,24 +1425,8 @@ static int launch_ffn(GemmArgs& g, int D, hipStream_t s) {
     PDM_CHECK_HIP(err[dev]);
     grid = std::min<int64_t>(tiles, (int64_t)std::max(ncu[dev], 1) * WPS);
   }
-  if (D == 256) hipLaunchKernelGGL((ffn_kernel<256, RB, NW, NST, WPS, OPROJ>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
-  else hipLaunchKernelGGL((ffn_kernel<128, RB, NW, NST, WPS, OPROJ>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
-  PDM_CHECK_LAUNCH();
-  return PDM_OK;
-}
-
-static int launch_rmsnorm(const float* x, int64_t x_bstride, int T, int64_t B, int D, const float* w, uint16_t* out,
-                          hipStream_t s) {
-  const int64_t rows = B * T;
-  if (rows == 0) return PDM_OK;
-  const int64_t blocks = (rows + 3) / 4;
-  switch (D / 64) {
-    case 2: hipLaunchKernelGGL(rmsnorm_bf16_kernel<2>, dim3((unsigned)blocks), dim3(256), 0, s, x, x_bstride, T, rows, w, out, 1e-6f); break;
-    case 4: hipLaunchKernelGGL(rmsnorm_bf16_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, s, x, x_bstride, T, rows, w, out, 1e-6f); break;
-    case 6: hipLaunchKernelGGL(rmsnorm_bf16_kernel<6>, dim3((unsigned)blocks), dim3(256), 0, s, x, x_bstride, T, rows, w, out, 1e-6f); break;
-    case 8: hipLaunchKernelGGL(rmsnorm_bf16_kernel<8>, dim3((unsigned)blocks), dim3(256), 0, s, x, x_bstride, T, rows, w, out, 1e-6f); break;
-    default: set_error("rmsnorm: unsupported d_model"); return PDM_ERR_UNSUPPORTED;
-  }
+  if (D == 256) hipLaunchKernelGGL((ffn_kernel<256, RB, NW, NST, WPS>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
+  else hipLaunchKernelGGL((ffn_kernel<128, RB, NW, NST, WPS>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
   PDM_CHECK_LAUNCH();
   return PDM_OK;
 }
@@ -2204,28 +1508,17 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     qa.q = q; qa.k = k; qa.vt = vt;
     qa.B = B; qa.kv = kv; qa.q_len = ql; qa.n_ns = nns; qa.kv_pad = L.vt_ld;
     if ((st = launch_qkv_stationary(qa, D, s)) != PDM_OK) return st;
-  } else if (fused_path(d)) {
-    // 1. Q (tail rows), K, V^T = RMSNorm1(x) . Wqkv^T  (norm fused into the GEMM)
-    GemmArgs g0{};
-    g0.A32 = x; g0.a_bstride = (int64_t)kv * D; g0.norm_w = w->norm1_w;
-    g0.W = reinterpret_cast<const uint16_t*>(w->s_qkv_w);
-    g0.W_ns = reinterpret_cast<const uint16_t*>(w->ns_qkv_w);
-    g0.B = B; g0.n_s = kv - nns; g0.n_ns = nns; g0.N = 3 * D; g0.K = D;
-    g0.q = q; g0.k = k; g0.vt = vt; g0.kv = kv; g0.q_len = ql; g0.kv_pad = L.vt_ld; g0.D = D;
-    if ((st = launch_rowgemm<EPI_QKV, true>(g0, D, s)) != PDM_OK) return st;
   } else {
-    // 1. h1 = RMSNorm1(x)  [B, kv, D]
-    if ((st = launch_rmsnorm(x, (int64_t)kv * D, kv, B, D, w->norm1_w, h, s)) != PDM_OK) return st;
-    // 2. Q (tail rows), K, V^T
-    GemmArgs g0{};
-    g0.A = h; g0.a_bstride = (int64_t)kv * D;
-    g0.W = reinterpret_cast<const uint16_t*>(w->s_qkv_w);
-    g0.W_ns = reinterpret_cast<const uint16_t*>(w->ns_qkv_w);
-    g0.B = B; g0.n_s = kv - nns; g0.n_ns = nns; g0.N = 3 * D; g0.K = D;
-    g0.q = q; g0.k = k; g0.vt = vt; g0.kv = kv; g0.q_len = ql; g0.kv_pad = L.vt_ld; g0.D = D;
-    if ((st = launch_gemm<EPI_QKV>(g0, s)) != PDM_OK) return st;
+    // 1. Q (tail rows), K, V^T = RMSNorm1(x) . Wqkv^T  (norm fused)
+    RowProjArgs r0{};
+    r0.x = x; r0.in_bstride = (int64_t)kv * D; r0.norm_w = w->norm1_w;
+    r0.W = reinterpret_cast<const uint16_t*>(w->s_qkv_w);
+    r0.W_ns = reinterpret_cast<const uint16_t*>(w->ns_qkv_w);
+    r0.B = B; r0.n_s = kv - nns; r0.n_ns = nns; r0.N = 3 * D;
+    r0.q = q; r0.k = k; r0.vt = vt; r0.kv = kv; r0.q_len = ql; r0.kv_pad = L.vt_ld;
+    if ((st = launch_row_proj(r0, D, ROWPROJ_QKV, s)) != PDM_OK) return st;
   }
-  // 3. attention -> O (written over Q: each wave reads its Q rows before writing them)
+  // 2. attention -> O (written over Q: each wave reads its Q rows before writing them)
   {
     AttnArgs aa{};
     aa.q = q; aa.k = k; aa.vt = vt; aa.o = q;
@@ -2263,9 +1556,8 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     }
     PDM_CHECK_LAUNCH();
   }
-#if PDM_FFN_OPROJ
   if (fused_path(d)) {
-    // 4. z = bf16(O . Wout^T) + x[:, kv - q_len:] (written to y), y = z + bf16(W2 . gelu(W1 . RMSNorm2(z))):
+    // 3. z = bf16(O . Wout^T) + x[:, kv - q_len:], y = z + bf16(W2 . gelu(W1 . RMSNorm2(z))):
     // out-projection, norm, both FFN GEMMs and GELU in one kernel
     GemmArgs g2{};
     g2.A = q; g2.a_bstride = (int64_t)ql * D;
@@ -2278,10 +1570,9 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     g2.W2_ns = reinterpret_cast<const uint16_t*>(w->ns_w2);
     g2.B = B; g2.n_s = ql - nns; g2.n_ns = nns; g2.N = F; g2.K = D;
     g2.out = y; g2.out_bstride = (int64_t)ql * D;
-    return launch_ffn<true>(g2, D, s);
+    return launch_ffn(g2, D, s);
   }
-#endif
-  // 4. z = bf16(O . Wout^T) + x[:, kv - q_len:]  -> y
+  // 3. z = bf16(O . Wout^T) + x[:, kv - q_len:]  -> y
   {
     GemmArgs g1{};
     g1.A = q; g1.a_bstride = (int64_t)ql * D;
@@ -2289,37 +1580,19 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     g1.B = B; g1.n_s = ql; g1.n_ns = 0; g1.N = D; g1.K = D;
     g1.out = y; g1.out_bstride = (int64_t)ql * D;
     g1.res = x; g1.res_bstride = (int64_t)kv * D; g1.res_toff = kv - ql;
-    if (fused_path(d)) {
-      if ((st = launch_rowgemm<EPI_RESID, false>(g1, D, s)) != PDM_OK) return st;
-    } else if ((st = launch_gemm<EPI_RESID>(g1, s)) != PDM_OK) {
-      return st;
-    }
+    if ((st = launch_gemm(g1, s)) != PDM_OK) return st;
   }
-  if (fused_path(d)) {
-    // 5. y = z + bf16(W2 . gelu(W1 . RMSNorm2(z)))  (norm, both GEMMs and GELU in one kernel)
-    GemmArgs g2{};
-    g2.A32 = y; g2.a_bstride = (int64_t)ql * D; g2.norm_w = w->norm2_w;
-    g2.W = reinterpret_cast<const uint16_t*>(w->s_w1);
-    g2.W_ns = reinterpret_cast<const uint16_t*>(w->ns_w1);
-    g2.W2 = reinterpret_cast<const uint16_t*>(w->s_w2);
-    g2.W2_ns = reinterpret_cast<const uint16_t*>(w->ns_w2);
-    g2.B = B; g2.n_s = ql - nns; g2.n_ns = nns; g2.N = F; g2.K = D;
-    g2.out = y; g2.out_bstride = (int64_t)ql * D; g2.res = y;
-    return launch_ffn<false>(g2, D, s);
-  }
-  // 5. h2 = RMSNorm2(z)  [B, q_len, D]
-  if ((st = launch_rmsnorm(y, (int64_t)ql * D, ql, B, D, w->norm2_w, h, s)) != PDM_OK) return st;
-  // 6. g = bf16(gelu(bf16(h2 . W1^T)))  [B, q_len, F]
+  // 4. h = RMSNorm2(z)  [B, q_len, D], g = bf16(gelu(bf16(h2 . W1^T)))  [B, q_len, F]
   {
-    GemmArgs g2{};
-    g2.A = h; g2.a_bstride = (int64_t)ql * D;
-    g2.W = reinterpret_cast<const uint16_t*>(w->s_w1);
-    g2.W_ns = reinterpret_cast<const uint16_t*>(w->ns_w1);
-    g2.B = B; g2.n_s = ql - nns; g2.n_ns = nns; g2.N = F; g2.K = D;
-    g2.out = g; g2.out_bstride = (int64_t)ql * F;
-    if ((st = launch_gemm<EPI_GELU>(g2, s)) != PDM_OK) return st;
+    RowProjArgs r2{};
+    r2.x = y; r2.norm_w = w->norm2_w; r2.in_bstride = (int64_t)ql * D;
+    r2.W = reinterpret_cast<const uint16_t*>(w->s_w1);
+    r2.W_ns = reinterpret_cast<const uint16_t*>(w->ns_w1);
+    r2.B = B; r2.n_s = ql - nns; r2.n_ns = nns; r2.N = F;
+    r2.h = h; r2.out = g; r2.out_bstride = (int64_t)ql * F;
+    if ((st = launch_row_proj(r2, D, ROWPROJ_GELU, s)) != PDM_OK) return st;
   }
-  // 7. y = z + bf16(g . W2^T)
+  // 5. y = z + bf16(g . W2^T)
   {
     GemmArgs g3{};
     g3.A = g; g3.a_bstride = (int64_t)ql * F;
@@ -2328,7 +1601,7 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     g3.B = B; g3.n_s = ql - nns; g3.n_ns = nns; g3.N = D; g3.K = F;
     g3.out = y; g3.out_bstride = (int64_t)ql * D;
     g3.res = y; g3.res_bstride = (int64_t)ql * D; g3.res_toff = 0;
-    if ((st = launch_gemm<EPI_RESID>(g3, s)) != PDM_OK) return st;
+    if ((st = launch_gemm(g3, s)) != PDM_OK) return st;
   }
   return PDM_OK;
 }

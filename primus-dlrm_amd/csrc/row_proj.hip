@@ -1,0 +1,429 @@
+// Row projections of the OneTrans block: out = RMSNorm(x) . W^T for fp32 rows of D <= 512 columns, with the Q/K/V
+// scatter or the GELU as the epilogue.
+//
+// Layout of the work.  A wave owns 32 rows and holds all D normalised columns of them in registers (the MFMA B
+// operand: lane l has row l % 32, k = 8 (l / 32) .. +8 of every 16-wide step), so a row is read and normalised once
+// whatever N is.  The weight streams through LDS in chunks of 32 output columns x D, filled by LDS DMA NST - 1 chunks
+// ahead and shared by the workgroup's four waves.  Within a wave, the DMA of a later chunk and the epilogue of the
+// previous one (rounding, GELU, stores) are issued between the MFMAs of the current chunk; two workgroups share a CU
+// with independent barriers, so one's row loads run beside the other's MFMAs.
+//
+// A wave's rows are 32 consecutive tokens of ONE sample (the shared S weight) or one NS token of 32 samples (that
+// token's weight): addresses are a wave-uniform base plus row * stride, and a feature row of V^T receives runs of 8
+// tokens at multiples of 8.  Padding rows (the last block of a sample, samples past the batch) read the block's last
+// row again and store nothing.
+//
+// What bounds it, at OneTransL's second layer (d 384, B = 1024, 1,552,384 rows in, 1,335,296 kept): the fp32 rows in and
+// the bf16 outputs out (5.8 GB for Q/K/V, about 1.2 ms at a device copy's rate; 1.37 TFLOP, 0.55 ms of MFMA), behind
+// them the vector instructions between the MFMAs.  Q/K/V 1.72 ms against 0.63 (RMSNorm kernel) + 2.52 ms (128 x 256
+// LDS-tiled GEMM); FFN-up + GELU 2.0 ms against 0.53 + 2.61 ms.  What that took: addresses kept in registers and the
+// GELU table reached by one shift (231 -> 144 vector instructions per chunk: 2.20 -> 2.00 ms), whole 64-byte segments
+// per store, the NS tiles spread over the XCDs (2.14 -> 1.86 ms for Q/K/V).  64 rows per wave (half the LDS reads and
+// weight traffic) need 192 operand registers and leave none to overlap the stores: 1.88 ms without the norm.
+//
+// Workgroups split the N columns of one row tile when there are few row tiles, so that a small batch fills the chip;
+// the splits of a tile are neighbours on one XCD, whose L2 then serves the rows to all of them (4 layers of d 128 at
+// B = 16: 186 -> 157 us with the splits).
+#include <algorithm>
+#include <mutex>
+#include <type_traits>
+
+#include "pdm_common.h"
+#include "mfma_common.h"
+#include "block_kernels.h"
+
+namespace pdm {
+
+// GELU table of this file: the top 2048 entries of mfma_common.h's range, |x| in (2^-13, 8].  Below it |x| is clamped
+// to the first entry, where e differs from its value at |x| by less than 5e-5: x e and x (1 - e) both round to the
+// bf16 value x / 2 (half a bf16 step is 2^-9 relative), so results are the longer table's bit for bit, and the table
+// takes 8 KB: with the 72 KB ring of D = 384 two workgroups fill the 160 KB of LDS exactly.
+constexpr uint32_t kGeluLo = GELU_T_HI - 2047u;
+constexpr int kGeluN = 2048;
+
+// g[0..3] = GELU of u[first .. first + 7], rounded to bf16 before and after; t: LDS address of the table.  The entry of
+// a bf16 pattern is at byte 4 (pattern - kGeluLo), i.e. (fp32 bits >> 14) - 4 kGeluLo: one shift and an immediate.
+__device__ __forceinline__ void gelu2048_pack(uint32_t t, const f32x16_t& u, int first, uint32_t* g) {
+  float x[8], e[8];
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) {
+    const uint32_t p = pack_bf16x2(u[first + i], u[first + i + 1]);
+    x[i] = __builtin_bit_cast(float, p << 16);
+    x[i + 1] = __builtin_bit_cast(float, p & 0xffff0000u);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float c = __builtin_amdgcn_fmed3f(fabsf(x[i]), __builtin_bit_cast(float, kGeluLo << 16), 8.0f);
+    e[i] = *reinterpret_cast<const __attribute__((address_space(3))) float*>((__builtin_bit_cast(uint32_t, c) >> 14) + (t - 4 * kGeluLo));
+  }
+#pragma unroll
+  for (int i = 0; i < 8; i += 2)
+    g[i >> 1] = pack_bf16x2(__builtin_fmaf(-fabsf(x[i]), e[i], fmaxf(x[i], 0.0f)),
+                            __builtin_fmaf(-fabsf(x[i + 1]), e[i + 1], fmaxf(x[i + 1], 0.0f)));
+}
+
+// exchanges lanes 32..63 of a with lanes 0..31 of b
+__device__ __forceinline__ void half_swap(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// exchanges lanes 16..31 (48..63) of a with lanes 0..15 (32..47) of b
+__device__ __forceinline__ void quarter_swap(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
+// The 32 x 32 output tile whose line l % 32 (a row, or a feature of V^T) lies in lanes l and l + 32, packed to bf16
+// (dword j of half h: outputs 16 h + 8 (j / 2) + 4 (l / 32) + 2 (j % 2) and the next), regrouped so that 16-byte
+// stores write whole 64-byte segments: part 0 are lines 0..15, part 1 lines 16..31, lane l of part i holding
+// outputs 8 piece .. 8 piece + 7 of line 16 i + l % 16, piece = 2 ((l / 16) % 2) + l / 32.
+__device__ __forceinline__ void tile_segments(uint32_t (&p)[2][4]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    half_swap(p[h][0], p[h][2]);
+    half_swap(p[h][1], p[h][3]);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) quarter_swap(p[0][j], p[1][j]);
+}
+
+// 16-byte store at base + off (base wave-uniform), dropped for lanes with off == kNoStore: a buffer store whose range
+// check discards them, so the instruction is always issued and the memory operations of a chunk can be counted.
+constexpr uint32_t kNoStore = 0xFFFFFFFFu;
+__device__ __forceinline__ void store16(void* base, uint32_t off, u32x4_t v) {
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7FFFFFFF, 0x00020000);
+  __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, (int)off, 0, 0);
+}
+
+// ring depth: as many 32-column chunks as two workgroups per CU leave room for, at most 4
+template <int D>
+constexpr int rowproj_stages() { return D <= 256 ? 4 : (D == 384 ? 3 : 2); }
+template <int D>
+constexpr int rowproj_lds(bool gelu) { return rowproj_stages<D>() * 64 * D + (gelu ? kGeluN * 4 : 0); }
+
+template <int D, int EPI>
+__global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
+  constexpr int KS = D / 16;          // MFMA k steps
+  constexpr int NST = rowproj_stages<D>(), PF = NST - 1;
+  constexpr int CHUNK = 64 * D;       // bytes of 32 weight rows
+  constexpr int P = D / 8;            // 16-byte pieces per weight row
+  constexpr int NDMA = P / 8;         // DMA instructions per wave and chunk: a wave fills 8 rows
+  constexpr int LEAD = 4;             // weight fragments read ahead of their MFMA
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  float* gelu_t = reinterpret_cast<float*>(lds + NST * CHUNK);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 31, hf = lane >> 5;
+  const int l16 = lane & 15, piece = 2 * ((lane >> 4) & 1) + hf;  // tile_segments
+
+  // workgroup -> (row tile, column split): the NS tiles first, then the S tiles, each group dealt so that neighbours
+  // share an XCD (workgroups go to the 8 XCDs in turn): a token's tiles share its weight, a tile's splits its rows.
+  // (With both groups in one such order the NS tiles, the slowest, all fell to the last XCD.)
+  const int n_ns_wgs = a.wgs_ns * a.split_ns;
+  const bool is_s = (int)blockIdx.x >= n_ns_wgs;
+  int rest = is_s ? (int)blockIdx.x - n_ns_wgs : (int)blockIdx.x;
+  const int full = (is_s ? a.wgs_s * a.split_s : n_ns_wgs) & ~7;
+  if (rest < full) rest = (rest & 7) * (full >> 3) + (rest >> 3);
+  const int split = is_s ? a.split_s : a.split_ns;
+  const int tile = rest / split, part = rest - tile * split;
+  // the wave's rows: row i is (sample b0, token t0 + i) or (sample b0 + i, token t0)
+  int b0, t0, rows, g = 0;
+  if (is_s) {
+    const int64_t blk = (int64_t)tile * 4 + wave;
+    b0 = (int)(blk / a.blocks_per_sample);
+    t0 = (int)(blk - (int64_t)b0 * a.blocks_per_sample) * 32;
+    rows = b0 < a.B ? min(32, a.n_s - t0) : 0;
+    if (b0 >= a.B) b0 = t0 = 0;
+  } else {
+    g = tile / a.tiles_per_token;
+    b0 = ((tile - g * a.tiles_per_token) * 4 + wave) * 32;
+    t0 = a.n_s + g;
+    rows = max(0, min(32, a.B - b0));
+    if (rows == 0) b0 = 0;
+  }
+  const int last = max(rows - 1, 0);
+  const uint16_t* W = is_s ? a.W : a.W_ns + (int64_t)g * a.N * D;
+
+  const int nchunks = a.N / 32;
+  const int c_begin = (int)((int64_t)nchunks * part / split), c_end = (int)((int64_t)nchunks * (part + 1) / split);
+
+  // instruction p of the DMA of weight chunk c into ring stage stg: 16-byte piece v of row r lies at slot
+  // v ^ (r & 15), so the 32 rows of a fragment read fall in distinct bank groups
+  uint32_t doff[NDMA];
+#pragma unroll
+  for (int p = 0; p < NDMA; ++p) {
+    const int o = p * 64 + lane, r = wave * 8 + o / P, v = (o % P) ^ (r & 15);
+    doff[p] = (uint32_t)(r * (2 * D) + v * 16);
+  }
+  auto dma = [&](int c, int stg, int p) {
+    lds_dma16((uint64_t)(uintptr_t)W + (uint64_t)c * CHUNK, doff[p],
+              (uint32_t)(uintptr_t)(lds + stg * CHUNK + (wave * 8 * P + p * 64) * 16));
+  };
+
+  if constexpr (EPI == ROWPROJ_GELU)
+    for (int i = tid; i < kGeluN; i += 256) gelu_t[i] = gelu_tail(__builtin_bit_cast(float, (kGeluLo + (uint32_t)i) << 16));
+
+  // RMSNorm: 16 lanes per fp32 row (256-byte segments), SL rows in flight; the bf16 rows pass through the wave's part
+  // of the (still unused) ring into the fragment layout
+  u32x4_t af[KS];
+  {
+    const int64_t rstride = is_s ? D : a.in_bstride;  // elements between the wave's rows
+    constexpr int SL = D <= 384 ? 16 : 8, NV = D / 64, STR = 2 * D + 16;
+    static_assert(4 * SL * STR <= NST * CHUNK, "the row scratch lies in the weight ring");
+    char* sc = lds + wave * SL * STR;
+    const float* x0 = a.x + (int64_t)b0 * a.in_bstride + (int64_t)t0 * D;
+    uint16_t* h0 = a.h + (int64_t)b0 * a.in_bstride + (int64_t)t0 * D;
+    const int sub = lane & 15, rq = lane >> 4;
+    f32x4_t w[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) w[j] = *reinterpret_cast<const f32x4_t*>(a.norm_w + j * 64 + sub * 4);
+#pragma unroll
+    for (int sl = 0; sl < 32 / SL; ++sl) {
+      f32x4_t v[SL / 4][NV];
+#pragma unroll
+      for (int p = 0; p < SL / 4; ++p) {
+        const float* xr = x0 + min(sl * SL + p * 4 + rq, last) * rstride + sub * 4;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[p][j] = *reinterpret_cast<const f32x4_t*>(xr + j * 64);
+      }
+      // every load of the slice is in flight before the first is used (left to itself the compiler loads and
+      // reduces 4 rows at a time, one memory latency each)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = 0; p < SL / 4; ++p) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+          ss += (v[p][j].x * v[p][j].x + v[p][j].y * v[p][j].y) + (v[p][j].z * v[p][j].z + v[p][j].w * v[p][j].w);
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+        const float rms = 1.0f / sqrtf(ss / (float)D + 1e-6f);
+        const int r = sl * SL + p * 4 + rq;
+        uint16_t* hr = h0 + (int64_t)r * rstride + sub * 4;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          const u32x2_t n = u32x2_t{pack_bf16x2((v[p][j].x * rms) * w[j].x, (v[p][j].y * rms) * w[j].y),
+                                    pack_bf16x2((v[p][j].z * rms) * w[j].z, (v[p][j].w * rms) * w[j].w)};
+          if (EPI == ROWPROJ_GELU && part == 0 && r < rows) *reinterpret_cast<u32x2_t*>(hr + j * 64) = n;
+          *reinterpret_cast<u32x2_t*>(sc + (p * 4 + rq) * STR + j * 128 + sub * 8) = n;
+        }
+      }
+      if (fr / SL == sl) {  // the wave's own LDS operations complete in order
+#pragma unroll
+        for (int s = 0; s < KS; ++s) af[s] = *reinterpret_cast<const u32x4_t*>(sc + (fr % SL) * STR + (2 * s + hf) * 16);
+      }
+    }
+    __syncthreads();  // every wave is done with the scratch before the ring fills it
+  }
+#pragma unroll
+  for (int j = 0; j < PF; ++j)
+#pragma unroll
+    for (int p = 0; p < NDMA; ++p) dma(min(c_begin + j, nchunks - 1), j, p);
+
+  // Q is needed of the kept tail tokens only: rows below q_first of this wave have none
+  const int q_first = a.kv - a.q_len - t0;
+  const bool skip_q = EPI == ROWPROJ_QKV && (is_s ? q_first >= rows : rows == 0);
+
+  // the previous chunk's tile, stored during the current one: line r (line_lo <= r < line_hi) at obase + r * ostride
+  // elements, of which the first `outs` outputs exist
+  f32x16_t prev;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) prev[e] = 0.0f;
+  uint16_t* obase = EPI == ROWPROJ_GELU ? a.out : a.k;
+  uint32_t ostride = 0;
+  int line_lo = 0, line_hi = 0, outs = 32;
+  uint32_t pk[2][4];
+  auto epi_pack = [&](int h) {
+    if constexpr (EPI == ROWPROJ_GELU) {
+      gelu2048_pack((uint32_t)(uintptr_t)lds + NST * CHUNK, prev, 8 * h, pk[h]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pk[h][j] = pack_bf16x2(prev[8 * h + 2 * j], prev[8 * h + 2 * j + 1]);
+    }
+  };
+  auto epi_store = [&](int i) {
+    const int r = 16 * i + l16;
+    const uint32_t off = ((uint32_t)r * ostride + piece * 8) * 2;
+    store16(obase, r >= line_lo && r < line_hi && piece * 8 + 8 <= outs ? off : kNoStore,
+            u32x4_t{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+  };
+  // a sample's last V^T tokens when they are no multiple of 8: not the NS tokens behind them
+  auto epi_tail = [&]() {
+    if (EPI == ROWPROJ_QKV && (outs & 7)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (piece == outs >> 3 && 16 * i + l16 < line_hi) {
+          uint16_t* v = obase + (int64_t)(16 * i + l16) * ostride + piece * 8;
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (piece * 8 + e < outs) v[e] = (uint16_t)(pk[i][e >> 1] >> (16 * (e & 1)));
+        }
+    }
+  };
+
+  int stg = 0;
+  // chunk c: its MFMAs (V: columns on lanes; otherwise rows on lanes), then where its tile goes
+  auto step = [&](int c, auto v_tag) {
+    constexpr bool V = decltype(v_tag)::value;
+    // Vector memory completes in issue order; behind chunk c's DMA the wave issued the DMAs of the PF - 1 chunks after
+    // it and, from the PF-th chunk on, two stores in each of the PF iterations since: chunk c has landed once no more
+    // than those are outstanding
+    if (c - c_begin >= PF) __builtin_amdgcn_s_waitcnt(waitcnt_vm((PF - 1) * NDMA + PF * 2));
+    else __builtin_amdgcn_s_waitcnt(waitcnt_vm((PF - 1) * NDMA));
+    __syncthreads();  // publishes every wave's part of the chunk and frees the stage of chunk c - 1
+    // past the end the last chunk is loaded again, into a stage that no later chunk reads
+    const int cn = min(c + PF, nchunks - 1), sn = stg == 0 ? NST - 1 : stg - 1;
+    // fragment s of the chunk: row fr, logical piece 2 s + hf, at slot (2 s) ^ (hf ^ (fr & 15)); rows and stages are
+    // multiples of 256 bytes, so 8 XORed addresses and immediate offsets reach every fragment
+    uint32_t wb = (uint32_t)(uintptr_t)lds + stg * CHUNK + fr * (2 * D) + ((hf ^ (fr & 15)) << 4);
+    asm volatile("" : "+v"(wb));  // not hoisted out of the chunk loop: the variants would take 8 registers
+    stg = stg + 1 == NST ? 0 : stg + 1;
+    auto wfrag = [&](int s) {
+      return reinterpret_cast<const __attribute__((address_space(3))) u32x4_t*>(wb ^ ((2 * s & 15) << 4))[2 * s & ~15];
+    };
+    const bool is_q = EPI == ROWPROJ_QKV && !V && c * 32 < D;
+    f32x16_t acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
+    if (is_q && skip_q) {
+#pragma unroll
+      for (int p = 0; p < NDMA; ++p) dma(cn, sn, p);
+      epi_pack(0);
+      epi_pack(1);
+      tile_segments(pk);
+      epi_store(0);
+      epi_store(1);
+    } else {
+      // MFMAs of chunk c, with the DMAs and the previous chunk's epilogue between them (the order is pinned)
+      u32x4_t wf[LEAD];
+#pragma unroll
+      for (int s = 0; s < LEAD; ++s) wf[s] = wfrag(s);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        acc = V ? mfma32x32x16(af[s], wf[s % LEAD], acc) : mfma32x32x16(wf[s % LEAD], af[s], acc);
+        if (s + LEAD < KS) wf[s % LEAD] = wfrag(s + LEAD);
+        if (s % 2 == 1 && s / 2 < NDMA) dma(cn, sn, s / 2);
+        if (s == KS / 4) epi_pack(0);
+        if (s == KS / 2) epi_pack(1);
+        if (s == KS * 5 / 8) tile_segments(pk);
+        if (s == KS * 6 / 8) epi_store(0);
+        if (s == KS * 7 / 8) epi_store(1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    epi_tail();
+
+    prev = acc;
+    if constexpr (EPI == ROWPROJ_GELU) {
+      obase = a.out + (int64_t)b0 * a.out_bstride + (int64_t)t0 * a.N + c * 32;
+      ostride = is_s ? (uint32_t)a.N : (uint32_t)a.out_bstride;
+      line_hi = rows;
+    } else if constexpr (V) {
+      // lines are features c*32 - 2D .. + 31, outputs the wave's tokens
+      const int64_t vbs = (int64_t)D * a.kv_pad;  // elements per sample
+      obase = a.vt + (int64_t)b0 * vbs + (int64_t)(c * 32 - 2 * D) * a.kv_pad + t0;
+      ostride = (uint32_t)a.kv_pad;
+      line_lo = 0;
+      line_hi = is_s && rows > 0 ? 32 : 0;
+      outs = is_s ? rows : 32;
+      if (!is_s) {
+        // one token of 32 samples: 2-byte stores at once, the sample stride added step by step
+        int64_t vstep = vbs;
+        asm volatile("" : "+s"(vstep));
+        uint16_t* v = obase + (int64_t)(hf * 4) * vbs + (int64_t)fr * a.kv_pad;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          if ((e >> 2) * 8 + hf * 4 + (e & 3) < rows) *v = (uint16_t)bf16_bits(acc[e]);
+          v += (e & 3) == 3 ? 5 * vstep : vstep;
+        }
+      }
+    } else if (is_q) {
+      obase = a.q + ((int64_t)b0 * a.q_len - q_first) * D + c * 32;
+      ostride = is_s ? (uint32_t)D : (uint32_t)(a.q_len * D);
+      line_lo = is_s ? max(q_first, 0) : 0;
+      line_hi = skip_q ? 0 : rows;
+    } else {
+      obase = a.k + ((int64_t)b0 * a.kv + t0) * D + c * 32 - D;
+      ostride = is_s ? (uint32_t)D : (uint32_t)(a.kv * D);
+      line_lo = 0;
+      line_hi = rows;
+    }
+  };
+  int c = c_begin;
+  const int c_v = EPI == ROWPROJ_QKV ? min(c_end, D / 16) : c_end;  // V chunks from 2 D columns on
+  for (; c < c_v; ++c) step(c, std::false_type{});
+  if constexpr (EPI == ROWPROJ_QKV)
+    for (; c < c_end; ++c) step(c, std::true_type{});
+  epi_pack(0);
+  epi_pack(1);
+  tile_segments(pk);
+  epi_store(0);
+  epi_store(1);
+  epi_tail();
+  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // no DMA may land in LDS after the workgroup ends
+}
+
+template <int D, int EPI>
+static int launch_one(RowProjArgs a, hipStream_t s) {
+  constexpr int lds = rowproj_lds<D>(EPI == ROWPROJ_GELU);
+  static std::once_flag once[64];
+  static hipError_t err[64];
+  int dev = 0;
+  PDM_CHECK_HIP(hipGetDevice(&dev));
+  PDM_CHECK_ARG(dev >= 0 && dev < 64, "device index out of range");
+  std::call_once(once[dev], [&] {
+    err[dev] = hipFuncSetAttribute(reinterpret_cast<const void*>(rowproj_kernel<D, EPI>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  });
+  PDM_CHECK_HIP(err[dev]);
+  a.blocks_per_sample = (a.n_s + 31) / 32;
+  const int64_t wgs_s = ((int64_t)a.B * a.blocks_per_sample + 3) / 4;
+  a.tiles_per_token = (a.B + 127) / 128;
+  const int64_t wgs_ns = (int64_t)a.n_ns * a.tiles_per_token;
+  // column splits: about two workgroups per CU, at least two chunks each
+  const int nchunks = a.N / 32;
+  const int64_t want = 512;
+  a.split_s = a.split_ns = 1;
+  while (wgs_s * a.split_s + wgs_ns * a.split_ns < want) {
+    // the side whose workgroups walk more chunks is split further
+    if (wgs_ns > 0 && (wgs_s == 0 || a.split_ns <= a.split_s)) {
+      if (a.split_ns * 4 > nchunks) break;
+      a.split_ns *= 2;
+    } else {
+      if (a.split_s * 4 > nchunks) break;
+      a.split_s *= 2;
+    }
+  }
+  const int64_t grid = wgs_s * a.split_s + wgs_ns * a.split_ns;
+  if (grid == 0) return PDM_OK;
+  PDM_CHECK_ARG(grid < (int64_t(1) << 31), "row projection grid too large");
+  // 32 lines of any output lie within 2^31 bytes of the wave's first
+  PDM_CHECK_ARG((int64_t)32 * std::max<int64_t>({a.out_bstride, (int64_t)a.kv * D, (int64_t)a.kv_pad}) * 2 < (int64_t(1) << 31),
+                "row projection rows too far apart");
+  a.wgs_s = (int)wgs_s;
+  a.wgs_ns = (int)wgs_ns;
+  hipLaunchKernelGGL((rowproj_kernel<D, EPI>), dim3((unsigned)grid), dim3(256), lds, s, a);
+  PDM_CHECK_LAUNCH();
+  return PDM_OK;
+}
+
+template <int EPI>
+static int launch_epi(const RowProjArgs& a, int D, hipStream_t s) {
+  switch (D) {
+    case 128: return launch_one<128, EPI>(a, s);
+    case 256: return launch_one<256, EPI>(a, s);
+    case 384: return launch_one<384, EPI>(a, s);
+    case 512: return launch_one<512, EPI>(a, s);
+    default: set_error("row projection: unsupported d_model"); return PDM_ERR_UNSUPPORTED;
+  }
+}
+
+int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s) {
+  return epi == ROWPROJ_QKV ? launch_epi<ROWPROJ_QKV>(a, D, s) : launch_epi<ROWPROJ_GELU>(a, D, s);
+}
+
+}  // namespace pdm

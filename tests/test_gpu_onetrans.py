@@ -118,6 +118,21 @@ def test_block_d512_tiled_path(pdm, dev):
     _run_case(pdm, dev, 3, 40, 20, 3, D=512, F=2048, seed=9, norm_std=0.2)
 
 
+@pytest.mark.parametrize("B,kv,q_len,n_ns,D", [
+    (1, 5, 5, 4, 384),      # one S token: a block of 31 padding rows, every column split of the small grid
+    (2, 47, 20, 7, 128),    # 40 S tokens: the last block stores one run of 8 V^T tokens
+    (3, 71, 40, 6, 512),    # 65 S tokens: the last block holds one token, no multiple of 8
+    (2, 30, 30, 0, 384),    # no NS tokens
+    (3, 16, 16, 16, 384),   # no S tokens
+    (140, 37, 24, 3, 384),  # NS tokens over two row tiles of 128 samples, the second partial
+    (700, 101, 50, 2, 128),  # enough row tiles that no column split is made; 99 S tokens, Q of the tail only
+])
+def test_block_row_projection_edges(pdm, dev, B, kv, q_len, n_ns, D):
+    """The Q/K/V and FFN-up projections (32-token blocks of a sample, 32-sample blocks of an NS token, column
+    splits) at the edges of their blocks, with the tolerance of every block test."""
+    _run_case(pdm, dev, B, kv, q_len, n_ns, D=D, F=2 * D, seed=B + kv, norm_std=0.1)
+
+
 def test_block_baseline_shape_reduced_batch(pdm, dev):
     """The 4-layer benchmark's first layer (400 tokens, 16 NS, d 256, FFN 1024) at batch 8."""
     _run_case(pdm, dev, 8, 400, 400, 16, seed=11)
