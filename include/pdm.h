@@ -347,7 +347,7 @@ int pdm_seq_tokenize_fwd(const pdm_seq_desc* desc, const void* const* tables,
 
 typedef struct {
   int32_t batch;    /* B */
-  int32_t d_model;  /* D: 128 or 256 (fused kernels), 384 or 512 (tiled kernels) */
+  int32_t d_model;  /* D: 128, 256, 384 or 512 */
   int32_t n_heads;  /* H (D / H = 64 supported) */
   int32_t n_ns;     /* NS tokens at the end of the sequence */
   int32_t ffn_dim;  /* FFN hidden (multiple of 128) */

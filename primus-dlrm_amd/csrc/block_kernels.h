@@ -53,4 +53,23 @@ struct RowProjArgs {
 };
 int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s);
 
+// Residual projection (resid_gemm.hip): out = A . W^T (rounded to bf16 with round_bf16) + res, fp32; S tokens (t < n_s) use W, NS token n_s + g
+// uses W_ns[g].
+struct ResidArgs {
+  const uint16_t* A;     // bf16 row (b, t) at A + b * a_bstride + t * K
+  int64_t a_bstride;
+  const uint16_t* W;     // [N, K]
+  const uint16_t* W_ns;  // [n_ns, N, K], or null when n_ns == 0
+  int B, n_s, n_ns, N, K;  // N and K multiples of 128
+  float* out;            // row (b, t) at out + b * out_bstride + t * N
+  int64_t out_bstride;
+  const float* res;      // row (b, t) at res + b * res_bstride + (t + res_toff) * N; may be out
+  int64_t res_bstride;
+  int res_toff;
+  int round_bf16;
+  // filled by the launcher
+  int tiles_s, tiles_b;
+};
+int launch_resid_gemm(const ResidArgs& a, hipStream_t s);
+
 }  // namespace pdm

@@ -11,19 +11,15 @@
 //   y  = z + FFN(RMSNorm2(z)), FFN = W2 gelu_erf(W1 .), S shared / NS per token (:172-204)
 // Every GEMM takes bf16 operands, accumulates in fp32 and rounds its output
 // to bf16 (autocast), GELU runs in fp32 on the bf16 GEMM output and rounds
-// to bf16, the residual additions run in fp32.  Exception (d_model 128/256,
-// the fused FFN): the FFN-down accumulates on top of z in fp32, so its output
-// is not rounded to bf16 before the residual addition (at most half a bf16
+// to bf16, the residual additions run in fp32.  Exception: the FFN-down's
+// output is added to z in fp32, not rounded to bf16 first (at most half a bf16
 // ulp of the FFN output away from the autocast result).
 //
 // Launches per block: Q/K/V projection with RMSNorm1 in front (Q tail rows, K, and V transposed per head), attention,
-// then either out-projection + FFN in one kernel (d_model 128 / 256) or out-projection GEMM (+x tail -> z in y),
-// FFN-up with RMSNorm2 in front (row_proj.hip), FFN-down GEMM (+z -> y).
-//
-// GEMM design (out-projection, FFN-down of d_model 384 / 512): tiles of A[M,K] . W[N,K]^T (both K-contiguous, the
-// nn.Linear layout), each wave 2x2 v_mfma_f32_32x32x16_bf16 tiles, K streamed in 64-wide slices through LDS.  Rows are
-// (sample, token) pairs; S-token rows use the shared weight and NS-token rows the weight of their token, so one launch
-// covers the shared GEMM and the 16 per-token GEMMs.
+// then either out-projection + FFN in one kernel or out-projection (+x tail -> z in y, resid_gemm.hip), FFN-up with
+// RMSNorm2 in front (row_proj.hip), FFN-down (+z -> y, resid_gemm.hip).  Rows are (sample, token) pairs; S-token rows use
+// the shared weight and NS-token rows the weight of their token, so one launch covers the shared GEMM and the 16
+// per-token GEMMs.
 //
 // Attention design: one wave owns 32 queries of one (sample, head).  It
 // computes S^T = K Q^T so that each lane holds one query's scores; the
@@ -38,11 +34,6 @@
 #include "mfma_common.h"
 #include "block_kernels.h"
 
-// d_model 256 runs the Q/K/V projection weight-stationary (1) or as the row GEMM (0)
-#ifndef PDM_QKV_STATIONARY
-#define PDM_QKV_STATIONARY 1
-#endif
-
 namespace pdm {
 
 // ---------------------------------------------------------------------------
@@ -50,7 +41,7 @@ namespace pdm {
 // ---------------------------------------------------------------------------
 enum { EPI_BIAS_GELU = 0, EPI_BIAS_F32 = 1 };
 
-constexpr int GBM = 128, GBN = 128, GBK = 64, GPAD = 8;
+constexpr int GBM = 128, GBN = 128, GBK = 64;
 
 struct GemmArgs {
   const uint16_t* A;  // bf16 rows: row (b, t) at A + b * a_bstride + t * K
@@ -138,159 +129,6 @@ __device__ __forceinline__ int ns_tile_xcd_major(const GemmArgs& a, int mt) {
     pre += ck;
   }
   return mt;  // not reached
-}
-
-// LDS stages of gemm_kernel: 2 (double buffer, two workgroups per CU) or 1 (the next step waits in
-// registers; up to four workgroups per CU), and the workgroups per CU its registers are sized for
-#ifndef PDM_GEMM_STAGES
-#define PDM_GEMM_STAGES 1
-#endif
-#ifndef PDM_GEMM_WPS
-#define PDM_GEMM_WPS 4
-#endif
-constexpr int kGemmStages = PDM_GEMM_STAGES;
-// rows per tile of gemm_kernel: 128 (4 waves) or 256 (8 waves, each wave still 64 x 64)
-#ifndef PDM_GEMM_TM
-#define PDM_GEMM_TM 256
-#endif
-template <int TM>
-__global__ __launch_bounds__(TM * 2, kGemmStages == 1 ? (TM == GBM ? PDM_GEMM_WPS : 4) : 2) void gemm_kernel(GemmArgs a) {
-  constexpr int NT = TM * 2;                 // threads: TM / 64 x 2 waves
-  constexpr int RPP = NT / 8;                // tile rows per pass of 16-byte loads
-  constexpr int PA = TM / RPP, PB = GBN / RPP;  // passes of the A and W tiles
-  // the A and W tiles; after the k loop the epilogue stages its rows in the same bytes
-  constexpr int kAElems = kGemmStages * TM * (GBK + GPAD), kBElems = kGemmStages * GBN * (GBK + GPAD);
-  __shared__ __attribute__((aligned(16))) uint16_t sAB[kAElems + kBElems];
-  uint16_t (*sA)[TM][GBK + GPAD] = reinterpret_cast<uint16_t (*)[TM][GBK + GPAD]>(sAB);
-  uint16_t (*sB)[GBN][GBK + GPAD] = reinterpret_cast<uint16_t (*)[GBN][GBK + GPAD]>(sAB + kAElems);
-  __shared__ int s_rb[TM];  // sample of tile row i, -1 = no row
-  __shared__ int s_rt[TM];  // token of tile row i
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-
-  // blocks sharing an M tile run on one XCD (block ids are dealt to the 8 XCDs round robin)
-  int64_t bid = blockIdx.x;
-  const int64_t full = a.total_blocks & ~int64_t(7);
-  if (bid < full) bid = (bid & 7) * (full >> 3) + (bid >> 3);
-  const int mt = (int)(bid / a.n_tiles);
-  const int n0 = (int)(bid - (int64_t)mt * a.n_tiles) * GBN;
-
-  const uint16_t* W = a.W;
-  if (tid < TM) tile_row(a, mt, TM, tid, s_rb[tid], s_rt[tid]);
-  if (mt >= a.tiles_s) W = a.W_ns + (int64_t)((mt - a.tiles_s) / a.tiles_b) * a.N * a.K;
-  __syncthreads();
-
-  // global -> LDS assignment: 8 threads x 16 B per 64-element row slice, RPP rows per pass.  Rows are 32-bit
-  // element offsets from the tile's first row (-1: no row), which launch_gemm bounds.
-  const int lr = tid >> 3, lc = (tid & 7) * 8;
-  const int b0 = s_rb[0];  // row 0 of every tile is a row
-  const uint16_t* abase = a.A + (int64_t)b0 * a.a_bstride;
-  int aoff[PA], woff[PB];
-#pragma unroll
-  for (int p = 0; p < PA; ++p) {
-    const int i = p * RPP + lr;
-    const int b = s_rb[i];
-    aoff[p] = b >= 0 ? (int)((int64_t)(b - b0) * a.a_bstride + (int64_t)s_rt[i] * a.K + lc) : -1;
-  }
-#pragma unroll
-  for (int p = 0; p < PB; ++p) {
-    const int n = n0 + p * RPP + lr;
-    woff[p] = n < a.N ? n * a.K + lc : -1;
-  }
-
-  u32x4_t ra[PA], rb[PB];
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int p = 0; p < PA; ++p)
-      ra[p] = aoff[p] >= 0 ? *reinterpret_cast<const u32x4_t*>(abase + aoff[p] + k0) : u32x4_t{0, 0, 0, 0};
-#pragma unroll
-    for (int p = 0; p < PB; ++p)
-      rb[p] = woff[p] >= 0 ? *reinterpret_cast<const u32x4_t*>(W + woff[p] + k0) : u32x4_t{0, 0, 0, 0};
-  };
-  auto sstore = [&](int buf) {
-#pragma unroll
-    for (int p = 0; p < PA; ++p) *reinterpret_cast<u32x4_t*>(&sA[buf][p * RPP + lr][lc]) = ra[p];
-#pragma unroll
-    for (int p = 0; p < PB; ++p) *reinterpret_cast<u32x4_t*>(&sB[buf][p * RPP + lr][lc]) = rb[p];
-  };
-
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  const int nk = a.K / GBK;
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  const int fr = lane & 31, fk = (lane >> 5) * 8;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int buf = kGemmStages == 1 ? 0 : kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * GBK);
-#pragma unroll
-    for (int ks = 0; ks < GBK / 16; ++ks) {
-      u32x4_t af[2], bf[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) af[i] = *reinterpret_cast<const u32x4_t*>(&sA[buf][wm * 64 + i * 32 + fr][ks * 16 + fk]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) bf[j] = *reinterpret_cast<const u32x4_t*>(&sB[buf][wn * 64 + j * 32 + fr][ks * 16 + fk]);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x16(af[i], bf[j], acc[i][j]);
-    }
-    if constexpr (kGemmStages == 1) {
-      __syncthreads();  // every wave is done with the step's tile
-      if (kt + 1 < nk) sstore(0);
-    } else if (kt + 1 < nk) {
-      sstore(buf ^ 1);
-    }
-    __syncthreads();
-  }
-
-  // epilogue: acc[i][j][e] is row wm*64 + i*32 + (e/4)*8 + (lane/32)*4 + e%4, column n0 + wn*64 + j*32 + lane%32
-  const int hf = lane >> 5;
-  // 64 rows at a time through LDS (fp32, rows of 128 + 4): the two waves that hold them write their accumulators,
-  // then every thread finishes 4 consecutive outputs of a row with one 16-byte residual read and one 16-byte store.
-  // The k loop ended with a barrier.  N = d_model is a multiple of 128.
-  constexpr int OS = GBN + 4;  // sO row stride (floats)
-  static_assert((kAElems + kBElems) * 2 >= 64 * OS * 4, "the staging rows must fit in the A and W tiles");
-  float* sO = reinterpret_cast<float*>(sAB);
-#pragma unroll
-  for (int rr = 0; rr < TM / 64; ++rr) {
-    if (wm == rr) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            sO[(i * 32 + (e >> 2) * 8 + hf * 4 + (e & 3)) * OS + wn * 64 + j * 32 + fr] = acc[i][j][e];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < 64 * (GBN / 4) / NT; ++it) {
-      const int idx = it * NT + tid;
-      const int rl = idx / (GBN / 4), cv = idx % (GBN / 4);
-      const int row = rr * 64 + rl;
-      const int b = s_rb[row];
-      if (b < 0) continue;
-      const int t = s_rt[row];
-      const int n = n0 + cv * 4;
-      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(sO + rl * OS + cv * 4);
-      const f32x4_t r = *reinterpret_cast<const f32x4_t*>(
-          a.res + (int64_t)b * a.res_bstride + (int64_t)(t + a.res_toff) * a.N + n);
-      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(a.out) + (int64_t)b * a.out_bstride + (int64_t)t * a.N + n) =
-          f32x4_t{bf16_round(v[0]) + r[0], bf16_round(v[1]) + r[1], bf16_round(v[2]) + r[2], bf16_round(v[3]) + r[3]};
-    }
-    __syncthreads();  // sO is read before the next round writes it
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1320,10 +1158,20 @@ struct BlockLayout {
 
 static int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 
-// d_model 128 and 256 run the fused kernels (RMSNorm inside the GEMMs, FFN in
-// registers); other widths run the tiled GEMM path, which also needs the
-// normalised rows (h) and the GELU activations (g) in the workspace.
-static bool fused_path(const pdm_block_desc& d) { return d.d_model == 128 || d.d_model == 256; }
+// d_model 128, and 256 above kFusedMinRows kept rows, run the out-projection, RMSNorm2 and the FFN in one kernel, whose
+// tiles of 128 rows walk the whole hidden dimension one after another: 50 us at d_model 256 however few rows there are,
+// 53 us for 17,408 rows, 81 us for 34,816.  Below, and at d_model 384 / 512 (whose rows do not fit its registers), three
+// kernels split that work over the chip: 30 us for 4,352 rows, 57 us for 17,408, 112 us for 34,816.  (At d_model 128 the
+// one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three also need the normalised rows
+// (h) and the GELU activations (g) in the workspace.
+constexpr int64_t kFusedMinRows = 14000;
+static bool fused_path(const pdm_block_desc& d) {
+  return d.d_model == 128 || (d.d_model == 256 && (int64_t)d.batch * d.q_len > kFusedMinRows);
+}
+// d_model 256: rows of x from which the weight-stationary Q/K/V projection (384 KB of weight into every CU's registers
+// first: 34 us however few rows) is faster than the streaming one.  Per block: 6,400 rows 34 against 14 us, 51,200 rows
+// 62 against 49 us, 102,400 rows 277 against 274 us (whole block), 204,800 rows 448 against 461 us (whole block).
+constexpr int64_t kQkvStationaryMinRows = 120000;
 
 static BlockLayout block_layout(const pdm_block_desc& d) {
   BlockLayout L;
@@ -1360,22 +1208,6 @@ static void gemm_tiles(GemmArgs& g) {
   g.tiles_b = (g.B + GBM - 1) / GBM;
   g.n_tiles = (g.N + GBN - 1) / GBN;
   g.total_blocks = ((int64_t)g.tiles_s + (int64_t)g.n_ns * g.tiles_b) * g.n_tiles;
-}
-
-static int launch_gemm(GemmArgs& g, hipStream_t s) {
-  constexpr int TM = PDM_GEMM_TM;
-  g.tiles_s = (int)(((int64_t)g.B * g.n_s + TM - 1) / TM);
-  g.tiles_b = (g.B + TM - 1) / TM;
-  g.n_tiles = (g.N + GBN - 1) / GBN;
-  g.total_blocks = ((int64_t)g.tiles_s + (int64_t)g.n_ns * g.tiles_b) * g.n_tiles;
-  if (g.total_blocks == 0) return PDM_OK;
-  PDM_CHECK_ARG(g.total_blocks < (int64_t(1) << 31), "GEMM grid too large");
-  // 32-bit element offsets of a tile's A rows from its first row, and of the weight rows
-  PDM_CHECK_ARG((int64_t)TM * g.a_bstride + g.a_bstride < (int64_t(1) << 31), "GEMM rows too far apart");
-  PDM_CHECK_ARG((int64_t)g.N * g.K < (int64_t(1) << 31), "GEMM weight too large");
-  hipLaunchKernelGGL((gemm_kernel<TM>), dim3((unsigned)g.total_blocks), dim3(TM * 2), 0, s, g);
-  PDM_CHECK_LAUNCH();
-  return PDM_OK;
 }
 
 // Row tiles of rows_per_tile rows: the shared group's tiles, then tiles_b per NS token.
@@ -1499,7 +1331,7 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
   const int kv = d.kv_len, ql = d.q_len, nns = d.n_ns;
   int st;
 
-  if (fused_path(d) && D == 256 && PDM_QKV_STATIONARY) {
+  if (D == 256 && (int64_t)B * kv > kQkvStationaryMinRows) {
     // 1. Q (tail rows), K, V^T = RMSNorm1(x) . Wqkv^T  (weight-stationary, norm fused)
     QkvArgs qa{};
     qa.x = x; qa.x_bstride = (int64_t)kv * D; qa.norm_w = w->norm1_w;
@@ -1574,13 +1406,14 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
   }
   // 3. z = bf16(O . Wout^T) + x[:, kv - q_len:]  -> y
   {
-    GemmArgs g1{};
+    ResidArgs g1{};
+    g1.round_bf16 = 1;
     g1.A = q; g1.a_bstride = (int64_t)ql * D;
     g1.W = reinterpret_cast<const uint16_t*>(w->out_w);
     g1.B = B; g1.n_s = ql; g1.n_ns = 0; g1.N = D; g1.K = D;
     g1.out = y; g1.out_bstride = (int64_t)ql * D;
     g1.res = x; g1.res_bstride = (int64_t)kv * D; g1.res_toff = kv - ql;
-    if ((st = launch_gemm(g1, s)) != PDM_OK) return st;
+    if ((st = launch_resid_gemm(g1, s)) != PDM_OK) return st;
   }
   // 4. h = RMSNorm2(z)  [B, q_len, D], g = bf16(gelu(bf16(h2 . W1^T)))  [B, q_len, F]
   {
@@ -1594,14 +1427,14 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
   }
   // 5. y = z + bf16(g . W2^T)
   {
-    GemmArgs g3{};
+    ResidArgs g3{};
     g3.A = g; g3.a_bstride = (int64_t)ql * F;
     g3.W = reinterpret_cast<const uint16_t*>(w->s_w2);
     g3.W_ns = reinterpret_cast<const uint16_t*>(w->ns_w2);
     g3.B = B; g3.n_s = ql - nns; g3.n_ns = nns; g3.N = D; g3.K = F;
     g3.out = y; g3.out_bstride = (int64_t)ql * D;
     g3.res = y; g3.res_bstride = (int64_t)ql * D; g3.res_toff = 0;
-    if ((st = launch_gemm(g3, s)) != PDM_OK) return st;
+    if ((st = launch_resid_gemm(g3, s)) != PDM_OK) return st;
   }
   return PDM_OK;
 }

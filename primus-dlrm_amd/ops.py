@@ -648,13 +648,13 @@ def onetrans_workspace_layout(B: int, kv: int, q_len: int, D: int, F: int) -> Di
     """Byte (offset, size) of each region of the block workspace, as laid out by
     pdm_onetrans_block_fwd: q (Q tail rows [B, q_len, D] bf16, later the
     attention output), k ([B, kv, D] bf16), vt (V transposed per head [B, D/64,
-    64, kv_ld] bf16, kv_ld = kv rounded up to 64).  d_model 128 and 256 run
-    fused kernels; other widths also hold h (normalised rows [B, kv, D] bf16)
-    and g (GELU of the FFN-up GEMM [B, q_len, F] bf16)."""
+    64, kv_ld] bf16, kv_ld = kv rounded up to 64).  d_model 384 and 512, and 256 with
+    at most 14,000 kept rows, run the FFN as separate kernels and also hold h (RMSNorm2
+    rows [B, q_len, D] bf16) and g (GELU of the FFN-up GEMM [B, q_len, F] bf16)."""
     a = lambda v: (v + 255) // 256 * 256  # noqa: E731
     kv_ld = (kv + 63) // 64 * 64
     sizes = [("q", B * q_len * D * 2), ("k", B * kv * D * 2), ("vt", B * D * kv_ld * 2)]
-    if D not in (128, 256):
+    if D > 256 or (D == 256 and B * q_len <= 14000):
         sizes += [("h", B * kv * D * 2), ("g", B * q_len * F * 2)]
     out, off = {}, 0
     for name, n in sizes:

@@ -125,11 +125,14 @@ def test_block_d512_tiled_path(pdm, dev):
     (2, 30, 30, 0, 384),    # no NS tokens
     (3, 16, 16, 16, 384),   # no S tokens
     (140, 37, 24, 3, 384),  # NS tokens over two row tiles of 128 samples, the second partial
+    (300, 61, 45, 3, 384),  # 13,500 kept rows: 128 x 128 tiles of the residual projections, the last one partial
+    (330, 61, 43, 5, 256),  # 14,190 kept rows: just above the fused FFN's limit
+    (325, 61, 43, 5, 256),  # 13,975 kept rows: just below it
     (700, 101, 50, 2, 128),  # enough row tiles that no column split is made; 99 S tokens, Q of the tail only
 ])
 def test_block_row_projection_edges(pdm, dev, B, kv, q_len, n_ns, D):
     """The Q/K/V and FFN-up projections (32-token blocks of a sample, 32-sample blocks of an NS token, column
-    splits) at the edges of their blocks, with the tolerance of every block test."""
+    splits) and the residual projections at the edges of their blocks, with the tolerance of every block test."""
     _run_case(pdm, dev, B, kv, q_len, n_ns, D=D, F=2 * D, seed=B + kv, norm_std=0.1)
 
 
