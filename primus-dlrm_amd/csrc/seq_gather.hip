@@ -15,6 +15,13 @@
 // loads (pool offsets, event ids, table rows) are issued for all TPG tokens
 // before the next phase, so the three dependent memory round trips are paid
 // once per TPG tokens.
+//
+// A lane has NCH * TPG pieces in flight, six to eight of them: TPG 8 for rows of one piece per lane, 4 of two, 2 of
+// more, and rows past 64 pieces take more lanes instead of more pieces per lane (eight pieces of eight tokens held 256
+// registers and ran one wave per SIMD).  Bound by the output's bytes, 393,216 tokens (126 us for fp32 rows of 384 at a
+// device copy's rate): fp32 256 + 64 + 64 over 16 lanes x 8 pieces x 8 tokens 260 us, 32 x 3 x 8 151, 32 x 3 x 4 138,
+// 32 x 3 x 2 131; fp32 128 + 64 (16 x 3) 8 tokens 74.9, 2 tokens 70.1; fp32 128 (16 x 2) 8 tokens 52.5, 4 tokens 48.0,
+// 2 tokens 49.7; bf16 128 (16 x 1) 8 tokens 25.5, 4 tokens 26.4, 2 tokens 29.4.
 #include <algorithm>
 
 #include "pdm_common.h"
@@ -56,10 +63,6 @@ template <class T>
 __device__ __forceinline__ T load_global(const void* p) {
   return *reinterpret_cast<const __attribute__((address_space(1))) T*>(reinterpret_cast<uintptr_t>(p));
 }
-
-#ifndef PDM_SEQ_TOKENS_PER_GROUP
-#define PDM_SEQ_TOKENS_PER_GROUP 8
-#endif
 
 template <int VB, int NCH, int TPG>
 __global__ __launch_bounds__(256) void seq_gather_kernel(SeqArgs a) {
@@ -219,15 +222,15 @@ using namespace pdm;
 
 namespace {
 using SeqFn = void (*)(SeqArgs);
-constexpr int kTpg = PDM_SEQ_TOKENS_PER_GROUP;
+constexpr int tokens_per_group(int nch) { return nch == 1 ? 8 : (nch == 2 ? 4 : 2); }
 template <int VB>
 SeqFn pick_seq(int nch) {
   switch (nch) {
-    case 1: return seq_gather_kernel<VB, 1, kTpg>;
-    case 2: return seq_gather_kernel<VB, 2, kTpg>;
-    case 3: return seq_gather_kernel<VB, 3, kTpg>;
-    case 4: return seq_gather_kernel<VB, 4, kTpg>;
-    case 8: return seq_gather_kernel<VB, 8, kTpg>;
+    case 1: return seq_gather_kernel<VB, 1, tokens_per_group(1)>;
+    case 2: return seq_gather_kernel<VB, 2, tokens_per_group(2)>;
+    case 3: return seq_gather_kernel<VB, 3, tokens_per_group(3)>;
+    case 4: return seq_gather_kernel<VB, 4, tokens_per_group(4)>;
+    case 8: return seq_gather_kernel<VB, 8, tokens_per_group(8)>;
     default: return nullptr;
   }
 }
@@ -295,8 +298,7 @@ extern "C" int pdm_seq_gather_fwd(const pdm_seq_desc* desc, const void* const* t
   const int vb = vec16 ? 16 : 4;
   a.chunks = a.tok_bytes / vb;
   int lpb = 1;
-  const int lpb_cap = a.chunks > 16 * 8 ? 64 : 16;
-  while (lpb < a.chunks && lpb < lpb_cap) lpb <<= 1;
+  while (lpb < a.chunks && lpb < 64 && (lpb < 16 || lpb * 4 < a.chunks)) lpb <<= 1;
   int nch = (a.chunks + lpb - 1) / lpb;
   if (nch > 4 && nch <= 8) nch = 8;
   SeqFn fn = vb == 16 ? pick_seq<16>(nch) : pick_seq<4>(nch);
@@ -307,7 +309,7 @@ extern "C" int pdm_seq_gather_fwd(const pdm_seq_desc* desc, const void* const* t
   int sh = 0;
   while ((1 << sh) < lpb) ++sh;
   a.lpb_shift = sh;
-  const int64_t tok_per_block = 4 * (64 / lpb) * kTpg;
+  const int64_t tok_per_block = 4 * (64 / lpb) * tokens_per_group(nch);
   const int64_t blocks = (a.num_tokens + tok_per_block - 1) / tok_per_block;
   PDM_CHECK_ARG(blocks < (int64_t(1) << 31), "too many tokens for one launch");
   hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a);

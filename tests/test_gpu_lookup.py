@@ -352,6 +352,22 @@ def test_seq_gather_narrow_rows(pdm, dev, dims):
     assert np.array_equal(got, want) and np.array_equal(mask, wmask)
 
 
+@pytest.mark.parametrize("dims", [
+    (64,), (68,), (128,), (132,),           # 16, 17, 32, 33 pieces of 16 bytes: one, two and three per lane
+    (192, 64), (192, 68),                   # 64, 65 pieces: 16 lanes x 4, 32 lanes x 3
+    (384, 128), (388, 128), (1020, 4),      # 128, 129, 256 pieces: 32 x 4, 64 x 3, 64 x 4
+    (1024, 4), (2044, 4),                   # 257, 512 pieces: 64 x 8
+    (65,), (130, 127),                      # 4-byte pieces
+])
+def test_seq_gather_lane_group_edges(pdm, dev, dims):
+    """Rows at the edges of the lane groups (bytes are copied: bit exact), a token count that no group divides."""
+    g = np.random.default_rng(sum(dims))
+    tabs_t, ids, offs = _seq_case(g, 7, (6, 4), [9, 4], dims, tuple(40 + 7 * i for i in range(len(dims))), "fp32")
+    got, mask, want, wmask, err, _ = _seq_run(pdm, dev, tabs_t, ids, offs, [9, 4], 0, 0)
+    assert np.array_equal(mask, wmask) and err == 0
+    assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
 def test_seq_gather_bad_ids_zeroed_and_flagged(pdm, dev):
     g = np.random.default_rng(23)
     tabs_t, ids, offs = _seq_case(g, 5, (6, 6), [4, 4], (8, 8), (40, 40), "bf16")
