@@ -36,13 +36,6 @@
 
 namespace pdm {
 
-// ---------------------------------------------------------------------------
-// Grouped GEMM  C = A . W^T  over (sample, token) rows.
-// ---------------------------------------------------------------------------
-enum { EPI_BIAS_GELU = 0, EPI_BIAS_F32 = 1 };
-
-constexpr int GBM = 128, GBN = 128, GBK = 64;
-
 struct GemmArgs {
   const uint16_t* A;  // bf16 rows: row (b, t) at A + b * a_bstride + t * K
   int64_t a_bstride;  // elements between samples
@@ -52,12 +45,10 @@ struct GemmArgs {
   int n_s;    // tokens of the shared group per sample (tokens 0 .. n_s-1)
   int n_ns;   // per-token groups (tokens n_s .. n_s+n_ns-1); 0 when W_ns is null
   int N, K;
-  int tiles_s;  // ceil(B * n_s / GBM)
-  int tiles_b;  // ceil(B / GBM)
-  int n_tiles;  // ceil(N / GBN)
+  int tiles_s, tiles_b;  // row tiles of the shared group, and per NS token
   int64_t total_blocks;
   // epilogue
-  void* out;            // bf16 (EPI_BIAS_GELU) or fp32 [B, T, N]
+  void* out;            // fp32 [B, T, D]
   int64_t out_bstride;  // elements between samples of out
   const float* res;     // residual fp32, row (b, t) at res + b * res_bstride + (t + res_toff) * N
   int64_t res_bstride;
@@ -67,19 +58,8 @@ struct GemmArgs {
   const float* norm_w;    // RMSNorm2 weight
   const uint16_t* W2;     // FFN-down [D, F] shared
   const uint16_t* W2_ns;  // [n_ns, D, F]
-  const uint16_t* bias;   // EPI_BIAS_*: bf16 [N]
   const uint16_t* Wo;     // FFN with the out-projection in front: Wout [D, D], shared by every token
 };
-
-// Stores one output element (b, t, n) of a Linear with bias (one rounding after the bias, as autocast makes it): its
-// GELU in bf16, or the bf16 result as fp32 (the promotion of the token concat).
-template <int EPI>
-__device__ __forceinline__ void epilogue_store(const GemmArgs& a, int b, int t, int n, float v) {
-  const int64_t o = (int64_t)b * a.out_bstride + (int64_t)t * a.N + n;
-  const float x = bf16_round(v + bf16_bits_to_f32(a.bias[n]));
-  if constexpr (EPI == EPI_BIAS_GELU) reinterpret_cast<uint16_t*>(a.out)[o] = (uint16_t)bf16_bits(gelu_erf(x));
-  else reinterpret_cast<float*>(a.out)[o] = x;
-}
 
 // (sample, token) of row i of GEMM row tile mt, or b = -1 past the end.  Tiles
 // 0 .. tiles_s-1 hold the shared group's rows (sample-major, token minor), the
@@ -1203,13 +1183,6 @@ static const char* check_desc(const pdm_block_desc* d) {
   return nullptr;
 }
 
-static void gemm_tiles(GemmArgs& g) {
-  g.tiles_s = (int)(((int64_t)g.B * g.n_s + GBM - 1) / GBM);
-  g.tiles_b = (g.B + GBM - 1) / GBM;
-  g.n_tiles = (g.N + GBN - 1) / GBN;
-  g.total_blocks = ((int64_t)g.tiles_s + (int64_t)g.n_ns * g.tiles_b) * g.n_tiles;
-}
-
 // Row tiles of rows_per_tile rows: the shared group's tiles, then tiles_b per NS token.
 static int64_t row_tiles(GemmArgs& g, int rows_per_tile) {
   g.tiles_s = (int)(((int64_t)g.B * g.n_s + rows_per_tile - 1) / rows_per_tile);
@@ -1555,364 +1528,4 @@ extern "C" int pdm_onetrans_stack_fwd(const pdm_block_desc* desc, const int32_t*
     d.kv_len = d.q_len;
   }
   return PDM_OK;
-}
-
-// ---------------------------------------------------------------------------
-// NS tokens: the NS input rows (scalar-feature rows and dense parts, bf16,
-// zero-padded to a multiple of 64 columns), then AutoSplitTokenizer's two
-// Linear layers on the tiled GEMM with bias epilogues.
-// ---------------------------------------------------------------------------
-namespace pdm {
-
-struct NsArgs {
-  const char* tables[PDM_NS_MAX_PARTS];
-  const int64_t* ids[PDM_NS_MAX_PARTS];
-  int64_t rows[PDM_NS_MAX_PARTS];
-  const float* dense[PDM_NS_MAX_PARTS];
-  int64_t dense_stride[PDM_NS_MAX_PARTS];
-  int32_t col[2 * PDM_NS_MAX_PARTS + 1];  // first column of part j (scalar parts, then dense parts)
-  int32_t n_scalar, n_parts, f32_tables, K, K64;
-  int64_t B;
-  uint16_t* raw;  // [B, K64] bf16
-  int32_t* err;
-};
-
-// one wave per sample: part by part, lanes over the part's columns, bf16 (round to nearest even) out
-__global__ __launch_bounds__(256) void ns_raw_kernel(NsArgs a) {
-  const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (b >= a.B) return;
-  uint16_t* dst = a.raw + b * a.K64;
-  bool bad = false;
-  for (int j = 0; j < a.n_parts; ++j) {
-    const int c0 = a.col[j], w = a.col[j + 1] - c0;
-    if (j < a.n_scalar) {
-      const int64_t id = a.ids[j][b];
-      const bool ok = id >= 0 && id < a.rows[j];
-      bad |= !ok;
-      if (a.f32_tables) {
-        const float* row = reinterpret_cast<const float*>(a.tables[j]) + (ok ? id : 0) * w;
-        for (int c = lane; c < w; c += 64) dst[c0 + c] = ok ? (uint16_t)f32_to_bf16_bits(row[c]) : 0;
-      } else {
-        const uint16_t* row = reinterpret_cast<const uint16_t*>(a.tables[j]) + (ok ? id : 0) * w;
-        for (int c = lane; c < w; c += 64) dst[c0 + c] = ok ? row[c] : 0;
-      }
-    } else {
-      const int d = j - a.n_scalar;
-      const float* row = a.dense[d] + b * a.dense_stride[d];
-      for (int c = lane; c < w; c += 64) dst[c0 + c] = (uint16_t)f32_to_bf16_bits(row[c]);
-    }
-  }
-  for (int c = a.K + lane; c < a.K64; c += 64) dst[c] = 0;
-  if (bad && a.err) a.err[0] = 1;
-}
-
-// W1 [N, K] -> [N, K64] with zero columns K .. K64
-__global__ __launch_bounds__(256) void ns_pad_w1_kernel(const uint16_t* __restrict__ w1, uint16_t* __restrict__ w1p,
-                                                        int N, int K, int K64) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (int64_t)N * K64) return;
-  const int n = (int)(i / K64), k = (int)(i - (int64_t)n * K64);
-  w1p[i] = k < K ? w1[(int64_t)n * K + k] : 0;
-}
-
-// Tiled GEMM for the NS tokenizer's Linear layers, C = A . W^T (+ bias epilogue), A [M, K] rows with stride
-// a_bstride, W [N, K], K a multiple of 64.  A 128 x 128 tile per workgroup of 8 waves, two per SIMD: waves w
-// and w + 4 compute the same 64 x 64 quarter of the tile over the two halves of every 64-wide k step.  The
-// LDS reads per MFMA are those of one wave per quarter (each 32x32x16 fragment feeds two MFMAs of the
-// wave's 2 x 2 tiles), but every SIMD has a second wave to issue while one waits; the two halves are added
-// through LDS at the end.  A and W tiles go global -> LDS by LDS DMA (global_load_lds_dwordx4, no staging registers) into an
-// NST-stage ring filled NST - 1 steps ahead; a tile row of 128 bytes holds 16-byte piece v of row r at
-// slot v ^ ((r >> 1) & 7), so the rows of one fragment read spread over all banks.  Rows past M or N read
-// the last row (their outputs are not stored).
-constexpr int kNsStages = 4;
-constexpr int kNsTileBytes = GBM * GBK * 2;  // one 128 x 64 bf16 tile
-
-__device__ __forceinline__ uint32_t ns_slot(int r, int v) { return (uint32_t)((v ^ ((r >> 1) & 7)) << 4); }
-
-template <int EPI, int NST>
-__global__ __launch_bounds__(512, 1) void ns_gemm_kernel(GemmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  char* sA = smem;                          // [NST][kNsTileBytes]
-  char* sB = smem + NST * kNsTileBytes;     // [NST][kNsTileBytes]
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q = wave & 3, kh = wave >> 2;
-  const int wm = q >> 1, wn = q & 1;
-  const int64_t bid = blockIdx.x;
-  int mt, nt;
-  if (a.n_tiles % 8 == 0) {
-    const int per = a.n_tiles / 8;
-    const int64_t x = bid & 7, j = bid >> 3;  // j-th block of XCD x: an eighth of the N tiles, every M tile
-    mt = (int)(j % a.tiles_s);
-    nt = (int)(x * per + j / a.tiles_s);
-  } else {
-    mt = (int)(bid / a.n_tiles);
-    nt = (int)(bid - (int64_t)mt * a.n_tiles);
-  }
-  const int m0 = mt * GBM, n0 = nt * GBN;
-  const int M = a.B;
-
-  // DMA: wave w loads chunks 2w, 2w + 1 (8 rows each) of the A tile and of the W tile; lane l of chunk c
-  // fills LDS slot l % 8 of tile row 8c + l / 8 with the piece that slot holds
-  uint32_t offa[2], offb[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int r = (2 * wave + h) * 8 + (lane >> 3), slot = lane & 7;
-    const int v = slot ^ ((r >> 1) & 7);
-    const int ra = min(m0 + r, M - 1) - m0, rb = min(n0 + r, a.N - 1) - n0;
-    offa[h] = (uint32_t)(((int64_t)ra * a.a_bstride + v * 8) * 2);
-    offb[h] = (uint32_t)(((int64_t)rb * a.K + v * 8) * 2);
-  }
-  const uint64_t abase = (uint64_t)(uintptr_t)(a.A + (int64_t)m0 * a.a_bstride);
-  const uint64_t wbase = (uint64_t)(uintptr_t)(a.W + (int64_t)n0 * a.K);
-  const int nk = a.K / GBK;
-  auto dma = [&](int kt, int stg) {
-    const uint64_t k2 = (uint64_t)kt * GBK * 2;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      lds_dma16(abase + k2, offa[h], (uint32_t)(uintptr_t)(sA + stg * kNsTileBytes + (2 * wave + h) * 1024));
-      lds_dma16(wbase + k2, offb[h], (uint32_t)(uintptr_t)(sB + stg * kNsTileBytes + (2 * wave + h) * 1024));
-    }
-  };
-
-  f32x16_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-
-  const int fr = lane & 31, hf = lane >> 5;
-  auto compute = [&](int stg) {
-    const char* ta = sA + stg * kNsTileBytes;
-    const char* tb = sB + stg * kNsTileBytes;
-#pragma unroll
-    for (int s2 = 0; s2 < 2; ++s2) {
-      const int v = (kh * 2 + s2) * 2 + hf;  // 16-byte piece of k = (kh*2 + s2)*16 + hf*8
-      u32x4_t af[2], bf[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int r = wm * 64 + i * 32 + fr;
-        af[i] = *reinterpret_cast<const u32x4_t*>(ta + r * 128 + ns_slot(r, v));
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int r = wn * 64 + j * 32 + fr;
-        bf[j] = *reinterpret_cast<const u32x4_t*>(tb + r * 128 + ns_slot(r, v));
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = mfma32x32x16(af[i], bf[j], acc[i][j]);
-    }
-  };
-  constexpr int PF = NST - 1;
-#pragma unroll
-  for (int j = 0; j < PF; ++j) dma(min(j, nk - 1), j);
-  // before the barrier of step kt every DMA but the 4 * (PF - 1) issued for steps kt + 1 .. kt + PF - 1 has
-  // landed (vector memory completes in issue order)
-  constexpr unsigned kWait = 0x0F70u | (unsigned)(4 * (PF - 1));
-  static_assert(4 * (PF - 1) < 16, "vmcnt immediate");
-  for (int kt = 0; kt < nk; ++kt) {
-    __builtin_amdgcn_s_waitcnt(kWait);
-    __syncthreads();  // step kt is in LDS; every wave is done with step kt - 1, whose stage is refilled
-    // unconditional (past the end it reloads the last step into the freed stage, read by no later step)
-    dma(min(kt + PF, nk - 1), (kt + PF) % NST);
-    compute(kt % NST);
-  }
-  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // no DMA may land in LDS after this point
-  __syncthreads();
-  // the second k half adds its quarter into the first through LDS: element e of acc[i][j] of lane l at
-  // float ((q * 64 + (i * 2 + j) * 16 + e) * 64 + l)
-  float* red = reinterpret_cast<float*>(smem);
-  if (kh == 1) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) red[(q * 64 + (i * 2 + j) * 16 + e) * 64 + lane] = acc[i][j][e];
-  }
-  __syncthreads();
-  if (kh == 1) return;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] += red[(q * 64 + (i * 2 + j) * 16 + e) * 64 + lane];
-
-  // epilogue: acc[i][j][e] is row wm*64 + i*32 + (e/4)*8 + hf*4 + e%4, column n0 + wn*64 + j*32 + lane%32
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int m = m0 + wm * 64 + i * 32 + (e >> 2) * 8 + hf * 4 + (e & 3);
-      if (m >= M) continue;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int n = n0 + wn * 64 + j * 32 + fr;
-        if (n < a.N) epilogue_store<EPI>(a, m, 0, n, acc[i][j][e]);
-      }
-    }
-}
-
-template <int EPI>
-static int launch_ns_gemm(GemmArgs& g, hipStream_t s) {
-  gemm_tiles(g);
-  if (g.total_blocks == 0) return PDM_OK;
-  PDM_CHECK_ARG(g.total_blocks < (int64_t(1) << 31), "GEMM grid too large");
-  // 32-bit per-lane DMA offsets within a tile's rows
-  PDM_CHECK_ARG((int64_t)GBM * std::max<int64_t>(g.a_bstride, g.K) * 2 < (int64_t(1) << 31), "rows too long");
-  constexpr int lds = 2 * kNsStages * kNsTileBytes;
-  static std::once_flag once[64];
-  static hipError_t err[64];
-  int dev = 0;
-  PDM_CHECK_HIP(hipGetDevice(&dev));
-  PDM_CHECK_ARG(dev >= 0 && dev < 64, "device index out of range");
-  std::call_once(once[dev], [&] {
-    err[dev] = hipFuncSetAttribute(reinterpret_cast<const void*>(ns_gemm_kernel<EPI, kNsStages>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  });
-  PDM_CHECK_HIP(err[dev]);
-  hipLaunchKernelGGL((ns_gemm_kernel<EPI, kNsStages>), dim3((unsigned)g.total_blocks), dim3(512), lds, s, g);
-  PDM_CHECK_LAUNCH();
-  return PDM_OK;
-}
-
-struct NsLayout {
-  int64_t raw, h, w1p, total;
-};
-
-// Row stride (elements) of the hidden activations h: N plus one 128-byte line, so that the rows an XCD's
-// tiles read at one k step do not all fall into the same few L2 sets (N is a multiple of 64).
-static int64_t ns_h_stride(int64_t N) { return N + 64; }
-
-static NsLayout ns_layout(int64_t B, int64_t K64, int64_t N) {
-  NsLayout l{};
-  l.raw = 0;
-  l.h = align256(B * K64 * 2);
-  l.w1p = l.h + align256(B * ns_h_stride(N) * 2);
-  l.total = l.w1p + align256(N * K64 * 2);
-  return l;
-}
-
-static const char* check_ns_desc(const pdm_ns_desc* d, int& K) {
-  if (!d) return "null desc";
-  if (d->num_scalar < 0 || d->num_scalar > PDM_NS_MAX_PARTS || d->num_dense < 0 || d->num_dense > PDM_NS_MAX_PARTS)
-    return "num_scalar and num_dense must be in [0, 8]";
-  if (d->num_scalar + d->num_dense == 0) return "no NS input parts";
-  if (d->table_dtype != PDM_F32 && d->table_dtype != PDM_BF16) return "table_dtype must be F32 or BF16";
-  if (d->n_out < 8 || d->n_out % 8 != 0) return "n_out must be a positive multiple of 8";
-  if (d->batch_size < 0) return "batch_size < 0";
-  K = 0;
-  for (int j = 0; j < d->num_scalar; ++j) {
-    if (d->scalar_dim[j] <= 0 || d->scalar_rows[j] < 0) return "bad scalar table shape";
-    K += d->scalar_dim[j];
-  }
-  for (int j = 0; j < d->num_dense; ++j) {
-    if (d->dense_dim[j] <= 0) return "bad dense part width";
-    K += d->dense_dim[j];
-  }
-  return nullptr;
-}
-
-}  // namespace pdm
-
-extern "C" int64_t pdm_ns_tokenize_workspace_size(const pdm_ns_desc* desc) {
-  clear_error();
-  int K = 0;
-  if (const char* e = check_ns_desc(desc, K)) {
-    set_error(std::string("pdm_ns_tokenize_workspace_size: ") + e);
-    return -1;
-  }
-  return ns_layout(desc->batch_size, (K + GBK - 1) / GBK * GBK, desc->n_out).total;
-}
-
-extern "C" int pdm_ns_tokenize_fwd(const pdm_ns_desc* desc, const void* const* tables, const int64_t* const* ids,
-                                   const float* const* dense, const int64_t* dense_stride, const uint16_t* w1,
-                                   const uint16_t* b1, const uint16_t* w2, const uint16_t* b2, float* out,
-                                   int64_t out_sample_stride, void* workspace, int64_t workspace_bytes,
-                                   int32_t* err_flag, pdm_stream_t stream) {
-  clear_error();
-  int K = 0;
-  if (const char* e = check_ns_desc(desc, K)) {
-    set_error(std::string("pdm_ns_tokenize_fwd: ") + e);
-    return PDM_ERR_INVALID;
-  }
-  const pdm_ns_desc& d = *desc;
-  const int N = d.n_out;
-  const int K64 = (K + GBK - 1) / GBK * GBK;
-  if (d.batch_size == 0) return PDM_OK;
-  PDM_CHECK_ARG(d.batch_size < (int64_t(1) << 31), "batch_size too large");
-  PDM_CHECK_ARG(w1 && b1 && w2 && b2 && out, "null weight or output pointer");
-  PDM_CHECK_ARG(((uintptr_t)w2 & 15) == 0 && ((uintptr_t)w1 & 1) == 0, "w2 must be 16-byte aligned");
-  PDM_CHECK_ARG(out_sample_stride >= N, "out_sample_stride must be >= n_out");
-  PDM_CHECK_ARG(N % GBK == 0, "n_out must be a multiple of 64");
-  NsArgs a{};
-  a.n_scalar = d.num_scalar;
-  a.n_parts = d.num_scalar + d.num_dense;
-  a.f32_tables = d.table_dtype == PDM_F32;
-  int col = 0;
-  for (int j = 0; j < d.num_scalar; ++j) {
-    PDM_CHECK_ARG(tables && ids && tables[j] && ids[j], "null scalar table or ids pointer");
-    a.tables[j] = reinterpret_cast<const char*>(tables[j]);
-    a.ids[j] = ids[j];
-    a.rows[j] = d.scalar_rows[j];
-    a.col[j] = col;
-    col += d.scalar_dim[j];
-  }
-  for (int j = 0; j < d.num_dense; ++j) {
-    PDM_CHECK_ARG(dense && dense_stride && dense[j], "null dense pointer");
-    PDM_CHECK_ARG(dense_stride[j] >= d.dense_dim[j], "dense_stride must be >= dense_dim");
-    a.dense[j] = dense[j];
-    a.dense_stride[j] = dense_stride[j];
-    a.col[d.num_scalar + j] = col;
-    col += d.dense_dim[j];
-  }
-  a.col[a.n_parts] = col;
-  a.K = K;
-  a.K64 = K64;
-  a.B = d.batch_size;
-  a.err = err_flag;
-  const NsLayout lay = ns_layout(d.batch_size, K64, N);
-  PDM_CHECK_ARG(workspace != nullptr && ((uintptr_t)workspace & 255) == 0, "workspace must be 256-byte aligned");
-  PDM_CHECK_ARG(workspace_bytes >= lay.total, "workspace too small");
-  char* ws = reinterpret_cast<char*>(workspace);
-  a.raw = reinterpret_cast<uint16_t*>(ws + lay.raw);
-  uint16_t* h = reinterpret_cast<uint16_t*>(ws + lay.h);
-  uint16_t* w1p = reinterpret_cast<uint16_t*>(ws + lay.w1p);
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-
-  hipLaunchKernelGGL(ns_raw_kernel, dim3((unsigned)((d.batch_size + 3) / 4)), dim3(256), 0, s, a);
-  PDM_CHECK_LAUNCH();
-  const int64_t wn = (int64_t)N * K64;
-  hipLaunchKernelGGL(ns_pad_w1_kernel, dim3((unsigned)((wn + 255) / 256)), dim3(256), 0, s, w1, w1p, N, K, K64);
-  PDM_CHECK_LAUNCH();
-  GemmArgs g{};
-  g.B = (int)d.batch_size;
-  g.n_s = 1;
-  g.n_ns = 0;
-  // Linear 1: h = bf16(gelu(bf16(raw . W1^T + b1)))
-  g.A = a.raw;
-  g.a_bstride = K64;
-  g.W = w1p;
-  g.N = N;
-  g.K = K64;
-  g.bias = b1;
-  g.out = h;
-  g.out_bstride = ns_h_stride(N);
-  if (int st = launch_ns_gemm<EPI_BIAS_GELU>(g, s)) return st;
-  // Linear 2: out = float(bf16(h . W2^T + b2))
-  g.A = h;
-  g.a_bstride = ns_h_stride(N);
-  g.W = w2;
-  g.K = N;
-  g.bias = b2;
-  g.out = out;
-  g.out_bstride = out_sample_stride;
-  return launch_ns_gemm<EPI_BIAS_F32>(g, s);
 }

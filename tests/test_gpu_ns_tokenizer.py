@@ -76,6 +76,24 @@ def test_ns_tokenize_matches_oracle(pdm, dev, case):
     _check(out.cpu(), tabs, ids, dense, w, n_ns)
 
 
+@pytest.mark.parametrize("B,dense_dims,d,n_ns", [
+    (1, [9], 64, 1),        # one row, one 64 x 64 tile, one k stage in both layers
+    (256, [396], 256, 16),  # 256 tiles of 64 x 64: the most that are used
+    (257, [396], 256, 16),  # 320: tiles of 128 x 128, the last row tile holds one row
+    (3270, [64], 64, 5),    # N = 320: a half-filled column tile, an odd number of stages; W1 read without padding
+    (65, [65, 62], 64, 3),  # two row tiles of 64 x 64, the second of one row; K one short of two stages
+])
+def test_ns_tokenize_tile_edges(pdm, dev, B, dense_dims, d, n_ns):
+    """Both tile shapes of the Linear layers at their edges, with the tolerance of every NS test."""
+    g = np.random.default_rng(B)
+    tabs, ids, dense = _parts(g, B, [], dense_dims, "bf16")
+    w = ot.random_autosplit_weights(sum(dense_dims), d * n_ns, seed=B)
+    wb = {k: v.to(torch.bfloat16).contiguous().to(dev) for k, v in w.items()}
+    out = pdm.ops.ns_tokenize_raw(*_dev(tabs, ids, dense, dev), wb["w1"], wb["b1"], wb["w2"], wb["b2"], n_ns)
+    torch.cuda.synchronize()
+    _check(out.cpu(), tabs, ids, dense, w, n_ns)
+
+
 def test_ns_tokens_into_block_input_and_bad_ids(pdm, dev):
     """out = the NS rows of a [B, S + n_ns, d] block input (S rows untouched); an id outside its table reads
     zeros and raises the flag."""
