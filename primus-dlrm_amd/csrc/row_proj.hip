@@ -76,6 +76,19 @@ __device__ __forceinline__ void quarter_swap(uint32_t& a, uint32_t& b) {
   b = r[1];
 }
 
+// sum over the 16 lanes of a row, in every lane: the butterfly's additions (after each rotation the sums repeat with
+// its period, so lane i - n holds what lane i ^ n does), without its trips through LDS
+__device__ __forceinline__ float row16_sum(float v) {
+  auto ror = [](float x, auto n) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 | decltype(n)::value, 0xf, 0xf, true));
+  };
+  v += ror(v, std::integral_constant<int, 8>{});
+  v += ror(v, std::integral_constant<int, 4>{});
+  v += ror(v, std::integral_constant<int, 2>{});
+  v += ror(v, std::integral_constant<int, 1>{});
+  return v;
+}
+
 // The 32 x 32 output tile whose line l % 32 (a row, or a feature of V^T) lies in lanes l and l + 32, packed to bf16
 // (dword j of half h: outputs 16 h + 8 (j / 2) + 4 (l / 32) + 2 (j % 2) and the next), regrouped so that 16-byte
 // stores write whole 64-byte segments: part 0 are lines 0..15, part 1 lines 16..31, lane l of part i holding
@@ -167,12 +180,13 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
   if constexpr (EPI == ROWPROJ_GELU)
     for (int i = tid; i < kGeluN; i += 256) gelu_t[i] = gelu_tail(__builtin_bit_cast(float, (kGeluLo + (uint32_t)i) << 16));
 
-  // RMSNorm: 16 lanes per fp32 row (256-byte segments), SL rows in flight; the bf16 rows pass through the wave's part
-  // of the (still unused) ring into the fragment layout
+  // RMSNorm: 16 lanes per fp32 row (256-byte segments), LD rows in flight (all 32 where the registers hold them); the
+  // bf16 rows pass, SL at a time, through the wave's part of the (still unused) ring into the fragment layout
   u32x4_t af[KS];
   {
     const int64_t rstride = is_s ? D : a.in_bstride;  // elements between the wave's rows
     constexpr int SL = D <= 384 ? 16 : 8, NV = D / 64, STR = 2 * D + 16;
+    constexpr int LD = D <= 256 ? 32 : SL;  // rows in flight
     static_assert(4 * SL * STR <= NST * CHUNK, "the row scratch lies in the weight ring");
     char* sc = lds + wave * SL * STR;
     const float* x0 = a.x + (int64_t)b0 * a.in_bstride + (int64_t)t0 * D;
@@ -181,33 +195,34 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
     f32x4_t w[NV];
 #pragma unroll
     for (int j = 0; j < NV; ++j) w[j] = *reinterpret_cast<const f32x4_t*>(a.norm_w + j * 64 + sub * 4);
+    f32x4_t v[LD / 4][NV];
 #pragma unroll
     for (int sl = 0; sl < 32 / SL; ++sl) {
-      f32x4_t v[SL / 4][NV];
+      if (sl * SL % LD == 0) {
 #pragma unroll
-      for (int p = 0; p < SL / 4; ++p) {
-        const float* xr = x0 + min(sl * SL + p * 4 + rq, last) * rstride + sub * 4;
+        for (int p = 0; p < LD / 4; ++p) {
+          const float* xr = x0 + min(sl * SL + p * 4 + rq, last) * rstride + sub * 4;
 #pragma unroll
-        for (int j = 0; j < NV; ++j) v[p][j] = *reinterpret_cast<const f32x4_t*>(xr + j * 64);
+          for (int j = 0; j < NV; ++j) v[p][j] = *reinterpret_cast<const f32x4_t*>(xr + j * 64);
+        }
+        // every load is in flight before the first is used (left to itself the compiler loads and reduces 4 rows at a
+        // time, one memory latency each)
+        __builtin_amdgcn_sched_barrier(0);
       }
-      // every load of the slice is in flight before the first is used (left to itself the compiler loads and
-      // reduces 4 rows at a time, one memory latency each)
-      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int p = 0; p < SL / 4; ++p) {
+        const f32x4_t(&u)[NV] = v[sl * SL % LD / 4 + p];
         float ss = 0.0f;
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-          ss += (v[p][j].x * v[p][j].x + v[p][j].y * v[p][j].y) + (v[p][j].z * v[p][j].z + v[p][j].w * v[p][j].w);
-#pragma unroll
-        for (int m = 8; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+        for (int j = 0; j < NV; ++j) ss += (u[j].x * u[j].x + u[j].y * u[j].y) + (u[j].z * u[j].z + u[j].w * u[j].w);
+        ss = row16_sum(ss);
         const float rms = 1.0f / sqrtf(ss / (float)D + 1e-6f);
         const int r = sl * SL + p * 4 + rq;
         uint16_t* hr = h0 + (int64_t)r * rstride + sub * 4;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
-          const u32x2_t n = u32x2_t{pack_bf16x2((v[p][j].x * rms) * w[j].x, (v[p][j].y * rms) * w[j].y),
-                                    pack_bf16x2((v[p][j].z * rms) * w[j].z, (v[p][j].w * rms) * w[j].w)};
+          const u32x2_t n = u32x2_t{pack_bf16x2((u[j].x * rms) * w[j].x, (u[j].y * rms) * w[j].y),
+                                    pack_bf16x2((u[j].z * rms) * w[j].z, (u[j].w * rms) * w[j].w)};
           if (EPI == ROWPROJ_GELU && part == 0 && r < rows) *reinterpret_cast<u32x2_t*>(hr + j * 64) = n;
           *reinterpret_cast<u32x2_t*>(sc + (p * 4 + rq) * STR + j * 128 + sub * 8) = n;
         }
@@ -384,14 +399,20 @@ static int launch_one(RowProjArgs a, hipStream_t s) {
   const int64_t wgs_s = ((int64_t)a.B * a.blocks_per_sample + 3) / 4;
   a.tiles_per_token = (a.B + 127) / 128;
   const int64_t wgs_ns = (int64_t)a.n_ns * a.tiles_per_token;
-  // column splits: as many as keep the grid within one round (two workgroups per CU), of at least two chunks each for
-  // the S tiles; what is left of the round goes to the NS tiles, down to single chunks: their weight is read from memory
-  // by few workgroups, and their V^T goes out in 2-byte stores (500 samples of 98 tokens, d 384: Q/K/V 111 -> 81 us
-  // with the NS tiles split)
+  // column splits: as many as keep the grid within one workgroup per CU, of at least two chunks each for the S tiles; a
+  // second workgroup per CU only where the first round leaves no room for a split.  Every split reads and normalises its
+  // tile's rows again, and at two per CU that took 5.0 us of a launch's 12 (one per CU 3.8; d 256, FFN-up of 16 samples
+  // of 272 tokens).  One round against two, stacks in us: d 256 B = 16 198 / 202, B = 4 167 / 170, d 384 B = 8 810 / 830,
+  // d 512 B = 4 305 / 321; without a split against two: d 256 B = 48 312 / 303, d 128 B = 100 194 / 183.
+  // What is left of the round goes to the NS tiles, down to single chunks: their weight is read from memory by few
+  // workgroups, and their V^T goes out in 2-byte stores (500 samples of 98 tokens, d 384: Q/K/V 111 -> 81 us with the NS
+  // tiles split).
   const int nchunks = a.N / 32;
-  constexpr int64_t kRound = 512;
-  a.split_s = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks / 2, kRound / std::max<int64_t>(1, wgs_s + wgs_ns)));
-  a.split_ns = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks, (kRound - wgs_s * a.split_s) / std::max<int64_t>(1, wgs_ns)));
+  constexpr int64_t kCus = 256;
+  const int64_t tiles = std::max<int64_t>(1, wgs_s + wgs_ns);
+  const int64_t round = 2 * tiles <= kCus ? kCus : 2 * kCus;
+  a.split_s = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks / 2, round / tiles));
+  a.split_ns = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks, (round - wgs_s * a.split_s) / std::max<int64_t>(1, wgs_ns)));
   const int64_t grid = wgs_s * a.split_s + wgs_ns * a.split_ns;
   if (grid == 0) return PDM_OK;
   PDM_CHECK_ARG(grid < (int64_t(1) << 31), "row projection grid too large");
