@@ -593,6 +593,7 @@ struct AttnArgs {
   int vt_ld;                     // V^T row stride in memory (kv rounded up to 64)
   float scale_log2;  // log2(e) / sqrt(64)
   int q_lds;         // attn_lds_kernel with 8 waves: Q of a head staged in LDS after K and V^T
+  int parts;         // attn_lds_kernel with 8 waves: workgroups that share the query tiles of a head
 };
 
 // ---------------------------------------------------------------------------
@@ -601,6 +602,9 @@ struct AttnArgs {
 // blockIdx.x + gridDim.x, ...  K rows and V^T rows of a head are read from
 // memory into registers while the previous head is computed, and written to
 // LDS between two barriers, so the copy hides behind the attention math.
+// With `parts` workgroups per head (one pass, the grid is parts * heads) workgroup
+// part * heads + head takes every parts-th wave's tiles of its head; O goes over Q, and
+// a wave uses only the Q rows of its own tiles, before it writes them.
 // Each wave sweeps 32-query tiles over the key tiles up to its causal limit
 // with no further barriers.  Query tiles go to waves in snake order of
 // decreasing cost (the causal sweep of tile t covers t + 1 key tiles), so the
@@ -841,9 +845,12 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_lds_kernel(AttnArgs a) {
   };
 
   const int ntiles = (a.q_len + 31) >> 5;
+  const int parts = NW == 8 ? a.parts : 1;
+  const int part = NW == 8 ? (int)blockIdx.x / BH : 0;  // 0 with one part: the grid is then at most BH
   // k-th tile of this wave in snake order (index into tiles sorted by decreasing cost), or -1
   auto tile_of = [&](int k) {
-    const int idx = NW * k + ((k & 1) ? NW - 1 - wave : wave);
+    const int nw = NW * parts, w = wave * parts + part;
+    const int idx = nw * k + ((k & 1) ? nw - 1 - w : w);
     return idx < ntiles ? ntiles - 1 - idx : -1;
   };
 
@@ -879,7 +886,7 @@ __global__ __launch_bounds__(NW * 64, 8 / NW) void attn_lds_kernel(AttnArgs a) {
   // With 4 waves (heads of at most 4 query tiles: one tile per wave) the wave's tile of the next head has its
   // Q requested during this head, like the next head's K and V^T.
   constexpr bool kQNext = NW == 4;
-  int bh = blockIdx.x;
+  int bh = (int)blockIdx.x - part * BH;
   u32x4_t qf[4], qn[4];
   const bool q_lds = !kQNext && a.q_lds;
   if constexpr (kQNext) qload(bh, max(tile_of(0), 0), qf);
@@ -1248,7 +1255,7 @@ constexpr int64_t kAttnLdsLimit = 160 * 1024;
 // fit on the device at once, each walking (sample, head) pairs.  The LDS limit
 // is raised above the default 64 KiB once per process, device and instance.
 template <int NP, int NW>
-static int launch_attn_lds(const AttnArgs& aa, int64_t lds, hipStream_t s) {
+static int launch_attn_lds(AttnArgs aa, int64_t lds, hipStream_t s) {
   static std::once_flag once[64];
   static hipError_t err[64];
   static int ncu[64];
@@ -1269,7 +1276,20 @@ static int launch_attn_lds(const AttnArgs& aa, int64_t lds, hipStream_t s) {
   PDM_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_lds_kernel<NP, NW>, NW * 64, (size_t)lds));
   const int64_t bh = (int64_t)aa.B * aa.H;
   PDM_CHECK_ARG(bh < (int64_t(1) << 31), "batch * heads too large");
-  const int64_t grid = std::min<int64_t>(bh, (int64_t)std::max(ncu[dev], 1) * std::max(per_cu, 1));
+  int64_t grid = std::min<int64_t>(bh, (int64_t)std::max(ncu[dev], 1) * std::max(per_cu, 1));
+  // Few heads leave CUs idle while a head's waves share four SIMDs: up to four workgroups then share its query tiles,
+  // each with its own copy of K and V^T (Q straight from memory).  1 / 2 / 4 workgroups per head, stacks in us:
+  // 4 layers d 256, B = 16 (64 heads, 9 tiles) 200.7 / 194.8 / 187.5; 3 layers d 256, B = 1, 596 keys 160.6 / 139.4 /
+  // 134.7, d 128, B = 60, 596 keys (120 heads, so two) 203.7 / 179.2; eight were no faster than four.
+  aa.parts = 1;
+  if (NW == 8) {
+    const int64_t tiles = (aa.q_len + 31) / 32;
+    aa.parts = (int)std::max<int64_t>(1, std::min<int64_t>({4, tiles, (int64_t)std::max(ncu[dev], 1) / bh}));
+  }
+  if (aa.parts > 1) {
+    aa.q_lds = 0;
+    grid = bh * aa.parts;
+  }
   hipLaunchKernelGGL((attn_lds_kernel<NP, NW>), dim3((unsigned)grid), dim3(NW * 64), (unsigned)lds, s, aa);
   PDM_CHECK_LAUNCH();
   return PDM_OK;

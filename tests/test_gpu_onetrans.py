@@ -119,6 +119,18 @@ def test_block_d512_tiled_path(pdm, dev):
 
 
 @pytest.mark.parametrize("B,kv,q_len,n_ns,D", [
+    (1, 608, 608, 5, 128),   # 19 query tiles on four workgroups per head, the longest keys held in LDS
+    (2, 300, 20, 4, 256),    # one query tile: one workgroup
+    (3, 290, 65, 4, 128),    # three tiles, the last of one row: three workgroups
+    (64, 290, 70, 2, 128),   # 128 heads: two workgroups each
+    (65, 290, 70, 2, 128),   # 130 heads: one each
+])
+def test_block_attention_workgroups_per_head(pdm, dev, B, kv, q_len, n_ns, D):
+    """The split of a head's query tiles over workgroups at its edges, with the tolerance of every block test."""
+    _run_case(pdm, dev, B, kv, q_len, n_ns, D=D, F=2 * D, seed=B + kv, norm_std=0.1)
+
+
+@pytest.mark.parametrize("B,kv,q_len,n_ns,D", [
     (1, 5, 5, 4, 384),      # one S token: a block of 31 padding rows, every column split of the small grid
     (2, 47, 20, 7, 128),    # 40 S tokens: the last block stores one run of 8 V^T tokens
     (3, 71, 40, 6, 512),    # 65 S tokens: the last block holds one token, no multiple of 8
