@@ -1171,7 +1171,7 @@ static BlockLayout block_layout(const pdm_block_desc& d) {
   L.k = off; off = align256(off + B * d.kv_len * D * 2);                // K
   L.vt = off; off = align256(off + B * (D / 64) * 64 * (int64_t)L.vt_ld * 2);  // V^T per head
   if (!fused) {
-    L.h = off; off = align256(off + B * d.kv_len * D * 2);                // h1, later h2
+    L.h = off; off = align256(off + B * d.kv_len * D * 2);                // RMSNorm2 rows
     L.g = off; off = align256(off + B * d.q_len * (int64_t)d.ffn_dim * 2);  // GELU(FFN-up)
   }
   L.total = off;
