@@ -368,7 +368,9 @@ typedef struct {
   const void* ns_w2;      /* bf16 [NS, D, F] */
 } pdm_block_weights;
 
-/* Bytes of device workspace pdm_onetrans_block_fwd needs for desc. */
+/* Bytes of device workspace pdm_onetrans_block_fwd needs for desc.  It never
+ * falls as batch, kv_len or q_len grows with the rest unchanged: a workspace
+ * sized for the largest batch is enough for every smaller one. */
 int64_t pdm_onetrans_block_workspace_size(const pdm_block_desc* desc);
 
 /* x: device fp32 [B, kv_len, D] (the residual stream); y: device fp32
@@ -393,7 +395,8 @@ int pdm_onetrans_block_fwd(const pdm_block_desc* desc, const float* x,
  * ------------------------------------------------------------------------ */
 #define PDM_STACK_MAX_LAYERS 64
 
-/* Bytes of device workspace pdm_onetrans_stack_fwd needs. */
+/* Bytes of device workspace pdm_onetrans_stack_fwd needs; like the block's, it
+ * never falls as batch, kv_len or an entry of q_s grows. */
 int64_t pdm_onetrans_stack_workspace_size(const pdm_block_desc* desc,
                                           const int32_t* q_s, int32_t n_layers);
 

@@ -1149,11 +1149,17 @@ static int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 // tiles of 128 rows walk the whole hidden dimension one after another: 50 us at d_model 256 however few rows there are,
 // 53 us for 17,408 rows, 81 us for 34,816.  Below, and at d_model 384 / 512 (whose rows do not fit its registers), three
 // kernels split that work over the chip: 30 us for 4,352 rows, 57 us for 17,408, 112 us for 34,816.  (At d_model 128 the
-// one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three also need the normalised rows
-// (h) and the GELU activations (g) in the workspace.
+// one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three keep RMSNorm2's rows (h) and
+// the GELU activations (g) in the workspace.
 constexpr int64_t kFusedMinRows = 14000;
 static bool fused_path(const pdm_block_desc& d) {
   return d.d_model == 128 || (d.d_model == 256 && (int64_t)d.batch * d.q_len > kFusedMinRows);
+}
+// Kept rows for which the workspace holds h and g.  At d_model 256 that is the largest batch the three kernels take,
+// also when this one is larger, so that a workspace sized for one batch is enough for every smaller one.
+static int64_t split_rows(const pdm_block_desc& d) {
+  const int64_t rows = (int64_t)d.batch * d.q_len;
+  return d.d_model == 128 ? 0 : (d.d_model == 256 ? std::min(rows, kFusedMinRows) : rows);
 }
 // d_model 256: rows of x from which the weight-stationary Q/K/V projection (384 KB of weight into every CU's registers
 // first: 34 us however few rows) is faster than the streaming one.  Per block: 6,400 rows 34 against 14 us, 51,200 rows
@@ -1163,17 +1169,15 @@ constexpr int64_t kQkvStationaryMinRows = 120000;
 static BlockLayout block_layout(const pdm_block_desc& d) {
   BlockLayout L;
   const int64_t B = d.batch, D = d.d_model;
-  const bool fused = fused_path(d);
   L.kv_pad = (d.kv_len + 31) & ~31;
   L.vt_ld = (d.kv_len + 63) & ~63;
   int64_t off = 0;
   L.q = off; off = align256(off + B * d.q_len * D * 2);                 // Q, later attention output
   L.k = off; off = align256(off + B * d.kv_len * D * 2);                // K
   L.vt = off; off = align256(off + B * (D / 64) * 64 * (int64_t)L.vt_ld * 2);  // V^T per head
-  if (!fused) {
-    L.h = off; off = align256(off + B * d.kv_len * D * 2);                // RMSNorm2 rows
-    L.g = off; off = align256(off + B * d.q_len * (int64_t)d.ffn_dim * 2);  // GELU(FFN-up)
-  }
+  const int64_t rows = split_rows(d);
+  L.h = off; off = align256(off + rows * D * 2);                        // RMSNorm2 rows
+  L.g = off; off = align256(off + rows * (int64_t)d.ffn_dim * 2);       // GELU(FFN-up)
   L.total = off;
   return L;
 }

@@ -134,6 +134,36 @@ def test_stack_workspace_size(pdm):
     assert L.lib().pdm_onetrans_stack_workspace_size(ctypes.byref(d), None, 2) == L.PDM_ERR_INVALID
 
 
+def test_block_and_stack_workspace_never_shrink(pdm):
+    """A workspace sized for the largest batch must be enough for every smaller one, also where a smaller batch
+    runs other kernels (d_model 256: 14,000 kept rows), and the Python layout agrees on both sides of that line."""
+    L = pdm._lib
+    lib = L.lib()
+
+    def block(B, kv, q, D, Fd, ns=16):
+        return lib.pdm_onetrans_block_workspace_size(ctypes.byref(L.BlockDesc(B, D, D // 64, ns, Fd, kv, q, 0)))
+
+    def stack(B, kv, D, Fd, q_s, ns=16):
+        arr = (ctypes.c_int32 * len(q_s))(*q_s)
+        return lib.pdm_onetrans_stack_workspace_size(ctypes.byref(L.BlockDesc(B, D, D // 64, ns, Fd, kv, 0, 0)), arr,
+                                                     len(q_s))
+
+    for D in (128, 256, 384):
+        for mult in (2, 4, 16):
+            batches = [*range(1, 12), 40, 51, 52, 64, 174, 175, 176, 370, 371, 1024]
+            for kv, q in ((272, 272), (144, 80), (400, 38)):
+                sizes = [block(B, kv, q, D, mult * D) for B in batches]
+                assert sizes == sorted(sizes) and sizes[0] > 0
+                for B, n in zip(batches, sizes):
+                    assert n == pdm.ops.onetrans_workspace_layout(B, kv, q, D, mult * D)["total"][0]
+            sizes = [block(50, 400, q, D, mult * D) for q in range(16, 401, 8)]  # 14,000 kept rows at q = 280
+            assert sizes == sorted(sizes)
+            sizes = [stack(B, 400, D, mult * D, [384, 256, 128, 64]) for B in batches]
+            assert sizes == sorted(sizes) and sizes[0] > 0
+            sizes = [stack(100, 400, D, mult * D, [384, q, 64]) for q in range(64, 385, 16)]
+            assert sizes == sorted(sizes)
+
+
 def test_kjt_row_count_overflow_is_rejected(pdm):
     """num_features * batch_size (and num_out * batch_size) must be checked before the product is formed: a
     huge batch_size would otherwise wrap the int64 row count and pass the limits."""
