@@ -49,7 +49,7 @@ struct RowProjArgs {
   uint16_t* vt;
   int kv, q_len, kv_pad;
   // filled by the launcher
-  int blocks_per_sample, tiles_per_token, wgs_s, wgs_ns, split_s, split_ns;
+  int blocks_per_sample, wgs_s, wgs_ns, split_s, split_ns;
 };
 int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s);
 

@@ -134,7 +134,11 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
   const int l16 = lane & 15, piece = 2 * ((lane >> 4) & 1) + hf;  // tile_segments
 
   // workgroup -> (row tile, column split): the NS tiles first, then the S tiles, each group dealt so that neighbours
-  // share an XCD (workgroups go to the 8 XCDs in turn): a token's tiles share its weight, a tile's splits its rows.
+  // share an XCD (workgroups go to the 8 XCDs in turn).  The NS tiles run sample by sample, all tokens of 128 samples
+  // behind each other, so that the 2-byte V^T stores of neighbouring tokens meet in one L2 line (token by token, each
+  // line went out from as many XCDs as it has NS tokens; 4,096 samples of 16 S and 16 NS tokens, whole block: d 128
+  // 229 -> 162 us, d 384 1,295 -> 1,109; 8 NS tokens alone, d 128: 121 -> 88); every XCD then reads every token's
+  // weight, which costs less.  A tile's splits share its rows.
   // (With both groups in one such order the NS tiles, the slowest, all fell to the last XCD.)
   const int n_ns_wgs = a.wgs_ns * a.split_ns;
   const bool is_s = (int)blockIdx.x >= n_ns_wgs;
@@ -152,8 +156,9 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
     rows = b0 < a.B ? min(32, a.n_s - t0) : 0;
     if (b0 >= a.B) b0 = t0 = 0;
   } else {
-    g = tile / a.tiles_per_token;
-    b0 = ((tile - g * a.tiles_per_token) * 4 + wave) * 32;
+    const int st = tile / a.n_ns;
+    g = tile - st * a.n_ns;
+    b0 = (st * 4 + wave) * 32;
     t0 = a.n_s + g;
     rows = max(0, min(32, a.B - b0));
     if (rows == 0) b0 = 0;
@@ -397,8 +402,7 @@ static int launch_one(RowProjArgs a, hipStream_t s) {
   PDM_CHECK_HIP(err[dev]);
   a.blocks_per_sample = (a.n_s + 31) / 32;
   const int64_t wgs_s = ((int64_t)a.B * a.blocks_per_sample + 3) / 4;
-  a.tiles_per_token = (a.B + 127) / 128;
-  const int64_t wgs_ns = (int64_t)a.n_ns * a.tiles_per_token;
+  const int64_t wgs_ns = (int64_t)a.n_ns * ((a.B + 127) / 128);
   // column splits: as many as keep the grid within one workgroup per CU, of at least two chunks each for the S tiles; a
   // second workgroup per CU only where the first round leaves no room for a split.  Every split reads and normalises its
   // tile's rows again, and at two per CU that took 5.0 us of a launch's 12 (one per CU 3.8; d 256, FFN-up of 16 samples

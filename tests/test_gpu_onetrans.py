@@ -137,6 +137,7 @@ def test_block_attention_workgroups_per_head(pdm, dev, B, kv, q_len, n_ns, D):
     (2, 30, 30, 0, 384),    # no NS tokens
     (3, 16, 16, 16, 384),   # no S tokens
     (140, 37, 24, 3, 384),  # NS tokens over two row tiles of 128 samples, the second partial
+    (513, 21, 21, 5, 384),  # NS tokens over five row tiles of 128 samples, the last of one sample
     (300, 61, 45, 3, 384),  # 13,500 kept rows: 128 x 128 tiles of the residual projections, the last one partial
     (330, 61, 43, 5, 256),  # 14,190 kept rows: just above the fused FFN's limit
     (325, 61, 43, 5, 256),  # 13,975 kept rows: just below it
