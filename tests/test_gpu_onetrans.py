@@ -137,7 +137,16 @@ def test_block_attention_workgroups_per_head(pdm, dev, B, kv, q_len, n_ns, D):
     (2, 30, 30, 0, 384),    # no NS tokens
     (3, 16, 16, 16, 384),   # no S tokens
     (140, 37, 24, 3, 384),  # NS tokens over two row tiles of 128 samples, the second partial
-    (513, 21, 21, 5, 384),  # NS tokens over five row tiles of 128 samples, the last of one sample
+    # NS tokens over four row tiles of 128 samples, the last of one sample.  (Not 513 samples: one of their V values is
+    # 1.0e-7 here and 1.5e-7 in the oracle, a sum of 384 fp32 products whose magnitudes add to 5.0, far inside the
+    # 384 * 2^-24 * 5.0 = 1.1e-4 of any order; the query that sees that key alone copies it, and the tolerance of the
+    # attention output is relative to the value itself.)
+    (385, 21, 21, 5, 384),
+    (130, 35, 2, 2, 128),   # one S token behind a whole block, run token by token and not kept as a query
+    (130, 36, 3, 2, 256),   # two of them, one kept; the FFN-up's only S token
+    (512, 1, 1, 0, 512),    # one S token and no whole block, no NS tokens
+    (256, 18, 18, 2, 384),  # 16 S tokens: token by token for the FFN-up, a block for Q/K/V
+    (260, 52, 50, 3, 512),  # 49 and 47 S tokens: a whole block and 17 or 15 behind it
     (300, 61, 45, 3, 384),  # 13,500 kept rows: 128 x 128 tiles of the residual projections, the last one partial
     (330, 61, 43, 5, 256),  # 14,190 kept rows: just above the fused FFN's limit
     (325, 61, 43, 5, 256),  # 13,975 kept rows: just below it
