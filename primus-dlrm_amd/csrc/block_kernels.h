@@ -48,8 +48,8 @@ struct RowProjArgs {
   uint16_t* k;
   uint16_t* vt;
   int kv, q_len, kv_pad;
-  // filled by the launcher
-  int blocks_per_sample, wgs_s, wgs_ns, split_s, split_ns;
+  // filled by the launcher: tokens t < n_blk run in 32-token blocks of a sample, the n_tok behind them token by token
+  int n_blk, n_tok, tiles_b, blocks_per_sample, wgs_s, wgs_tok, split_s, split_tok;
 };
 int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s);
 

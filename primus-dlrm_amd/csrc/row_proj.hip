@@ -8,10 +8,10 @@
 // previous one (rounding, GELU, stores) are issued between the MFMAs of the current chunk; two workgroups share a CU
 // with independent barriers, so one's row loads run beside the other's MFMAs.
 //
-// A wave's rows are 32 consecutive tokens of ONE sample (the shared S weight) or one NS token of 32 samples (that
-// token's weight): addresses are a wave-uniform base plus row * stride, and a feature row of V^T receives runs of 8
-// tokens at multiples of 8.  Padding rows (the last block of a sample, samples past the batch) read the block's last
-// row again and store nothing.
+// A wave's rows are 32 consecutive tokens of ONE sample (S tokens, the shared weight) or one token of 32 samples (an NS
+// token with its weight, or a last S token of every sample where few are left behind its whole blocks): addresses are a
+// wave-uniform base plus row * stride, and a feature row of V^T receives runs of 8 tokens at multiples of 8.  Padding
+// rows (the last block of a sample, samples past the batch) read the block's last row again and store nothing.
 //
 // What bounds it, at OneTransL's second layer (d 384, B = 1024, 1,552,384 rows in, 1,335,296 kept): the fp32 rows in and
 // the bf16 outputs out (5.8 GB for Q/K/V, about 1.2 ms at a device copy's rate; 1.37 TFLOP, 0.55 ms of MFMA), behind
@@ -133,38 +133,46 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
   const int fr = lane & 31, hf = lane >> 5;
   const int l16 = lane & 15, piece = 2 * ((lane >> 4) & 1) + hf;  // tile_segments
 
-  // workgroup -> (row tile, column split): the NS tiles first, then the S tiles, each group dealt so that neighbours
-  // share an XCD (workgroups go to the 8 XCDs in turn).  The NS tiles run sample by sample, all tokens of 128 samples
+  // workgroup -> (row tile, column split): the token tiles first, then the S blocks, each group dealt so that neighbours
+  // share an XCD (workgroups go to the 8 XCDs in turn).  The token tiles run sample by sample, all tokens of 128 samples
   // behind each other, so that the 2-byte V^T stores of neighbouring tokens meet in one L2 line (token by token, each
   // line went out from as many XCDs as it has NS tokens; 4,096 samples of 16 S and 16 NS tokens, whole block: d 128
   // 229 -> 162 us, d 384 1,295 -> 1,109; 8 NS tokens alone, d 128: 121 -> 88); every XCD then reads every token's
-  // weight, which costs less.  A tile's splits share its rows.
-  // (With both groups in one such order the NS tiles, the slowest, all fell to the last XCD.)
-  const int n_ns_wgs = a.wgs_ns * a.split_ns;
-  const bool is_s = (int)blockIdx.x >= n_ns_wgs;
-  int rest = is_s ? (int)blockIdx.x - n_ns_wgs : (int)blockIdx.x;
-  const int full = (is_s ? a.wgs_s * a.split_s : n_ns_wgs) & ~7;
+  // weight, which costs less.  With less than four tiles of samples, whose last may be nearly empty, they run token by
+  // token, or the XCDs with the last tile would idle (130 samples of 17 S and 16 NS tokens, d 384: 85 against 81 us).
+  // A tile's splits share its rows.
+  // (With both groups in one such order the token tiles, the slowest, all fell to the last XCD.)
+  const int n_tok_wgs = a.wgs_tok * a.split_tok;
+  const bool is_s = (int)blockIdx.x >= n_tok_wgs;
+  int rest = is_s ? (int)blockIdx.x - n_tok_wgs : (int)blockIdx.x;
+  const int full = (is_s ? a.wgs_s * a.split_s : n_tok_wgs) & ~7;
   if (rest < full) rest = (rest & 7) * (full >> 3) + (rest >> 3);
-  const int split = is_s ? a.split_s : a.split_ns;
+  const int split = is_s ? a.split_s : a.split_tok;
   const int tile = rest / split, part = rest - tile * split;
   // the wave's rows: row i is (sample b0, token t0 + i) or (sample b0 + i, token t0)
-  int b0, t0, rows, g = 0;
+  int b0, t0, rows;
   if (is_s) {
     const int64_t blk = (int64_t)tile * 4 + wave;
     b0 = (int)(blk / a.blocks_per_sample);
     t0 = (int)(blk - (int64_t)b0 * a.blocks_per_sample) * 32;
-    rows = b0 < a.B ? min(32, a.n_s - t0) : 0;
+    rows = b0 < a.B ? min(32, a.n_blk - t0) : 0;
     if (b0 >= a.B) b0 = t0 = 0;
   } else {
-    const int st = tile / a.n_ns;
-    g = tile - st * a.n_ns;
+    int st, g;
+    if (a.tiles_b >= 4) {
+      st = tile / a.n_tok;
+      g = tile - st * a.n_tok;
+    } else {
+      g = tile / a.tiles_b;
+      st = tile - g * a.tiles_b;
+    }
     b0 = (st * 4 + wave) * 32;
-    t0 = a.n_s + g;
+    t0 = a.n_blk + g;
     rows = max(0, min(32, a.B - b0));
     if (rows == 0) b0 = 0;
   }
   const int last = max(rows - 1, 0);
-  const uint16_t* W = is_s ? a.W : a.W_ns + (int64_t)g * a.N * D;
+  const uint16_t* W = t0 < a.n_s ? a.W : a.W_ns + (int64_t)(t0 - a.n_s) * a.N * D;
 
   const int nchunks = a.N / 32;
   const int c_begin = (int)((int64_t)nchunks * part / split), c_end = (int)((int64_t)nchunks * (part + 1) / split);
@@ -246,7 +254,7 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
 
   // Q is needed of the kept tail tokens only: rows below q_first of this wave have none
   const int q_first = a.kv - a.q_len - t0;
-  const bool skip_q = EPI == ROWPROJ_QKV && (is_s ? q_first >= rows : rows == 0);
+  const bool skip_q = EPI == ROWPROJ_QKV && (is_s ? q_first >= rows : rows == 0 || q_first > 0);
 
   // the previous chunk's tile, stored during the current one: line r (line_lo <= r < line_hi) at obase + r * ostride
   // elements, of which the first `outs` outputs exist
@@ -400,31 +408,40 @@ static int launch_one(RowProjArgs a, hipStream_t s) {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   });
   PDM_CHECK_HIP(err[dev]);
-  a.blocks_per_sample = (a.n_s + 31) / 32;
-  const int64_t wgs_s = ((int64_t)a.B * a.blocks_per_sample + 3) / 4;
-  const int64_t wgs_ns = (int64_t)a.n_ns * ((a.B + 127) / 128);
+  // The S tokens behind a sample's last whole block: a block of their own, mostly padding when they are few, or tiles of
+  // one token of 128 samples, like the NS tokens, without padding but with 2-byte V^T stores.  Tiles where they are few
+  // enough workgroups: up to 16 tokens of many samples for the FFN-up, 4 for Q/K/V.  Whole blocks of 4,096 samples in
+  // us, blocks / tiles for the FFN-up / tiles for both: d 512, 1 S token 769 / 561 / 464, 4 829 / 648 / 542, 8 925 / 788
+  // / 768, 16 1,764 / 1,659 / 1,674, 28 1,453 / 1,430 / 1,504; Q/K/V alone at d 128: 1 87 / 77, 4 92 / 88, 8 94 / 104.
+  const int tail = a.n_s % 32, whole = a.n_s - tail;
+  a.tiles_b = (a.B + 127) / 128;
+  auto blocks = [&](int n) { return ((int64_t)a.B * ((n + 31) / 32) + 3) / 4; };
+  a.n_blk = (int64_t)tail * a.tiles_b * (EPI == ROWPROJ_QKV ? 8 : 2) <= blocks(a.n_s) - blocks(whole) ? whole : a.n_s;
+  a.blocks_per_sample = (a.n_blk + 31) / 32;
+  a.n_tok = a.n_s - a.n_blk + a.n_ns;
+  const int64_t wgs_s = blocks(a.n_blk), wgs_tok = (int64_t)a.n_tok * a.tiles_b;
   // column splits: as many as keep the grid within one workgroup per CU, of at least two chunks each for the S tiles; a
   // second workgroup per CU only where the first round leaves no room for a split.  Every split reads and normalises its
   // tile's rows again, and at two per CU that took 5.0 us of a launch's 12 (one per CU 3.8; d 256, FFN-up of 16 samples
   // of 272 tokens).  One round against two, stacks in us: d 256 B = 16 198 / 202, B = 4 167 / 170, d 384 B = 8 810 / 830,
   // d 512 B = 4 305 / 321; without a split against two: d 256 B = 48 312 / 303, d 128 B = 100 194 / 183.
-  // What is left of the round goes to the NS tiles, down to single chunks: their weight is read from memory by few
+  // What is left of the round goes to the token tiles, down to single chunks: their weight is read from memory by few
   // workgroups, and their V^T goes out in 2-byte stores (500 samples of 98 tokens, d 384: Q/K/V 111 -> 81 us with the NS
   // tiles split).
   const int nchunks = a.N / 32;
   constexpr int64_t kCus = 256;
-  const int64_t tiles = std::max<int64_t>(1, wgs_s + wgs_ns);
+  const int64_t tiles = std::max<int64_t>(1, wgs_s + wgs_tok);
   const int64_t round = 2 * tiles <= kCus ? kCus : 2 * kCus;
   a.split_s = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks / 2, round / tiles));
-  a.split_ns = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks, (round - wgs_s * a.split_s) / std::max<int64_t>(1, wgs_ns)));
-  const int64_t grid = wgs_s * a.split_s + wgs_ns * a.split_ns;
+  a.split_tok = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks, (round - wgs_s * a.split_s) / std::max<int64_t>(1, wgs_tok)));
+  const int64_t grid = wgs_s * a.split_s + wgs_tok * a.split_tok;
   if (grid == 0) return PDM_OK;
   PDM_CHECK_ARG(grid < (int64_t(1) << 31), "row projection grid too large");
   // 32 lines of any output lie within 2^31 bytes of the wave's first
   PDM_CHECK_ARG((int64_t)32 * std::max<int64_t>({a.out_bstride, (int64_t)a.kv * D, (int64_t)a.kv_pad}) * 2 < (int64_t(1) << 31),
                 "row projection rows too far apart");
   a.wgs_s = (int)wgs_s;
-  a.wgs_ns = (int)wgs_ns;
+  a.wgs_tok = (int)wgs_tok;
   hipLaunchKernelGGL((rowproj_kernel<D, EPI>), dim3((unsigned)grid), dim3(256), lds, s, a);
   PDM_CHECK_LAUNCH();
   return PDM_OK;
