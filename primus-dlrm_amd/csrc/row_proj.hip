@@ -279,16 +279,22 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
     store16(obase, r >= line_lo && r < line_hi && piece * 8 + 8 <= outs ? off : kNoStore,
             u32x4_t{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
   };
-  // a sample's last V^T tokens when they are no multiple of 8: not the NS tokens behind them
+  // a sample's last V^T tokens when they are no multiple of 8: not the NS tokens behind them.  Four of them in one store
+  // (blocks of 4,096 samples of 60 S and 4 NS tokens, d 128: 295 -> 288 us; any number of them in that way took more
+  // registers and 303)
   auto epi_tail = [&]() {
     if (EPI == ROWPROJ_QKV && (outs & 7)) {
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         if (piece == outs >> 3 && 16 * i + l16 < line_hi) {
           uint16_t* v = obase + (int64_t)(16 * i + l16) * ostride + piece * 8;
+          if ((outs & 7) == 4) {
+            *reinterpret_cast<u32x2_t*>(v) = u32x2_t{pk[i][0], pk[i][1]};
+          } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            if (piece * 8 + e < outs) v[e] = (uint16_t)(pk[i][e >> 1] >> (16 * (e & 1)));
+            for (int e = 0; e < 8; ++e)
+              if (piece * 8 + e < outs) v[e] = (uint16_t)(pk[i][e >> 1] >> (16 * (e & 1)));
+          }
         }
     }
   };
