@@ -1151,16 +1151,16 @@ static int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 // kernels split that work over the chip: 30 us for 4,352 rows, 57 us for 17,408, 112 us for 34,816.  (At d_model 128 the
 // one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three keep RMSNorm2's rows (h) and
 // the GELU activations (g) in the workspace.
+// The residual GEMM reaches the rows of g within 2^32 bytes, so d_model 256 takes the three only where all of g lies in them.
 constexpr int64_t kFusedMinRows = 14000;
-static bool fused_path(const pdm_block_desc& d) {
-  return d.d_model == 128 || (d.d_model == 256 && (int64_t)d.batch * d.q_len > kFusedMinRows);
+static int64_t split_max_rows(const pdm_block_desc& d) {  // kept rows up to which the three kernels run
+  if (d.d_model == 128) return 0;
+  return d.d_model == 256 ? std::min(kFusedMinRows, ((int64_t(1) << 31) - 1) / d.ffn_dim) : INT64_MAX;
 }
+static bool fused_path(const pdm_block_desc& d) { return (int64_t)d.batch * d.q_len > split_max_rows(d); }
 // Kept rows for which the workspace holds h and g.  At d_model 256 that is the largest batch the three kernels take,
 // also when this one is larger, so that a workspace sized for one batch is enough for every smaller one.
-static int64_t split_rows(const pdm_block_desc& d) {
-  const int64_t rows = (int64_t)d.batch * d.q_len;
-  return d.d_model == 128 ? 0 : (d.d_model == 256 ? std::min(rows, kFusedMinRows) : rows);
-}
+static int64_t split_rows(const pdm_block_desc& d) { return std::min((int64_t)d.batch * d.q_len, split_max_rows(d)); }
 // d_model 256: rows of x from which the weight-stationary Q/K/V projection (384 KB of weight into every CU's registers
 // first: 34 us however few rows) is faster than the streaming one.  Per block: 6,400 rows 34 against 14 us, 51,200 rows
 // 62 against 49 us, 102,400 rows 277 against 274 us (whole block), 204,800 rows 448 against 461 us (whole block).

@@ -173,7 +173,8 @@ static int launch_tiles(ResidArgs a, hipStream_t s) {
   if (grid == 0) return PDM_OK;
   PDM_CHECK_ARG(grid < (int64_t(1) << 31), "GEMM grid too large");
   // a tile's rows lie within 2^32 bytes of its first sample, and its weight rows of its first
-  PDM_CHECK_ARG((TM + 1) * a.a_bstride * 2 < (int64_t(1) << 32), "GEMM rows too far apart");
+  const int64_t samples = std::min<int64_t>(a.B, std::max(a.n_s ? (TM - 2) / a.n_s + 2 : 1, a.n_ns ? TM : 1));
+  PDM_CHECK_ARG(samples * a.a_bstride * 2 < (int64_t(1) << 32), "GEMM rows too far apart");
   PDM_CHECK_ARG((int64_t)TN * a.K * 2 < (int64_t(1) << 32), "GEMM weight too large");
   a.tiles_s = (int)tiles_s;
   hipLaunchKernelGGL((resid_gemm_kernel<TM, TN, WM, BK, NST>), dim3((unsigned)grid), dim3(256), 0, s, a);

@@ -443,9 +443,8 @@ static int launch_one(RowProjArgs a, hipStream_t s) {
   const int64_t grid = wgs_s * a.split_s + wgs_tok * a.split_tok;
   if (grid == 0) return PDM_OK;
   PDM_CHECK_ARG(grid < (int64_t(1) << 31), "row projection grid too large");
-  // 32 lines of any output lie within 2^31 bytes of the wave's first
-  PDM_CHECK_ARG((int64_t)32 * std::max<int64_t>({a.out_bstride, (int64_t)a.kv * D, (int64_t)a.kv_pad}) * 2 < (int64_t(1) << 31),
-                "row projection rows too far apart");
+  // the 32 features of a V^T tile lie within 2^31 bytes of the first
+  PDM_CHECK_ARG((int64_t)32 * a.kv_pad * 2 < (int64_t(1) << 31), "row projection rows too far apart");
   a.wgs_s = (int)wgs_s;
   a.wgs_tok = (int)wgs_tok;
   hipLaunchKernelGGL((rowproj_kernel<D, EPI>), dim3((unsigned)grid), dim3(256), lds, s, a);
@@ -465,7 +464,29 @@ static int launch_epi(const RowProjArgs& a, int D, hipStream_t s) {
 }
 
 int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s) {
-  return epi == ROWPROJ_QKV ? launch_epi<ROWPROJ_QKV>(a, D, s) : launch_epi<ROWPROJ_GELU>(a, D, s);
+  auto launch = [&](const RowProjArgs& r) {
+    return epi == ROWPROJ_QKV ? launch_epi<ROWPROJ_QKV>(r, D, s) : launch_epi<ROWPROJ_GELU>(r, D, s);
+  };
+  // a wave's lines, the same token of up to 32 samples, lie within 2^31 bytes of its first: samples that are further
+  // apart go out as many at a time as do
+  const int64_t apart = 2 * (epi == ROWPROJ_QKV ? (int64_t)a.kv * D : a.out_bstride);
+  const int64_t fit = std::max<int64_t>(1, ((int64_t(1) << 31) - 1) / apart);
+  if (fit >= std::min(a.B, 32)) return launch(a);
+  for (int64_t b = 0; b < a.B; b += fit) {
+    RowProjArgs r = a;
+    r.B = (int)std::min<int64_t>(fit, a.B - b);
+    r.x += b * a.in_bstride;
+    if (epi == ROWPROJ_QKV) {
+      r.q += b * a.q_len * D;
+      r.k += b * a.kv * D;
+      r.vt += b * D * a.kv_pad;
+    } else {
+      r.h += b * a.in_bstride;
+      r.out += b * a.out_bstride;
+    }
+    if (int st = launch(r)) return st;
+  }
+  return PDM_OK;
 }
 
 }  // namespace pdm

@@ -649,18 +649,19 @@ def onetrans_workspace_layout(B: int, kv: int, q_len: int, D: int, F: int) -> Di
     pdm_onetrans_block_fwd: q (Q tail rows [B, q_len, D] bf16, later the
     attention output), k ([B, kv, D] bf16), vt (V transposed per head [B, D/64,
     64, kv_ld] bf16, kv_ld = kv rounded up to 64).  d_model 384 and 512, and 256 with
-    at most 14,000 kept rows, run the FFN as separate kernels and also hold h (RMSNorm2
-    rows [B, q_len, D] bf16) and g (GELU of the FFN-up GEMM [B, q_len, F] bf16); d_model
-    256 with more rows leaves room for 14,000 (``reserve``), so that the workspace of a
-    batch is enough for every smaller one."""
+    at most 14,000 kept rows (and less than 2^31 elements of g), run the FFN as separate
+    kernels and also hold h (RMSNorm2 rows [B, q_len, D] bf16) and g (GELU of the FFN-up
+    GEMM [B, q_len, F] bf16); d_model 256 with more rows leaves room for that many
+    (``reserve``), so that the workspace of a batch is enough for every smaller one."""
     a = lambda v: (v + 255) // 256 * 256  # noqa: E731
     kv_ld = (kv + 63) // 64 * 64
     sizes = [("q", B * q_len * D * 2), ("k", B * kv * D * 2), ("vt", B * D * kv_ld * 2)]
     rows = B * q_len
-    if D > 256 or (D == 256 and rows <= 14000):
+    most = min(14000, (2 ** 31 - 1) // F)
+    if D > 256 or (D == 256 and rows <= most):
         sizes += [("h", rows * D * 2), ("g", rows * F * 2)]
     elif D == 256:
-        sizes += [("reserve", a(14000 * D * 2) + 14000 * F * 2)]
+        sizes += [("reserve", a(most * D * 2) + most * F * 2)]
     out, off = {}, 0
     for name, n in sizes:
         out[name] = (off, n)

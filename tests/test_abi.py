@@ -149,7 +149,7 @@ def test_block_and_stack_workspace_never_shrink(pdm):
                                                      len(q_s))
 
     for D in (128, 256, 384):
-        for mult in (2, 4, 16):
+        for mult in (2, 4, 16, 1024):
             batches = [*range(1, 12), 40, 51, 52, 64, 174, 175, 176, 370, 371, 1024]
             for kv, q in ((272, 272), (144, 80), (400, 38)):
                 sizes = [block(B, kv, q, D, mult * D) for B in batches]

@@ -168,6 +168,30 @@ def test_block_row_projection_tokens_of_many_samples(pdm, dev, B, kv, q_len, n_n
     _run_case(pdm, dev, B, kv, q_len, n_ns, D=D, F=2 * D, seed=B + kv, norm_std=0.1, v_sums=True)
 
 
+def test_block_wide_ffn(pdm, dev):
+    """d_model 256 with an FFN of 65,536: one sample's hidden activations are 68 MB, so 32 samples' would lie more than
+    2^31 bytes apart."""
+    _run_case(pdm, dev, 2, 520, 520, 2, D=256, F=65536, seed=21, w_std=0.01)
+
+
+def test_block_samples_far_apart(pdm, dev):
+    """33 samples of 262,150 tokens at d_model 128: the same token of 32 samples lies more than 2^31 bytes apart in K,
+    and K of all samples fills 2.2 GB.  The first, the 32nd and the last sample are compared with the oracle."""
+    B, kv, q_len, n_ns, D, F = 33, 262150, 20, 3, 128, 128
+    w = ot.random_weights(D, F, n_ns, std=0.02, seed=22, norm_std=0.1)
+    x = torch.empty(B, kv, D, device=dev)
+    for b in range(B):
+        x[b] = torch.randn(kv, D, generator=torch.Generator(device=dev).manual_seed(b), device=dev)
+    print(f"block B={B} kv={kv} q_len={q_len} D={D}", flush=True)
+    got = pdm.ops.onetrans_block_raw(x, _gpu_weights(w, dev), D // 64, q_len).cpu()
+    for b in (0, 31, 32):
+        xs = x[b:b + 1].cpu()
+        want, parts = ot.block_forward(xs, w, q_len, D // 64, mode="autocast", return_parts=True)
+        terms = ot.term_magnitudes(xs, w, q_len, D // 64, parts)
+        tail = xs[:, kv - q_len:]
+        _close(f"sample {b} update", got[b:b + 1] - tail, want - tail, terms["y"])
+
+
 def test_block_baseline_shape_reduced_batch(pdm, dev):
     """The 4-layer benchmark's first layer (400 tokens, 16 NS, d 256, FFN 1024) at batch 8."""
     _run_case(pdm, dev, 8, 400, 400, 16, seed=11)
