@@ -24,6 +24,7 @@ struct NsArgs {
   const uint16_t* w1;  // [N, K]
   uint16_t* w1p;       // [N, K64]
   int32_t N;
+  int64_t w1p_elems;  // 0: W1 is read where it is
   int32_t* err;
 };
 
@@ -33,9 +34,10 @@ struct NsArgs {
 // own another 5; together 5 us).  The blocks after them: W1 [N, K] -> [N, K64] with zero columns K .. K64, 4 columns a
 // thread.
 __global__ __launch_bounds__(256) void ns_prep_kernel(NsArgs a) {
-  if ((int64_t)blockIdx.x >= a.B) {
-    const int64_t i = (((int64_t)blockIdx.x - a.B) * 256 + threadIdx.x) * 4;
-    if (i >= (int64_t)a.N * a.K64) return;
+  const int64_t block = linear_block();
+  if (block >= a.B) {
+    const int64_t i = ((block - a.B) * 256 + threadIdx.x) * 4;
+    if (i >= a.w1p_elems) return;
     const int n = (int)(i / a.K64), k = (int)(i - (int64_t)n * a.K64);
     const uint16_t* src = a.w1 + (int64_t)n * a.K;
     uint32_t v[4];
@@ -46,14 +48,13 @@ __global__ __launch_bounds__(256) void ns_prep_kernel(NsArgs a) {
     *reinterpret_cast<u32x2_t*>(a.w1p + i) = u32x2_t{v[0] | v[1] << 16, v[2] | v[3] << 16};
     return;
   }
-  const int64_t b = blockIdx.x;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint16_t* dst = a.raw + b * a.K64;
+  uint16_t* dst = a.raw + block * a.K64;
   bool bad = false;
   for (int j = wave; j < a.n_parts; j += 4) {
     const int c0 = a.col[j], w = a.col[j + 1] - c0;
     if (j < a.n_scalar) {
-      const int64_t id = a.ids[j][b];
+      const int64_t id = a.ids[j][block];
       const bool ok = id >= 0 && id < a.rows[j];
       bad |= !ok;
       if (!ok) {
@@ -67,7 +68,7 @@ __global__ __launch_bounds__(256) void ns_prep_kernel(NsArgs a) {
       }
     } else {
       const int d = j - a.n_scalar;
-      const float* row = a.dense[d] + b * a.dense_stride[d];
+      const float* row = a.dense[d] + block * a.dense_stride[d];
       for (int c = lane; c < w; c += 64) dst[c0 + c] = (uint16_t)f32_to_bf16_bits(row[c]);
     }
   }
@@ -417,9 +418,8 @@ extern "C" int pdm_ns_tokenize_fwd(const pdm_ns_desc* desc, const void* const* t
   a.w1 = w1;
   a.w1p = w1p;
   a.N = N;
-  const int64_t pad_blocks = pad ? ((int64_t)N * K64 / 4 + 255) / 256 : 0;
-  PDM_CHECK_ARG(d.batch_size + pad_blocks < (int64_t(1) << 31), "grid too large");
-  hipLaunchKernelGGL(ns_prep_kernel, dim3((unsigned)(d.batch_size + pad_blocks)), dim3(256), 0, s, a);
+  a.w1p_elems = pad ? (int64_t)N * K64 : 0;
+  hipLaunchKernelGGL(ns_prep_kernel, linear_grid(d.batch_size + (a.w1p_elems / 4 + 255) / 256), dim3(256), 0, s, a);
   PDM_CHECK_LAUNCH();
   NsGemmArgs g{};
   g.M = (int)d.batch_size;

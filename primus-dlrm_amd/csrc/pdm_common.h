@@ -53,6 +53,15 @@ struct SideFork {
 int side_fork(hipStream_t caller, SideFork& f);       // PDM_OK or PDM_ERR_HIP (f.side may be null)
 int side_join(hipStream_t caller, const SideFork& f);  // no-op when f.side is null
 
+// ---- launches of many blocks -------------------------------------------------
+// A dimension of a launch holds less than 2^32 threads: a list of blocks (of at most 256 threads) that may be longer than
+// 2^24 goes on in y.  The last row of blocks is not full, so kernels check linear_block against their work.
+inline dim3 linear_grid(int64_t blocks) {
+  const int64_t x = blocks < (int64_t(1) << 23) ? blocks : int64_t(1) << 23;
+  return dim3((unsigned)x, (unsigned)((blocks + x - 1) / x));
+}
+__device__ __forceinline__ int64_t linear_block() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+
 inline int dtype_size(int dt) {
   switch (dt) {
     case PDM_F32: return 4;

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(256) void seq_gather_kernel(SeqArgs a) {
   const int lane = threadIdx.x & 63;
   const int lpb = 1 << a.lpb_shift;
   const int j = lane & (lpb - 1);
-  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int64_t wave = linear_block() * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int64_t tok0 = ((wave << (6 - a.lpb_shift)) + (lane >> a.lpb_shift)) * TPG;
   if (tok0 >= a.num_tokens) return;  // all lanes of a group share tok0
   bool bad = false;
@@ -312,7 +312,7 @@ extern "C" int pdm_seq_gather_fwd(const pdm_seq_desc* desc, const void* const* t
   const int64_t tok_per_block = 4 * (64 / lpb) * tokens_per_group(nch);
   const int64_t blocks = (a.num_tokens + tok_per_block - 1) / tok_per_block;
   PDM_CHECK_ARG(blocks < (int64_t(1) << 31), "too many tokens for one launch");
-  hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a);
+  hipLaunchKernelGGL(fn, linear_grid(blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a);
   PDM_CHECK_LAUNCH();
   return PDM_OK;
 }

@@ -368,6 +368,23 @@ def test_seq_gather_lane_group_edges(pdm, dev, dims):
     assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
 
 
+def test_seq_gather_more_tokens_than_one_grid_dimension(pdm, dev):
+    """134,218,752 tokens of 257 4-byte pieces (8 per workgroup, 138 GB): one workgroup per 8 tokens is more threads
+    than a dimension of a launch holds.  Slices at the start, the middle and the end are compared."""
+    B, S, dim = 131073, 1024, 257
+    tab = torch.arange(50 * dim, dtype=torch.float32, device=dev).view(50, dim)
+    offs = torch.arange(B + 1, dtype=torch.int64, device=dev) * 3
+    ids = (torch.arange(3 * B, device=dev) * 7) % 50
+    print(f"gather of {B * S} tokens", flush=True)
+    out, mask = pdm.ops.seq_gather_raw([tab], [[ids]], [offs], [S], 0, 0)
+    for b in (0, 1, B // 2 - 1, B // 2, B - 2, B - 1):
+        want = tab[torch.cat([ids.new_zeros(S - 3), ids[3 * b:3 * b + 3]])]
+        assert torch.equal(out[b], want)
+        assert torch.equal(mask[b].cpu(), (torch.arange(S) >= S - 3).to(torch.uint8))
+    del out, mask
+    torch.cuda.empty_cache()
+
+
 def test_seq_gather_bad_ids_zeroed_and_flagged(pdm, dev):
     g = np.random.default_rng(23)
     tabs_t, ids, offs = _seq_case(g, 5, (6, 6), [4, 4], (8, 8), (40, 40), "bf16")

@@ -94,6 +94,19 @@ def test_ns_tokenize_tile_edges(pdm, dev, B, dense_dims, d, n_ns):
     _check(out.cpu(), tabs, ids, dense, w, n_ns)
 
 
+def test_ns_tokenize_more_samples_than_one_grid_dimension(pdm, dev):
+    """2^24 + 5 samples: one block each is more threads than a dimension of a launch holds.  The first and last samples
+    and those around each multiple of 2^23 are compared."""
+    B, d = (1 << 24) + 5, 64
+    w = ot.random_autosplit_weights(4, d, seed=4)
+    wb = {k: v.to(torch.bfloat16).contiguous().to(dev) for k, v in w.items()}
+    x = torch.randn(B, 4, generator=torch.Generator(device=dev).manual_seed(4), device=dev)
+    print(f"NS tokens of {B} samples", flush=True)
+    out = pdm.ops.ns_tokenize_raw([], [], [x], wb["w1"], wb["b1"], wb["w2"], wb["b2"], 1)
+    pick = torch.tensor([*range(40), *range((1 << 23) - 40, (1 << 23) + 40), *range((1 << 24) - 40, B)])
+    _check(out[pick.to(dev)].cpu(), [], [], [x[pick.to(dev)].cpu().numpy()], w, 1)
+
+
 def test_ns_tokens_into_block_input_and_bad_ids(pdm, dev):
     """out = the NS rows of a [B, S + n_ns, d] block input (S rows untouched); an id outside its table reads
     zeros and raises the flag."""
