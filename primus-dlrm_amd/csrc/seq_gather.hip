@@ -16,12 +16,13 @@
 // before the next phase, so the three dependent memory round trips are paid
 // once per TPG tokens.
 //
-// A lane has NCH * TPG pieces in flight, six to eight of them: TPG 8 for rows of one piece per lane, 4 of two, 2 of
-// more, and rows past 64 pieces take more lanes instead of more pieces per lane (eight pieces of eight tokens held 256
-// registers and ran one wave per SIMD).  Bound by the output's bytes, 393,216 tokens (126 us for fp32 rows of 384 at a
-// device copy's rate): fp32 256 + 64 + 64 over 16 lanes x 8 pieces x 8 tokens 260 us, 32 x 3 x 8 151, 32 x 3 x 4 138,
-// 32 x 3 x 2 131; fp32 128 + 64 (16 x 3) 8 tokens 74.9, 2 tokens 70.1; fp32 128 (16 x 2) 8 tokens 52.5, 4 tokens 48.0,
-// 2 tokens 49.7; bf16 128 (16 x 1) 8 tokens 25.5, 4 tokens 26.4, 2 tokens 29.4.
+// A lane has NCH * TPG pieces in flight, mostly six to eight of them: TPG 8 for rows of one piece per lane, 4 of two, 2 of
+// more (16 pieces for rows past 256), and rows past 64 pieces take more lanes instead of more pieces per lane (eight
+// pieces of eight tokens held 256 registers and ran one wave per SIMD).  seq_shape has the exceptions.  Bound by the
+// output's bytes, 393,216 tokens (126 us for fp32 rows of 384 at a device copy's rate): fp32 256 + 64 + 64 over 16 lanes
+// x 8 pieces x 8 tokens 260 us, 32 x 3 x 8 151, 32 x 3 x 4 138, 32 x 3 x 2 131; fp32 128 + 64 (16 x 3) 8 tokens 74.9, 2
+// tokens 70.1; fp32 128 (16 x 2) 8 tokens 52.5, 4 tokens 48.0, 2 tokens 49.7; bf16 128 (16 x 1) 8 tokens 25.5, 4 tokens
+// 26.4, 2 tokens 29.4.
 #include <algorithm>
 
 #include "pdm_common.h"
@@ -222,15 +223,50 @@ using namespace pdm;
 
 namespace {
 using SeqFn = void (*)(SeqArgs);
-constexpr int tokens_per_group(int nch) { return nch == 1 ? 8 : (nch == 2 ? 4 : 2); }
+// Lanes per token and tokens per lane group (TPG).  Times in us for 393,216 tokens of tables of 20,000 / 2,000,000 rows,
+// lanes x pieces per lane x tokens.
+struct SeqShape {
+  int lanes, tokens;
+};
+SeqShape seq_shape(int vb, int pieces, int64_t num_tokens, int64_t table_bytes) {
+  constexpr int64_t kSome = 1 << 13, kMany = 1 << 16, kMost = 1 << 18, kInfinityCache = int64_t(1) << 28;
+  int lanes = 1;
+  while (lanes < pieces && lanes < 64 && (lanes < 16 || lanes * 4 < pieces)) lanes <<= 1;
+  const int per_lane = (pieces + lanes - 1) / lanes;
+  if (vb == 4) {
+    // 4-byte pieces: a quarter of the bytes in flight, and what bounds a token are the instructions of its group, so
+    // that more tokens per group pay: 17 pieces 16x2x4 34 / 37, 32x1x8 23 / 27; 64 pieces 16x4x2 53 / 57, 32x2x8 45 / 47;
+    // 129 pieces 64x3x2 154 / 159, 64x3x4 130 / 135; 40 pieces 16x3x2 45 / 50, 16x3x8 41 / 49.  Only where every CU has
+    // several groups, though: 400 tokens of 17 pieces 7.0 and 8.8, of 129 pieces 5.0 and 7.9, 49,152 of 64 pieces 9.2
+    // and 10.7, 196,608 of 40 pieces 23 / 27 and 26 / 31.
+    if (pieces >= 32 && pieces <= 48 && num_tokens >= kMost) return {16, 8};
+    if (pieces > 16 && pieces <= 32 && num_tokens >= kSome) return {32, 8};
+    if (pieces > 48 && pieces <= 64 && num_tokens >= kMany) return {32, 8};
+    if (pieces > 128 && pieces <= 256 && num_tokens >= kSome) return {64, 4};
+  } else if (table_bytes > kInfinityCache) {
+    // rows from memory instead of the caches have a longer way: 64 pieces 16x4x2 88 / 131, 32x2x8 97 / 114; 256 pieces
+    // 64x4x2 345 / 475, 64x4x8 370 / 449 (98,304 tokens 93 / 123 and 97 / 110); 48 pieces, 768,000 tokens 16x3x2 220,
+    // 16x3x8 176 (from memory; 262,144 tokens 48 and 53)
+    if (pieces >= 40 && pieces <= 48 && num_tokens >= 2 * kMost) return {16, 8};
+    if (pieces > 48 && pieces <= 64 && num_tokens >= kMost / 2 * 3) return {32, 8};
+    if (pieces == 256 && num_tokens >= kMany) return {64, 8};
+  }
+  return {lanes, per_lane == 1 ? 8 : (per_lane == 2 ? 4 : 2)};
+}
+
 template <int VB>
-SeqFn pick_seq(int nch) {
-  switch (nch) {
-    case 1: return seq_gather_kernel<VB, 1, tokens_per_group(1)>;
-    case 2: return seq_gather_kernel<VB, 2, tokens_per_group(2)>;
-    case 3: return seq_gather_kernel<VB, 3, tokens_per_group(3)>;
-    case 4: return seq_gather_kernel<VB, 4, tokens_per_group(4)>;
-    case 8: return seq_gather_kernel<VB, 8, tokens_per_group(8)>;
+SeqFn pick_seq(int nch, int tpg) {
+  switch (nch * 10 + tpg) {
+    case 18: return seq_gather_kernel<VB, 1, 8>;
+    case 24: return seq_gather_kernel<VB, 2, 4>;
+    case 28: return seq_gather_kernel<VB, 2, 8>;
+    case 32: return seq_gather_kernel<VB, 3, 2>;
+    case 38: return seq_gather_kernel<VB, 3, 8>;
+    case 42: return seq_gather_kernel<VB, 4, 2>;
+    case 82: return seq_gather_kernel<VB, 8, 2>;
+    case 34: if constexpr (VB == 4) return seq_gather_kernel<VB, 3, 4>; else return nullptr;
+    case 44: if constexpr (VB == 4) return seq_gather_kernel<VB, 4, 4>; else return nullptr;
+    case 48: if constexpr (VB == 16) return seq_gather_kernel<VB, 4, 8>; else return nullptr;
     default: return nullptr;
   }
 }
@@ -297,11 +333,13 @@ extern "C" int pdm_seq_gather_fwd(const pdm_seq_desc* desc, const void* const* t
   a.align_left = d.align == PDM_ALIGN_LEFT;
   const int vb = vec16 ? 16 : 4;
   a.chunks = a.tok_bytes / vb;
-  int lpb = 1;
-  while (lpb < a.chunks && lpb < 64 && (lpb < 16 || lpb * 4 < a.chunks)) lpb <<= 1;
+  int64_t table_bytes = 0;
+  for (int f = 0; f < a.F; ++f) table_bytes += a.rows[f] * a.feat_bytes[f];
+  const SeqShape shape = seq_shape(vb, a.chunks, a.num_tokens, table_bytes);
+  const int lpb = shape.lanes;
   int nch = (a.chunks + lpb - 1) / lpb;
   if (nch > 4 && nch <= 8) nch = 8;
-  SeqFn fn = vb == 16 ? pick_seq<16>(nch) : pick_seq<4>(nch);
+  SeqFn fn = vb == 16 ? pick_seq<16>(nch, shape.tokens) : pick_seq<4>(nch, shape.tokens);
   if (!fn) {
     set_error("pdm_seq_gather_fwd: token row of " + std::to_string(a.tok_bytes) + " bytes is too wide");
     return PDM_ERR_UNSUPPORTED;
@@ -309,7 +347,7 @@ extern "C" int pdm_seq_gather_fwd(const pdm_seq_desc* desc, const void* const* t
   int sh = 0;
   while ((1 << sh) < lpb) ++sh;
   a.lpb_shift = sh;
-  const int64_t tok_per_block = 4 * (64 / lpb) * tokens_per_group(nch);
+  const int64_t tok_per_block = 4 * (64 / lpb) * shape.tokens;
   const int64_t blocks = (a.num_tokens + tok_per_block - 1) / tok_per_block;
   PDM_CHECK_ARG(blocks < (int64_t(1) << 31), "too many tokens for one launch");
   hipLaunchKernelGGL(fn, linear_grid(blocks), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a);

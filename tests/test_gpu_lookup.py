@@ -368,6 +368,25 @@ def test_seq_gather_lane_group_edges(pdm, dev, dims):
     assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
 
 
+@pytest.mark.parametrize("dims,B,rows", [
+    ((17,), 300, 50), ((31, 1), 300, 50), ((31, 1), 9, 50),   # 17, 32 pieces of 4 bytes: one per lane of 32
+    ((31, 1), 2100, 50), ((47, 1), 2100, 50), ((33,), 9, 50),  # 32, 48: 16 lanes, eight tokens each in large calls
+    ((49,), 600, 50), ((63, 1), 600, 50),                     # 49, 64: 32 lanes
+    ((129,), 300, 50), ((255, 1), 300, 50),                   # 129, 256: 64 lanes, four tokens each
+    ((196,), 3100, 400_000), ((256,), 3100, 300_000),         # 49, 64 pieces of 16 bytes of tables past 256 MB
+    ((160,), 4100, 450_000), ((1024,), 600, 70_000),          # 40, 256 of them
+])
+def test_seq_gather_group_shapes_by_size(pdm, dev, dims, B, rows):
+    """The lane groups that depend on the number of tokens and the size of the tables, with a token count that no
+    group divides (bytes are copied: bit exact)."""
+    g = np.random.default_rng(sum(dims) + B)
+    tabs_t, ids, offs = _seq_case(g, B, (60, 40), [66, 63], dims, (rows,) * len(dims), "fp32")
+    print(f"gather dims={dims} B={B} rows={rows}", flush=True)
+    got, mask, want, wmask, err, _ = _seq_run(pdm, dev, tabs_t, ids, offs, [66, 63], 0, 0)
+    assert np.array_equal(mask, wmask) and err == 0
+    assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+
+
 def test_seq_gather_more_tokens_than_one_grid_dimension(pdm, dev):
     """134,218,752 tokens of 257 4-byte pieces (8 per workgroup, 138 GB): one workgroup per 8 tokens is more threads
     than a dimension of a launch holds.  Slices at the start, the middle and the end are compared."""
