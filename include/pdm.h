@@ -353,8 +353,13 @@ typedef struct {
   int32_t ffn_dim;  /* FFN hidden (multiple of 128) */
   int32_t kv_len;   /* tokens in x */
   int32_t q_len;    /* tokens kept (tail of x), n_ns <= q_len <= kv_len */
-  int32_t reserved;
+  int32_t flags;    /* 0, or PDM_BLOCK_KEEP_NORM2 */
 } pdm_block_desc;
+
+/* Leave RMSNorm2's rows (bf16 [B, q_len, D]) in the workspace, between V^T and
+ * the GELU activations, where the FFN runs as separate kernels.  Nothing reads
+ * them: for checks of the intermediate results. */
+#define PDM_BLOCK_KEEP_NORM2 1
 
 typedef struct {
   const float* norm1_w;   /* fp32 [D] */

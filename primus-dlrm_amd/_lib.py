@@ -32,6 +32,7 @@ PDM_WD_NONE, PDM_WD_L2 = 0, 1
 PDM_KJT_MAX_FEATURES = 64
 PDM_KJT_NOALLOC_MAX_ROWS = 67108864
 PDM_STACK_MAX_LAYERS = 64
+PDM_BLOCK_KEEP_NORM2 = 1
 
 # Every symbol include/pdm.h declares (checked by the ABI test).
 EXPORTED_SYMBOLS = (
@@ -155,7 +156,7 @@ class BlockDesc(ctypes.Structure):
         ("ffn_dim", ctypes.c_int32),
         ("kv_len", ctypes.c_int32),
         ("q_len", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("flags", ctypes.c_int32),
     ]
 
 

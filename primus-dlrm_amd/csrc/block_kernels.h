@@ -39,7 +39,7 @@ struct RowProjArgs {
   const uint16_t* W_ns;  // [n_ns, N, D], or null when n_ns == 0
   int B, n_s, n_ns, N;
   // ROWPROJ_GELU: out row (b, t) at out + b * out_bstride + t * N; the normalised bf16 rows are also left in h (the
-  // layout of x)
+  // layout of x) unless it is null
   uint16_t* h;
   uint16_t* out;
   int64_t out_bstride;

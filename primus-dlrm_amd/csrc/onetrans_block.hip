@@ -1149,8 +1149,8 @@ static int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 // tiles of 128 rows walk the whole hidden dimension one after another: 50 us at d_model 256 however few rows there are,
 // 53 us for 17,408 rows, 81 us for 34,816.  Below, and at d_model 384 / 512 (whose rows do not fit its registers), three
 // kernels split that work over the chip: 30 us for 4,352 rows, 57 us for 17,408, 112 us for 34,816.  (At d_model 128 the
-// one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three keep RMSNorm2's rows (h) and
-// the GELU activations (g) in the workspace.
+// one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three keep the GELU activations (g)
+// in the workspace, and RMSNorm2's rows (h) for a caller that asks for them.
 // The residual GEMM reaches the rows of g within 2^32 bytes, so d_model 256 takes the three only where all of g lies in them.
 constexpr int64_t kFusedMinRows = 14000;
 static int64_t split_max_rows(const pdm_block_desc& d) {  // kept rows up to which the three kernels run
@@ -1412,14 +1412,14 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     g1.res = x; g1.res_bstride = (int64_t)kv * D; g1.res_toff = kv - ql;
     if ((st = launch_resid_gemm(g1, s)) != PDM_OK) return st;
   }
-  // 4. h = RMSNorm2(z)  [B, q_len, D], g = bf16(gelu(bf16(h2 . W1^T)))  [B, q_len, F]
+  // 4. g = bf16(gelu(bf16(RMSNorm2(z) . W1^T)))  [B, q_len, F]; RMSNorm2(z) itself only on request, nothing here reads it
   {
     RowProjArgs r2{};
     r2.x = y; r2.norm_w = w->norm2_w; r2.in_bstride = (int64_t)ql * D;
     r2.W = reinterpret_cast<const uint16_t*>(w->s_w1);
     r2.W_ns = reinterpret_cast<const uint16_t*>(w->ns_w1);
     r2.B = B; r2.n_s = ql - nns; r2.n_ns = nns; r2.N = F;
-    r2.h = h; r2.out = g; r2.out_bstride = (int64_t)ql * F;
+    r2.h = (d.flags & PDM_BLOCK_KEEP_NORM2) ? h : nullptr; r2.out = g; r2.out_bstride = (int64_t)ql * F;
     if ((st = launch_row_proj(r2, D, ROWPROJ_GELU, s)) != PDM_OK) return st;
   }
   // 5. y = z + bf16(g . W2^T)

@@ -203,7 +203,8 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
     static_assert(4 * SL * STR <= NST * CHUNK, "the row scratch lies in the weight ring");
     char* sc = lds + wave * SL * STR;
     const float* x0 = a.x + (int64_t)b0 * a.in_bstride + (int64_t)t0 * D;
-    uint16_t* h0 = a.h + (int64_t)b0 * a.in_bstride + (int64_t)t0 * D;
+    const bool keep_h = EPI == ROWPROJ_GELU && part == 0 && a.h != nullptr;
+    uint16_t* h0 = keep_h ? a.h + (int64_t)b0 * a.in_bstride + (int64_t)t0 * D : nullptr;
     const int sub = lane & 15, rq = lane >> 4;
     f32x4_t w[NV];
 #pragma unroll
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256, 2) void rowproj_kernel(RowProjArgs a) {
         for (int j = 0; j < NV; ++j) {
           const u32x2_t n = u32x2_t{pack_bf16x2((u[j].x * rms) * w[j].x, (u[j].y * rms) * w[j].y),
                                     pack_bf16x2((u[j].z * rms) * w[j].z, (u[j].w * rms) * w[j].w)};
-          if (EPI == ROWPROJ_GELU && part == 0 && r < rows) *reinterpret_cast<u32x2_t*>(hr + j * 64) = n;
+          if (keep_h && r < rows) *reinterpret_cast<u32x2_t*>(hr + j * 64) = n;
           *reinterpret_cast<u32x2_t*>(sc + (p * 4 + rq) * STR + j * 128 + sub * 8) = n;
         }
       }
@@ -481,7 +482,7 @@ int launch_row_proj(const RowProjArgs& a, int D, int epi, hipStream_t s) {
       r.k += b * a.kv * D;
       r.vt += b * D * a.kv_pad;
     } else {
-      r.h += b * a.in_bstride;
+      if (r.h) r.h += b * a.in_bstride;
       r.out += b * a.out_bstride;
     }
     if (int st = launch(r)) return st;

@@ -676,7 +676,8 @@ def onetrans_block_raw(x: torch.Tensor, w: Dict[str, torch.Tensor], n_heads: int
     """x: fp32 [B, kv, D]; w: norm1_w/norm2_w fp32 [D], the GEMM weights bf16
     in nn.Linear layout.  Returns fp32 [B, q_len, D].  ``workspace`` (uint8,
     at least pdm_onetrans_block_workspace_size bytes) is allocated when not
-    given."""
+    given; a caller's own holds every region of ``onetrans_workspace_layout``
+    after the call."""
     names = ("norm1_w", "s_qkv_w", "ns_qkv_w", "out_w", "norm2_w", "s_w1", "s_w2", "ns_w1", "ns_w2")
     dev = _require_cuda(x, *[w[k] for k in names])
     if x.dtype != torch.float32 or x.dim() != 3 or not x.is_contiguous():
@@ -693,7 +694,7 @@ def onetrans_block_raw(x: torch.Tensor, w: Dict[str, torch.Tensor], n_heads: int
             raise ValueError(f"{k}: expected contiguous {want} {shapes[k]}, got {t.dtype} {tuple(t.shape)}")
     if not (n_ns <= q_len <= kv):
         raise ValueError(f"need n_ns <= q_len <= kv_len, got n_ns={n_ns} q_len={q_len} kv_len={kv}")
-    desc = L.BlockDesc(B, D, n_heads, n_ns, Fd, kv, q_len, 0)
+    desc = L.BlockDesc(B, D, n_heads, n_ns, Fd, kv, q_len, 0 if workspace is None else L.PDM_BLOCK_KEEP_NORM2)
     ws_bytes = int(L.lib().pdm_onetrans_block_workspace_size(ctypes.byref(desc)))
     if ws_bytes < 0:
         raise L.PdmError(ws_bytes, "pdm_onetrans_block_workspace_size", L.last_error())

@@ -168,6 +168,35 @@ def test_block_row_projection_tokens_of_many_samples(pdm, dev, B, kv, q_len, n_n
     _run_case(pdm, dev, B, kv, q_len, n_ns, D=D, F=2 * D, seed=B + kv, norm_std=0.1, v_sums=True)
 
 
+@pytest.mark.parametrize("D", [256, 384])
+def test_block_stores_norm2_rows_only_on_request(pdm, dev, D):
+    """Nothing in the library reads RMSNorm2's rows: a call without PDM_BLOCK_KEEP_NORM2 leaves their region of the
+    workspace as it was, and the result is the same bit for bit."""
+    import ctypes
+
+    B, kv, q_len, n_ns, F = 6, 45, 40, 3, 2 * D
+    L = pdm._lib
+    w = _gpu_weights(ot.random_weights(D, F, n_ns, std=0.02, seed=23, norm_std=0.1), dev)
+    x = torch.randn(B, kv, D, generator=torch.Generator().manual_seed(23)).to(dev)
+    layout = pdm.ops.onetrans_workspace_layout(B, kv, q_len, D, F)
+    names = ("norm1_w", "s_qkv_w", "ns_qkv_w", "out_w", "norm2_w", "s_w1", "s_w2", "ns_w1", "ns_w2")
+    outs, kept = [], []
+    for flags in (0, L.PDM_BLOCK_KEEP_NORM2):
+        ws = torch.full((layout["total"][0],), 0xAB, dtype=torch.uint8, device=dev)
+        out = torch.empty(B, q_len, D, device=dev)
+        desc = L.BlockDesc(B, D, D // 64, n_ns, F, kv, q_len, flags)
+        status = L.lib().pdm_onetrans_block_fwd(ctypes.byref(desc), x.data_ptr(),
+                                                ctypes.byref(L.BlockWeights(*[w[k].data_ptr() for k in names])),
+                                                out.data_ptr(), ws.data_ptr(), ws.numel(), L.stream_ptr(dev))
+        L.check(status, "pdm_onetrans_block_fwd")
+        torch.cuda.synchronize()
+        outs.append(out)
+        off, size = layout["h"]
+        kept.append(bool((ws[off:off + size] == 0xAB).all()))
+    assert kept == [True, False]
+    assert torch.equal(outs[0], outs[1])
+
+
 def test_block_wide_ffn(pdm, dev):
     """d_model 256 with an FFN of 65,536: one sample's hidden activations are 68 MB, so 32 samples' would lie more than
     2^31 bytes apart."""
