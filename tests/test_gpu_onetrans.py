@@ -53,9 +53,11 @@ def _ws_view(ws, layout, name, shape, dtype=torch.bfloat16):
 
 def _check_layer(pdm, dev, x, w, q_len, label="", v_sums=False):
     """Runs one block on the GPU and checks its intermediates and output against the oracle on the same x.  With
-    v_sums the attention output is also allowed what its V may differ by, at most D * 2^-24 * |h| . |W| (fp32 sums of
-    D products in another order): a query that sees one key copies that key's V, whatever cancelled in it, and among
-    many samples some V is far smaller than its terms (1.0e-7 against 1.5e-7 out of terms of 5.0)."""
+    v_sums the attention output is also allowed what its V may differ by: D * 2^-24 * |h| . |W| (fp32 sums of D
+    products in another order) and two columns of h on the other side of a bf16 rounding (the row's fp32 norm differs in
+    its last bit: one column in about 60,000).  A query that sees one key copies that key's V, whatever cancelled in it,
+    and among many samples some V is far smaller than its terms (1.0e-7 against 1.5e-7 out of terms of 5.0; 3e-5 against
+    3e-4 with one column of h rounded the other way)."""
     B, kv, D = x.shape
     H = D // 64
     F = w["s_w1"].shape[0]
@@ -75,8 +77,10 @@ def _check_layer(pdm, dev, x, w, q_len, label="", v_sums=False):
     _close("k", k, parts["k"], terms["k"])
     _close("v", v, parts["v"], terms["v"])
     o_terms = terms["o"].double().reshape(B, q_len, D)
-    if v_sums:  # the largest over the keys a query sees; the scale is multiplied by ELEM_TOL in _close
-        o_terms = o_terms + (terms["v"].double().reshape(B, kv, D) * (D * 2.0 ** -24 / ELEM_TOL)).cummax(1)[0][:, kv - q_len:]
+    if v_sums:  # the scale is multiplied by ELEM_TOL in _close
+        w_max = max(w["s_qkv"].abs().max().item(), w["ns_qkv"].abs().max().item() if w["ns_qkv"].numel() else 0.0)
+        h_max = (x * x.square().mean(-1, keepdim=True).rsqrt() * w["norm1"]).abs().max().item()
+        o_terms = o_terms + (terms["v"].max().item() * D * 2.0 ** -24 + 2 * 2.0 ** -8 * h_max * w_max) / ELEM_TOL
     _close("attention out", o, parts["o"], o_terms)
     if "g" in layout:  # the tiled path keeps RMSNorm2 rows and GELU activations in the workspace
         g = _ws_view(ws, layout, "g", (B, q_len, F))
@@ -227,16 +231,14 @@ def test_block_baseline_shape_reduced_batch(pdm, dev):
 
 
 def test_block_batch1024_short_sequence(pdm, dev):
-    """Batch 1024 (the benchmark's batch: 48 k rows, hundreds of GEMM row tiles and 4096 attention
-    (sample, head) pairs over the persistent grids) at a short sequence of 48 tokens keeping 32."""
+    """Batch 1024 (the benchmark's batch: 48 k rows of the streaming Q/K/V projection, hundreds of fused-FFN row tiles
+    and 4096 attention (sample, head) pairs over the persistent grids) at a short sequence of 48 tokens keeping 32."""
     _run_case(pdm, dev, 1024, 48, 32, 16, seed=12, norm_std=0.1)
 
 
 def test_block_vt_paired_tiles(pdm, dev):
-    """Batch 160 with 128 S tokens: 640 S tiles over the Q/K/V projection's 256 workgroups, shares of 2 or 3
-    consecutive tiles, so some workgroups write two tiles' V^T as whole lines together and others write a
-    tile alone (a share starting at token 64 pairs it with token 96; a share's last tile at token 0 goes
-    alone)."""
+    """Batch 160 with 128 S tokens: four 32-token blocks per sample, of which the streaming Q/K/V projection writes the
+    32 tokens of every V^T row, and a tail of which half a block is kept."""
     _run_case(pdm, dev, 160, 144, 32, 16, seed=14, norm_std=0.1)
 
 
@@ -247,11 +249,54 @@ def test_block_ffn_ns_last_round(pdm, dev):
 
 
 def test_block_ns_tiles_cross_tokens(pdm, dev):
-    """Batch 1100 with 16 NS tokens: 35 row tiles of 32 samples per NS token (the last partial), 560 NS
-    tiles over the Q/K/V projection's persistent grid, so workgroups' shares start and end inside a token's
-    tiles and cross from one NS token's weight to the next; 33 S tokens (one full and one single-row tile per
-    sample) with the kept tail starting inside the first tile."""
+    """Batch 1100 with 16 NS tokens on the streaming Q/K/V projection: nine tiles of 128 samples per NS token (the last
+    partial); 33 S tokens (one whole block and one token run by itself) with the kept tail starting inside the block."""
     _run_case(pdm, dev, 1100, 49, 20, 16, seed=13, norm_std=0.1)
+
+
+@pytest.mark.parametrize("B,kv,q_len,n_ns", [
+    # 128 S tokens, 3,600 S tiles of 32 over 256 workgroups: shares of 14 or 15 consecutive tiles, so some write two
+    # tiles' V^T as whole lines together and others a tile alone (a share starting at token 64 pairs it with token 96, a
+    # share's last tile at token 0 goes alone)
+    (900, 144, 32, 16),
+    # 16 NS tokens: 82 tiles of 32 samples each (the last of 8), shares that cross from one NS token's weight to the
+    # next; 33 S tokens (a whole and a single-row tile per sample), the kept tail starting inside the whole one
+    (2600, 49, 20, 16),
+    (2599, 48, 48, 16),   # 32 S tokens: unpaired tiles only; every token kept; the last NS tile of 7 samples
+    (1277, 95, 17, 0),    # no NS tokens; two whole tiles and one of 31 rows; a tail inside the last tile
+    (3001, 41, 3, 3),     # kept tail of the NS tokens alone
+    (120, 1001, 520, 5),  # 32 tiles per sample, an odd number of keys, streaming attention
+    (2450, 49, 20, 16),   # 120,050 rows: just above the line between the two projections
+    (2448, 49, 20, 16),   # 119,952 rows: just below it
+])
+def test_block_stationary_projection(pdm, dev, B, kv, q_len, n_ns):
+    """d_model 256 with more than 120,000 rows: the weight-stationary Q/K/V projection at ragged sizes, every sample
+    compared."""
+    assert (B * kv > 120_000) == ((B, kv) != (2448, 49))
+    _run_case(pdm, dev, B, kv, q_len, n_ns, D=256, F=256, seed=B, norm_std=0.1, v_sums=True)
+
+
+@pytest.mark.parametrize("B,kv,q_len,n_ns,D,F", [
+    (1010, 100, 100, 2, 512, 512),  # 526 and 528 row tiles x 4 column tiles
+    (1301, 110, 104, 5, 384, 384),  # 705 and 706 x 3
+])
+def test_block_residual_192_row_tiles(pdm, dev, B, kv, q_len, n_ns, D, F):
+    """Enough rows for the 192 x 128 tiles of the residual projections (2,048 of them), the last S tile and every NS
+    token's last tile partial.  The first and last samples and those at the edges of the NS tiles are compared."""
+    tiles = lambda n_s, n_ns_: (-(-B * n_s // 192) + n_ns_ * -(-B // 192)) * D // 128  # noqa: E731
+    assert tiles(q_len, 0) >= 2048 and tiles(q_len - n_ns, n_ns) >= 2048
+    assert B * q_len % 192 and B * (q_len - n_ns) % 192 and B % 192
+    print(f"block B={B} kv={kv} q_len={q_len} D={D} n_ns={n_ns}, sampled", flush=True)
+    w = ot.random_weights(D, F, n_ns, std=0.02, seed=B, norm_std=0.1)
+    x = torch.randn(B, kv, D, generator=torch.Generator().manual_seed(B + 1))
+    got = pdm.ops.onetrans_block_raw(x.to(dev), _gpu_weights(w, dev), D // 64, q_len).cpu()
+    edge = B // 192 * 192
+    pick = torch.tensor([0, 1, 2, 95, 190, 191, 192, 193, 383, 384, edge - 1, edge, edge + 1, B - 3, B - 2, B - 1])
+    xs = x[pick]
+    want, parts = ot.block_forward(xs, w, q_len, D // 64, mode="autocast", return_parts=True)
+    terms = ot.term_magnitudes(xs, w, q_len, D // 64, parts)
+    tail = xs[:, kv - q_len:]
+    _close("block update y - x_tail", got[pick] - tail, want - tail, terms["y"])
 
 
 @pytest.mark.parametrize("B,kv,q_len,D", [
