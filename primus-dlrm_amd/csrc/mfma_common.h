@@ -91,13 +91,6 @@ __device__ __forceinline__ void gelu_table_fill(float* t, int tid, int nthreads)
     t[i] = gelu_tail(__builtin_bit_cast(float, (GELU_T_LO + (uint32_t)i) << 16));
 }
 
-__device__ __forceinline__ float gelu_lut(const float* t, float x) {  // x: a bf16 value held as fp32
-  const float ax = fabsf(x);
-  const float c = __builtin_amdgcn_fmed3f(ax, 0x1p-16f, 8.0f);
-  const float e = t[(__builtin_bit_cast(uint32_t, c) >> 16) - GELU_T_LO];
-  return __builtin_fmaf(-ax, e, fmaxf(x, 0.0f));
-}
-
 // G[i] = bf16(GELU(bf16(u[2i]))) | bf16(GELU(bf16(u[2i+1]))) << 16 for N values: all N table reads are
 // issued before the first is used, so the LDS latency is paid once.
 template <int N>

@@ -50,10 +50,9 @@ struct GemmArgs {
   // epilogue
   void* out;            // fp32 [B, T, D]
   int64_t out_bstride;  // elements between samples of out
-  const float* res;     // residual fp32, row (b, t) at res + b * res_bstride + (t + res_toff) * N
+  const float* res;     // residual fp32, row (b, t) at res + b * res_bstride + (t + res_toff) * K
   int64_t res_bstride;
   int res_toff;
-  int D;
   // the fused FFN
   const float* norm_w;    // RMSNorm2 weight
   const uint16_t* W2;     // FFN-down [D, F] shared
@@ -112,61 +111,39 @@ __device__ __forceinline__ int ns_tile_xcd_major(const GemmArgs& a, int mt) {
 }
 
 // ---------------------------------------------------------------------------
-// Fused FFN:  y = z + W2 . gelu(W1 . RMSNorm2(z))  for K = d_model = D, hidden F.
+// Out-projection and FFN in one kernel:  z = bf16(O . Wout^T) + x,  y = z + W2 . gelu(W1 . RMSNorm2(z))  for
+// K = d_model = D, hidden F.
 //
-// Each of the NW waves owns RB x 32 rows; with RB = 1 and 8 waves, two waves
-// share a SIMD and one's GELU (VALU) overlaps the other's MFMAs, which the
-// hardware does not do within a wave.  RMSNorm2(z) rows stay in registers
-// (same layout as rowgemm's A fragments) and so do the D fp32 outputs of the
-// wave's rows.  The hidden dimension is walked in chunks of 32 units:
-// U^T = W1_c . h^T puts hidden units on the accumulator rows and token rows
-// on the columns, so lane l holds token row l%32 of each row block and 16
-// hidden units of it.  After GELU (fp32 on the bf16-rounded value, then bf16)
-// those values are the B operand of y^T += W2[:, c] . G^T without leaving
-// registers.  Every weight fragment read from LDS feeds RB MFMAs.  With
-// PDM_FFN_UP16 (the default) the FFN-up runs as 16x16x32 MFMAs into four
-// independent accumulators (two 16-unit hidden blocks x two 16-token blocks):
-// one exchange of the RMSNorm2 fragments per tile and one of the GELU values
-// per chunk (v_permlane16_swap) keep both sides' operand reads single 16-byte
-// LDS reads, and LDS row r of the W1 chunk holds hidden unit r.  Otherwise the
-// accumulator row e/4*8 + (l/32)*4 + e%4 of a 16-unit half must meet hidden
-// unit (l/32)*8 + e%8 for the W2 operand to be one contiguous 16-byte read,
-// so LDS row r of the W1 chunk holds hidden unit r with bits 2 and 3 swapped.
-// W1 and W2 chunks go global -> LDS by LDS DMA into an NST-stage ring, chunk
-// c + NST - 1 issued right after the barrier that publishes chunk c.  Without
-// OPROJ the epilogue adds z (fp32, read from the residual rows) to the
-// bf16-rounded FFN output.
+// Each of the NW waves owns 32 rows.  The out-projection runs in front: z^T = Wout . O^T accumulates straight into
+// the y registers (lane l holds row l%32), every O fragment of the lane's row is requested up front and the Wout
+// chunks (D rows x 64 columns, exactly one ring stage) go through the weight ring in front of the FFN chunks.  z is
+// added to the residual x and normalised in registers; the RMSNorm2 values reach the B-operand layout of the FFN-up
+// with one exchange of two words per 16-column step between the half-waves.  The FFN-down then accumulates on top of
+// z, so y = z + FFN leaves the registers once and z never goes to memory.  The one difference from the reference's
+// autocast rounding points: the FFN-down output is added to z in fp32 instead of being rounded to bf16 first, a
+// difference of at most half a bf16 ulp of the FFN output.
 //
-// OPROJ: the out-projection runs in front, z = bf16(O . Wout^T) + x, so z is
-// produced on chip.  z^T = Wout . O^T accumulates straight into the y
-// registers (the same layout: lane l holds row l%32), every O fragment of the
-// lane's row is requested up front and the Wout chunks (D rows x 64 columns,
-// exactly one ring stage) go through the same ring in front of the FFN chunks.
-// z is added to the residual x and normalised in registers; the RMSNorm2
-// values reach the B-operand layout of the FFN-up with one exchange of two
-// words per 16-column step between the half-waves.  The FFN-down then
-// accumulates on top of z, so y = z + FFN leaves the registers once and z never
-// goes to memory.  The one difference from the reference's autocast rounding
-// points: the FFN-down output is added to z in fp32 instead of being rounded
-// to bf16 first, a difference of at most half a bf16 ulp of the FFN output.
+// The hidden dimension is walked in chunks of 32 units: U^T = W1_c . h^T puts hidden units on the accumulator rows and
+// token rows on the columns.  The FFN-up runs as 16x16x32 MFMAs into four independent accumulators (two 16-unit hidden
+// blocks x two 16-token blocks): one exchange of the RMSNorm2 fragments per tile and one of the GELU values per chunk
+// (v_permlane16_swap) keep both sides' operand reads single 16-byte LDS reads.  After GELU (fp32 on the bf16-rounded
+// value, then bf16) those values are the B operand of y^T += W2[:, c] . G^T without leaving registers.
+// W1 and W2 chunks go global -> LDS by LDS DMA into a 2-stage ring, chunk c + 1 issued right after the barrier that
+// publishes chunk c.  Two workgroups of four waves share a CU (two waves per SIMD, 75 KB of LDS each): their barriers
+// are independent, so one's GELU, prologue and epilogue run beside the other's MFMAs (one workgroup of eight waves
+// keeps every wave of a SIMD in the same phase, and the hardware does not overlap them within a wave).
 //
 // The grid is persistent: WPS workgroups per CU walk the row tiles
 // blockIdx.x, blockIdx.x + gridDim.x, ...
 // ---------------------------------------------------------------------------
-// PDM_FFN_UP16: the FFN-up runs as 16x16x32 MFMAs into four independent accumulators (no dependent chain of
-// KS MFMAs into one), with the operand exchanges described at their code; 0: one 32x32x16 chain.
-#ifndef PDM_FFN_UP16
-#define PDM_FFN_UP16 1
-#endif
-
-template <int D, int RB, int NW, int NST, int WPS>
+template <int D, int NW, int WPS>
 __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
-  static_assert(!PDM_FFN_UP16 || RB == 1, "the 16x16x32 FFN-up assumes one row block per wave");
+  constexpr int NST = 2;                     // ring stages
   constexpr int NT = NW * 64;                // threads
   constexpr int PF = NST - 1;                // chunks read ahead
   constexpr int KS = D / 16;
   constexpr int DB = D / 32;                 // 32-row blocks of the output (d)
-  constexpr int TROWS = NW * RB * 32;
+  constexpr int TROWS = NW * 32;
   constexpr int W1_BYTES = 32 * 2 * D;       // 32 hidden units x D
   constexpr int W2_BYTES = D * 64;           // D outputs x 32 hidden units
   // one LDS block: the weight ring, reused by the epilogue's staging tile
@@ -204,8 +181,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
   // Weight chunk c goes from global memory straight into LDS (global_load_lds_dwordx4: lane l of a wave
   // writes the 16 bytes at the wave's LDS base + 16 l), so LDS piece o of a stage is loaded by thread
   // o mod NT, round o / NT, and the source address is what decides the layout.
-  // W1 stage: row r = hidden unit c*32 + r (c*32 + swap23(r), bits 2 and 3 swapped, without PDM_FFN_UP16),
-  // D columns in 2D bytes,
+  // W1 stage: row r = hidden unit c*32 + r, D columns in 2D bytes,
   // 16-byte piece v of the row at slot v ^ (r & 15), so the 32 rows of one fragment read hit distinct
   // bank groups.  W2 stage: W2[d, c*32 .. c*32+32) as D rows of 64 bytes, piece v at v ^ ((d >> 2) & 3).
   constexpr int L1 = W1_BYTES / 16 / NT;     // pieces per thread of a W1 chunk
@@ -226,8 +202,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < NLO; ++j) {
       const int r = j * RP + r0;  // < 16
-      const int hid = PDM_FFN_UP16 ? r : ((r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1));
-      off1[j] = (uint32_t)((hid * D + ((slot ^ (r & 15)) << 3)) * 2);
+      off1[j] = (uint32_t)((r * D + ((slot ^ (r & 15)) << 3)) * 2);
     }
   }
   const uint32_t off2 = (uint32_t)(((tid >> 2) * F + (((tid & 3) ^ ((tid >> 4) & 3)) * 8)) * 2);
@@ -267,10 +242,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
     W2 = gsel < 0 ? a.W2 : a.W2_ns + gsel * (int64_t)D * F;
   }
   __syncthreads();
-  u32x4_t hfr[RB][KS];
-  f32x16_t y[RB][DB];
+  u32x4_t hfr[KS];
+  f32x16_t y[DB];
   {
-    static_assert(RB == 1 && NST == 2, "the out-projection prologue assumes one row block and a 2-stage ring");
     constexpr int DW = D / 64;  // Wout chunks of 64 columns, each D rows x 128 bytes = one ring stage
     static_assert(DW % NST == 0, "FFN chunk c must keep stage c % NST");
     // Wout chunk kc: LDS row r (output feature) = Wout[r, kc*64 .. +64), rows 0 .. D/2 - 1 in the W1 part of
@@ -303,7 +277,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) y[0][db][e] = 0.0f;
+      for (int e = 0; e < 16; ++e) y[db][e] = 0.0f;
 #pragma unroll
     for (int kc = 0; kc < DW; ++kc) {
       const int stg = kc % NST;
@@ -336,7 +310,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int db = 0; db < DB; ++db) y[0][db] = mfma32x32x16(wf[s * DB + db], ofr[kc][s], y[0][db]);
+        for (int db = 0; db < DB; ++db) y[db] = mfma32x32x16(wf[s * DB + db], ofr[kc][s], y[db]);
       sched_mfma_ds_pipeline<4 * DB, 4>();
     }
     // z = bf16(O . Wout^T) + x[:, t + res_toff] in y (lane: row fr, outputs db*32 + g*8 + hf*4 + 0..3): the FFN
@@ -354,8 +328,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
       for (int g = 0; g < 4; ++g) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const float z = bf16_round(y[0][db][4 * g + j]) + xv[db][g][j];
-          y[0][db][4 * g + j] = z;
+          const float z = bf16_round(y[db][4 * g + j]) + xv[db][g][j];
+          y[db][4 * g + j] = z;
           ss += z * z;
         }
       }
@@ -371,7 +345,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
       const int db = s >> 1, g0 = 2 * (s & 1);
       const f32x4_t w0 = *reinterpret_cast<const f32x4_t*>(nw + db * 32 + g0 * 8);
       const f32x4_t w1 = *reinterpret_cast<const f32x4_t*>(nw + db * 32 + g0 * 8 + 8);
-      const f32x16_t& zb = y[0][db];
+      const f32x16_t& zb = y[db];
       const int e0 = 4 * g0;
       const uint32_t a0 = pack_bf16x2((zb[e0] * rms) * w0.x, (zb[e0 + 1] * rms) * w0.y);
       const uint32_t a1 = pack_bf16x2((zb[e0 + 2] * rms) * w0.z, (zb[e0 + 3] * rms) * w0.w);
@@ -379,11 +353,10 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
       const uint32_t b1 = pack_bf16x2((zb[e0 + 6] * rms) * w1.z, (zb[e0 + 7] * rms) * w1.w);
       const uint32_t r0 = (uint32_t)__shfl_xor((int)(hf ? a0 : b0), 32, 64);
       const uint32_t r1 = (uint32_t)__shfl_xor((int)(hf ? a1 : b1), 32, 64);
-      hfr[0][s] = hf ? u32x4_t{r0, r1, b0, b1} : u32x4_t{a0, a1, r0, r1};
+      hfr[s] = hf ? u32x4_t{r0, r1, b0, b1} : u32x4_t{a0, a1, r0, r1};
     }
   }
 
-#if PDM_FFN_UP16
   // hfr (lane l: token l % 32, columns 16 s + 8 (l / 32) .. + 7 of step s) -> the B operand of the 16x16x32
   // FFN-up, two 16-token blocks tb: hfr[2 s2 + tb] of lane l then holds token 16 tb + l % 16, columns
   // 32 s2 + 16 (G & 1) + 8 (G >> 1) .. + 7 with G = l / 16.  Lanes l and l ^ 16 (same half-wave, tokens of the
@@ -393,11 +366,10 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
   for (int s2 = 0; s2 < KS / 2; ++s2)
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const auto sw = __builtin_amdgcn_permlane16_swap(hfr[0][2 * s2][w], hfr[0][2 * s2 + 1][w], false, false);
-      hfr[0][2 * s2][w] = sw[0];
-      hfr[0][2 * s2 + 1][w] = sw[1];
+      const auto sw = __builtin_amdgcn_permlane16_swap(hfr[2 * s2][w], hfr[2 * s2 + 1][w], false, false);
+      hfr[2 * s2][w] = sw[0];
+      hfr[2 * s2 + 1][w] = sw[1];
     }
-#endif
 
   // The chunk loop is unrolled by the ring depth so that every stage index is a constant: the LDS reads of
   // stage k and the LDS DMA into stage (k + PF) % NST are then distinct objects to the compiler.
@@ -416,8 +388,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
       // it reloads the last chunk into the stage just freed, which no later chunk reads
       dma(min(c + PF, nchunks - 1), (k + PF) % NST);
       const char* w1 = sW1[k];
-      uint32_t gp[RB][8];
-#if PDM_FFN_UP16
+      uint32_t gp[8];
       // FFN-up with 16x16x32 MFMAs into four independent accumulators u4[hb][tb]: hidden units 16 hb + 4 G
       // + i (G = lane / 16, element i) of token 16 tb + lane % 16.  Step s2 takes the W1 fragment of row
       // 16 hb + lane % 16, piece 4 s2 + 2 (G & 1) + (G >> 1) (the columns the lane's hfr pieces hold).
@@ -441,8 +412,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
 #pragma unroll
         for (int w = 0; w < 2; ++w) {
           const auto sw = __builtin_amdgcn_permlane16_swap(t[w], t[2 + w], false, false);
-          gp[0][4 * h2 + w] = sw[0];
-          gp[0][4 * h2 + 2 + w] = sw[1];
+          gp[4 * h2 + w] = sw[0];
+          gp[4 * h2 + 2 + w] = sw[1];
         }
       };
       {
@@ -459,7 +430,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
 #pragma unroll
           for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
-            for (int tb = 0; tb < 2; ++tb) u4[hb][tb] = mfma16x16x32(wf[2 * s2 + hb], hfr[0][2 * s2 + tb], u4[hb][tb]);
+            for (int tb = 0; tb < 2; ++tb) u4[hb][tb] = mfma16x16x32(wf[2 * s2 + hb], hfr[2 * s2 + tb], u4[hb][tb]);
         // 4 fragment reads ahead, then 4 MFMAs and the next step's 2 reads in turn
         __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
@@ -470,41 +441,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
       }
       gelu_half(0);
-#else
-      // FFN-up: U^T[rb] = W1_c . h[rb]^T, each W1 fragment feeding RB MFMAs
-      f32x16_t u[RB];
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) u[rb][e] = 0.0f;
-      {
-        u32x4_t wf[KS];
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-          wf[s] = *reinterpret_cast<const u32x4_t*>(w1 + fr * (2 * D) + (((2 * s + hf) ^ (fr & 15)) << 4));
-#pragma unroll
-        for (int s = 0; s < KS; ++s)
-#pragma unroll
-          for (int rb = 0; rb < RB; ++rb) u[rb] = mfma32x32x16(wf[s], hfr[rb][s], u[rb]);
-        if constexpr (RB == 1) sched_mfma_ds_pipeline<KS, 3>();
-      }
-      // G = bf16(gelu(bf16(U))): u[rb][e] is hidden unit (e/4)*8 + hf*4 + e%4 (LDS row order) of token fr.
-      auto gelu_half = [&](int h2) {
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          float uv[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) uv[e] = u[rb][8 * h2 + e];
-          gelu_lut_pack<8>(sGelu, uv, gp[rb] + 4 * h2);
-        }
-      };
-#endif
       // The first half (G^T chunk c2 = 0) is computed before the FFN-down; the second half between the c2 = 0
       // MFMAs, which do not need it
-#if !PDM_FFN_UP16
-      gelu_half(0);
-#endif
-      // FFN-down: y^T[rb][db] += W2[db rows, chunk c] . G[rb]^T; chunk c2 of G^T holds hidden units
+      // FFN-down: y^T[db] += W2[db rows, chunk c] . G^T; chunk c2 of G^T holds hidden units
       // 16*c2 + hf*8 + 0..7, piece 2*c2 + hf of W2 row d, stored at (2*c2 + hf) ^ ((d >> 2) & 3)
       const char* w2 = sW2[k];
       {
@@ -522,50 +461,46 @@ __global__ __launch_bounds__(NW * 64, WPS) void ffn_kernel(GemmArgs a) {
 #pragma unroll
         for (int c2 = 0; c2 < 2; ++c2) {
 #pragma unroll
-          for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-              const u32x4_t gb = {gp[rb][4 * c2], gp[rb][4 * c2 + 1], gp[rb][4 * c2 + 2], gp[rb][4 * c2 + 3]};
-              y[rb][db] = mfma32x32x16(wf[c2 * DB + db], gb, y[rb][db]);
-            }
+          for (int db = 0; db < DB; ++db) {
+            const u32x4_t gb = {gp[4 * c2], gp[4 * c2 + 1], gp[4 * c2 + 2], gp[4 * c2 + 3]};
+            y[db] = mfma32x32x16(wf[c2 * DB + db], gb, y[db]);
+          }
         }
       }
     }
   }
 
-  // Epilogue.  y[rb][db][e] is output d = db*32 + (e/4)*8 + hf*4 + e%4 of row wave*RB*32 + rb*32 + fr.
+  // Epilogue.  y[db][e] is output d = db*32 + (e/4)*8 + hf*4 + e%4 of row wave*32 + fr.
   // y already holds z + FFN (the FFN-down accumulated on top of z).  The values go through LDS (the weight ring is
   // free now) SEG outputs at a time, so that y is written as whole row segments of SEG outputs, with non-temporal
   // stores (y is streamed to memory; the next kernel reads it from there).
-  constexpr int SEG = NW * RB * 32 * (64 * 4 + 16) <= RING_BYTES ? 64 : 32;  // outputs per pass
+  constexpr int SEG = NW * 32 * (64 * 4 + 16) <= RING_BYTES ? 64 : 32;  // outputs per pass
   constexpr int SROW = SEG * 4 + 16;       // LDS row stride (bytes), padded against bank conflicts
   constexpr int NQ = D / SEG;              // passes
-  constexpr int EK = RB * 32 * (SEG / 4) / 64;  // 16-byte pieces per lane and pass
-  static_assert(NW * RB * 32 * SROW <= RING_BYTES, "epilogue staging must fit the weight ring");
+  constexpr int EK = 32 * (SEG / 4) / 64;  // 16-byte pieces per lane and pass
+  static_assert(NW * 32 * SROW <= RING_BYTES, "epilogue staging must fit the weight ring");
   int64_t eoff[EK];  // piece k of this lane: its row's output offset + its 4 columns (pass 0), or -1
 #pragma unroll
   for (int k = 0; k < EK; ++k) {
-    const int piece = k * 64 + lane;     // 16-byte piece of the wave's RB*32 x SEG tile
+    const int piece = k * 64 + lane;     // 16-byte piece of the wave's 32 x SEG tile
     const int r = piece / (SEG / 4), c4 = piece - (piece / (SEG / 4)) * (SEG / 4);
-    const int row = wave * RB * 32 + r;
+    const int row = wave * 32 + r;
     const int b = s_rb[row];
     eoff[k] = b < 0 ? -1 : (int64_t)b * a.out_bstride + (int64_t)s_rt[row] * D + c4 * 4;
   }
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);  // the last DMA must land before the ring is reused
   __syncthreads();
-  char* stage = sRing + wave * (RB * 32 * SROW);
+  char* stage = sRing + wave * (32 * SROW);
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
+    for (int db2 = 0; db2 < SEG / 32; ++db2) {
+      const int db = q * (SEG / 32) + db2;
 #pragma unroll
-      for (int db2 = 0; db2 < SEG / 32; ++db2) {
-        const int db = q * (SEG / 32) + db2;
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4_t*>(stage + (rb * 32 + fr) * SROW + (db2 * 32 + g * 8 + hf * 4) * 4) =
-              f32x4_t{y[rb][db][4 * g], y[rb][db][4 * g + 1], y[rb][db][4 * g + 2], y[rb][db][4 * g + 3]};
-      }
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4_t*>(stage + fr * SROW + (db2 * 32 + g * 8 + hf * 4) * 4) =
+            f32x4_t{y[db][4 * g], y[db][4 * g + 1], y[db][4 * g + 2], y[db][4 * g + 3]};
+    }
     // each wave reads back only its own tile; a wave's LDS accesses execute in order, so no barrier
 #pragma unroll
     for (int k = 0; k < EK; ++k) {
@@ -1201,48 +1136,24 @@ static int64_t row_tiles(GemmArgs& g, int rows_per_tile) {
   return (int64_t)g.tiles_s + (int64_t)g.n_ns * g.tiles_b;
 }
 
-// FFN launch shape: RB * 32 rows per wave, NW waves per workgroup, an NST-stage
-// weight ring, WPS workgroups per CU.  Two workgroups of four 32-row waves per
-// CU (two waves per SIMD, 2-stage ring, 75 KB of LDS each) measured fastest at
-// d_model 256: the workgroups' barriers are independent, so one's GELU,
-// prologue and epilogue run beside the other's MFMAs (one workgroup of eight
-// waves keeps every wave of a SIMD in the same phase).
-#ifndef PDM_FFN_RB
-#define PDM_FFN_RB 1
-#endif
-#ifndef PDM_FFN_NW
-#define PDM_FFN_NW 4
-#endif
-#ifndef PDM_FFN_NST
-#define PDM_FFN_NST 2
-#endif
-#ifndef PDM_FFN_WPS
-#define PDM_FFN_WPS 2
-#endif
-// The FFN grid is persistent (WPS workgroups per CU walk the row tiles; 0: one workgroup per tile).
-#ifndef PDM_FFN_PERSIST
-#define PDM_FFN_PERSIST 1
-#endif
+// Two workgroups of four waves per CU walk the row tiles of the fused FFN.
 static int launch_ffn(GemmArgs& g, int D, hipStream_t s) {
-  constexpr int RB = PDM_FFN_RB, NW = PDM_FFN_NW, NST = PDM_FFN_NST, WPS = PDM_FFN_WPS;
-  const int64_t tiles = row_tiles(g, NW * RB * 32);
+  constexpr int NW = 4, WPS = 2;
+  const int64_t tiles = row_tiles(g, NW * 32);
   if (tiles == 0) return PDM_OK;
   PDM_CHECK_ARG(tiles < (int64_t(1) << 31), "FFN grid too large");
   g.total_blocks = tiles;
-  int64_t grid = tiles;
-  if (PDM_FFN_PERSIST) {
-    static std::once_flag once[64];
-    static hipError_t err[64];
-    static int ncu[64];
-    int dev = 0;
-    PDM_CHECK_HIP(hipGetDevice(&dev));
-    PDM_CHECK_ARG(dev >= 0 && dev < 64, "device index out of range");
-    std::call_once(once[dev], [&] { err[dev] = hipDeviceGetAttribute(&ncu[dev], hipDeviceAttributeMultiprocessorCount, dev); });
-    PDM_CHECK_HIP(err[dev]);
-    grid = std::min<int64_t>(tiles, (int64_t)std::max(ncu[dev], 1) * WPS);
-  }
-  if (D == 256) hipLaunchKernelGGL((ffn_kernel<256, RB, NW, NST, WPS>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
-  else hipLaunchKernelGGL((ffn_kernel<128, RB, NW, NST, WPS>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
+  static std::once_flag once[64];
+  static hipError_t err[64];
+  static int ncu[64];
+  int dev = 0;
+  PDM_CHECK_HIP(hipGetDevice(&dev));
+  PDM_CHECK_ARG(dev >= 0 && dev < 64, "device index out of range");
+  std::call_once(once[dev], [&] { err[dev] = hipDeviceGetAttribute(&ncu[dev], hipDeviceAttributeMultiprocessorCount, dev); });
+  PDM_CHECK_HIP(err[dev]);
+  const int64_t grid = std::min<int64_t>(tiles, (int64_t)std::max(ncu[dev], 1) * WPS);
+  if (D == 256) hipLaunchKernelGGL((ffn_kernel<256, NW, WPS>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
+  else hipLaunchKernelGGL((ffn_kernel<128, NW, WPS>), dim3((unsigned)grid), dim3(NW * 64), 0, s, g);
   PDM_CHECK_LAUNCH();
   return PDM_OK;
 }
@@ -1386,7 +1297,7 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     PDM_CHECK_LAUNCH();
   }
   if (fused_path(d)) {
-    // 3. z = bf16(O . Wout^T) + x[:, kv - q_len:], y = z + bf16(W2 . gelu(W1 . RMSNorm2(z))):
+    // 3. z = bf16(O . Wout^T) + x[:, kv - q_len:], y = z + W2 . gelu(W1 . RMSNorm2(z)):
     // out-projection, norm, both FFN GEMMs and GELU in one kernel
     GemmArgs g2{};
     g2.A = q; g2.a_bstride = (int64_t)ql * D;
@@ -1422,7 +1333,7 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     r2.h = (d.flags & PDM_BLOCK_KEEP_NORM2) ? h : nullptr; r2.out = g; r2.out_bstride = (int64_t)ql * F;
     if ((st = launch_row_proj(r2, D, ROWPROJ_GELU, s)) != PDM_OK) return st;
   }
-  // 5. y = z + bf16(g . W2^T)
+  // 5. y = z + g . W2^T
   {
     ResidArgs g3{};
     g3.A = g; g3.a_bstride = (int64_t)ql * F;

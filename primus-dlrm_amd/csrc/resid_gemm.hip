@@ -9,7 +9,6 @@
 // shared weight, every NS token has row tiles of its own with its own weight; rows past the end read the tile's last
 // row again and are not stored.
 #include <algorithm>
-#include <mutex>
 
 #include "pdm_common.h"
 #include "mfma_common.h"
@@ -171,7 +170,7 @@ static int launch_tiles(ResidArgs a, hipStream_t s) {
   a.tiles_b = (a.B + TM - 1) / TM;
   const int64_t grid = (tiles_s + (int64_t)a.n_ns * a.tiles_b) * (a.N / TN);
   if (grid == 0) return PDM_OK;
-  PDM_CHECK_ARG(grid < (int64_t(1) << 31), "GEMM grid too large");
+  PDM_CHECK_ARG(grid < (int64_t(1) << 24), "GEMM grid too large");  // a launch dimension holds less than 2^32 threads
   // a tile's rows lie within 2^32 bytes of its first sample, and its weight rows of its first
   const int64_t samples = std::min<int64_t>(a.B, std::max(a.n_s ? (TM - 2) / a.n_s + 2 : 1, a.n_ns ? TM : 1));
   PDM_CHECK_ARG(samples * a.a_bstride * 2 < (int64_t(1) << 32), "GEMM rows too far apart");

@@ -443,7 +443,8 @@ static int launch_one(RowProjArgs a, hipStream_t s) {
   a.split_tok = (int)std::max<int64_t>(1, std::min<int64_t>(nchunks, (round - wgs_s * a.split_s) / std::max<int64_t>(1, wgs_tok)));
   const int64_t grid = wgs_s * a.split_s + wgs_tok * a.split_tok;
   if (grid == 0) return PDM_OK;
-  PDM_CHECK_ARG(grid < (int64_t(1) << 31), "row projection grid too large");
+  // a launch dimension holds less than 2^32 threads
+  PDM_CHECK_ARG(grid < (int64_t(1) << 24), "row projection grid too large");
   // the 32 features of a V^T tile lie within 2^31 bytes of the first
   PDM_CHECK_ARG((int64_t)32 * a.kv_pad * 2 < (int64_t(1) << 31), "row projection rows too far apart");
   a.wgs_s = (int)wgs_s;
