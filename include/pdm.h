@@ -375,7 +375,10 @@ typedef struct {
 
 /* Bytes of device workspace pdm_onetrans_block_fwd needs for desc.  It never
  * falls as batch, kv_len or q_len grows with the rest unchanged: a workspace
- * sized for the largest batch is enough for every smaller one. */
+ * sized for the largest batch is enough for every smaller one.  At d_model 256
+ * the call also takes one that holds Q [B, q_len, D], K [B, kv_len, D] and V^T
+ * [B, D, kv_len rounded up to 64] in bf16 alone, each rounded up to 256 bytes,
+ * and then runs the one-kernel FFN at any size. */
 int64_t pdm_onetrans_block_workspace_size(const pdm_block_desc* desc);
 
 /* x: device fp32 [B, kv_len, D] (the residual stream); y: device fp32
@@ -401,7 +404,8 @@ int pdm_onetrans_block_fwd(const pdm_block_desc* desc, const float* x,
 #define PDM_STACK_MAX_LAYERS 64
 
 /* Bytes of device workspace pdm_onetrans_stack_fwd needs; like the block's, it
- * never falls as batch, kv_len or an entry of q_s grows. */
+ * never falls as batch, kv_len or an entry of q_s grows, and at d_model 256 the
+ * largest layer's Q, K and V^T and the inner outputs alone are also taken. */
 int64_t pdm_onetrans_stack_workspace_size(const pdm_block_desc* desc,
                                           const int32_t* q_s, int32_t n_layers);
 

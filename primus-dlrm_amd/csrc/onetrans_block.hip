@@ -1101,7 +1101,9 @@ static int64_t split_rows(const pdm_block_desc& d) { return std::min((int64_t)d.
 // 62 against 49 us, 102,400 rows 277 against 274 us (whole block), 204,800 rows 448 against 461 us (whole block).
 constexpr int64_t kQkvStationaryMinRows = 120000;
 
-static BlockLayout block_layout(const pdm_block_desc& d) {
+// room: with space for h and g wherever split_rows asks for it; without it a d_model 256 block runs the fused FFN
+// whatever its rows, so that a workspace of Q, K and V^T is enough at any size.
+static BlockLayout block_layout(const pdm_block_desc& d, bool room = true) {
   BlockLayout L;
   const int64_t B = d.batch, D = d.d_model;
   L.kv_pad = (d.kv_len + 31) & ~31;
@@ -1110,7 +1112,7 @@ static BlockLayout block_layout(const pdm_block_desc& d) {
   L.q = off; off = align256(off + B * d.q_len * D * 2);                 // Q, later attention output
   L.k = off; off = align256(off + B * d.kv_len * D * 2);                // K
   L.vt = off; off = align256(off + B * (D / 64) * 64 * (int64_t)L.vt_ld * 2);  // V^T per head
-  const int64_t rows = split_rows(d);
+  const int64_t rows = room || d.d_model > 256 ? split_rows(d) : 0;
   L.h = off; off = align256(off + rows * D * 2);                        // RMSNorm2 rows
   L.g = off; off = align256(off + rows * (int64_t)d.ffn_dim * 2);       // GELU(FFN-up)
   L.total = off;
@@ -1225,10 +1227,11 @@ extern "C" int64_t pdm_onetrans_block_workspace_size(const pdm_block_desc* desc)
 
 namespace pdm {
 
-// One block on stream s; the descriptor is checked, the pointers are not.
+// One block on stream s; the descriptor is checked, the pointers are not.  room: as block_layout's.
 static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_weights* w, float* y, void* workspace,
-                     hipStream_t s) {
-  const BlockLayout L = block_layout(d);
+                     bool room, hipStream_t s) {
+  const BlockLayout L = block_layout(d, room);
+  const bool fused = fused_path(d) || (d.d_model == 256 && !room);
   char* ws = reinterpret_cast<char*>(workspace);
   uint16_t* h = reinterpret_cast<uint16_t*>(ws + L.h);
   uint16_t* q = reinterpret_cast<uint16_t*>(ws + L.q);
@@ -1296,7 +1299,7 @@ static int block_fwd(const pdm_block_desc& d, const float* x, const pdm_block_we
     }
     PDM_CHECK_LAUNCH();
   }
-  if (fused_path(d)) {
+  if (fused) {
     // 3. z = bf16(O . Wout^T) + x[:, kv - q_len:], y = z + W2 . gelu(W1 . RMSNorm2(z)):
     // out-projection, norm, both FFN GEMMs and GELU in one kernel
     GemmArgs g2{};
@@ -1371,15 +1374,16 @@ extern "C" int pdm_onetrans_block_fwd(const pdm_block_desc* desc, const float* x
   PDM_CHECK_ARG(x && w && y && workspace, "null pointer");
   int st;
   if ((st = check_block_weights(d, w)) != PDM_OK) return st;
-  const BlockLayout L = block_layout(d);
-  if (workspace_bytes < L.total) {
+  const int64_t need = block_layout(d).total;
+  const bool room = workspace_bytes >= need;
+  if (!room && workspace_bytes < block_layout(d, false).total) {
     set_error("pdm_onetrans_block_fwd: workspace of " + std::to_string(workspace_bytes) + " bytes, need " +
-              std::to_string(L.total));
+              std::to_string(need));
     return PDM_ERR_WORKSPACE;
   }
   PDM_CHECK_ARG(aligned16(x) && aligned16(y) && aligned16(workspace), "every tensor must be 16-byte aligned");
   PDM_CHECK_ARG((const void*)y != (const void*)x, "y must not alias x");
-  return block_fwd(d, x, w, y, workspace, reinterpret_cast<hipStream_t>(stream));
+  return block_fwd(d, x, w, y, workspace, room, reinterpret_cast<hipStream_t>(stream));
 }
 
 // ---------------------------------------------------------------------------
@@ -1397,7 +1401,8 @@ struct StackLayout {
   int64_t total;
 };
 
-static const char* stack_layout(const pdm_block_desc* desc, const int32_t* q_s, int32_t n_layers, StackLayout& S) {
+static const char* stack_layout(const pdm_block_desc* desc, const int32_t* q_s, int32_t n_layers, StackLayout& S,
+                                bool room = true) {
   if (!desc) return "null desc";
   if (!q_s) return "null q_s";
   if (n_layers < 1 || n_layers > PDM_STACK_MAX_LAYERS) return "n_layers must be in [1, PDM_STACK_MAX_LAYERS]";
@@ -1407,7 +1412,7 @@ static const char* stack_layout(const pdm_block_desc* desc, const int32_t* q_s, 
     if (q_s[l] < 0) return "q_s must be >= 0";
     d.q_len = q_s[l] + desc->n_ns;
     if (const char* e = check_desc(&d)) return e;
-    block = std::max(block, block_layout(d).total);
+    block = std::max(block, block_layout(d, room).total);
     if (l + 1 < n_layers) inner = std::max(inner, align256((int64_t)d.batch * d.q_len * d.d_model * 4));
     d.kv_len = d.q_len;
   }
@@ -1441,9 +1446,12 @@ extern "C" int pdm_onetrans_stack_fwd(const pdm_block_desc* desc, const int32_t*
     return PDM_ERR_INVALID;
   }
   PDM_CHECK_ARG(x && weights && y && workspace, "null pointer");
+  const int64_t need = S.total;
+  const bool room = workspace_bytes >= need;
+  if (!room) stack_layout(desc, q_s, n_layers, S, false);
   if (workspace_bytes < S.total) {
     set_error("pdm_onetrans_stack_fwd: workspace of " + std::to_string(workspace_bytes) + " bytes, need " +
-              std::to_string(S.total));
+              std::to_string(need));
     return PDM_ERR_WORKSPACE;
   }
   PDM_CHECK_ARG(aligned16(x) && aligned16(y) && aligned16(workspace), "every tensor must be 16-byte aligned");
@@ -1458,7 +1466,7 @@ extern "C" int pdm_onetrans_stack_fwd(const pdm_block_desc* desc, const int32_t*
   for (int l = 0; l < n_layers; ++l) {
     d.q_len = q_s[l] + desc->n_ns;
     float* out = l + 1 == n_layers ? y : reinterpret_cast<float*>(ws + S.buf[l & 1]);
-    if ((st = block_fwd(d, in, &weights[l], out, ws, s)) != PDM_OK) return st;
+    if ((st = block_fwd(d, in, &weights[l], out, ws, room, s)) != PDM_OK) return st;
     in = out;
     d.kv_len = d.q_len;
   }

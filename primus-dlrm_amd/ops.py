@@ -700,14 +700,16 @@ def onetrans_block_raw(x: torch.Tensor, w: Dict[str, torch.Tensor], n_heads: int
         raise L.PdmError(ws_bytes, "pdm_onetrans_block_workspace_size", L.last_error())
     if workspace is None:
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    elif workspace.dtype != torch.uint8 or workspace.numel() < ws_bytes or workspace.device != dev:
+    elif workspace.dtype != torch.uint8 or workspace.device != dev:
         raise ValueError(f"workspace must be a uint8 tensor of >= {ws_bytes} bytes on {dev}")
     ws = workspace
     if out is None:
         out = torch.empty((B, q_len, D), dtype=torch.float32, device=dev)
     bw = L.BlockWeights(*[w[k].data_ptr() for k in names])
     status = L.lib().pdm_onetrans_block_fwd(ctypes.byref(desc), x.data_ptr(), ctypes.byref(bw), out.data_ptr(),
-                                            ws.data_ptr(), ws_bytes, L.stream_ptr(dev))
+                                            ws.data_ptr(), ws.numel(), L.stream_ptr(dev))
+    if status == L.PDM_ERR_WORKSPACE:
+        raise ValueError(f"workspace must be a uint8 tensor of >= {ws_bytes} bytes on {dev}")
     L.check(status, "pdm_onetrans_block_fwd")
     return out
 
@@ -773,13 +775,15 @@ def onetrans_stack_raw(x: torch.Tensor, layers: Sequence[Dict[str, torch.Tensor]
     ws_bytes = onetrans_stack_workspace_bytes(B, kv, D, Fd, n_ns, n_heads, q_s)
     if workspace is None:
         workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-    elif workspace.dtype != torch.uint8 or workspace.numel() < ws_bytes or workspace.device != dev:
+    elif workspace.dtype != torch.uint8 or workspace.device != dev:
         raise ValueError(f"workspace must be a uint8 tensor of >= {ws_bytes} bytes on {dev}")
     if out is None:
         out = torch.empty((B, int(q_s[-1]) + n_ns, D), dtype=torch.float32, device=dev)
     bw = (L.BlockWeights * n)(*[L.BlockWeights(*[w[k].data_ptr() for k in _BLOCK_WEIGHT_NAMES]) for w in layers])
     status = L.lib().pdm_onetrans_stack_fwd(ctypes.byref(desc), qs, n, x.data_ptr(), bw, out.data_ptr(),
-                                            workspace.data_ptr(), ws_bytes, L.stream_ptr(dev))
+                                            workspace.data_ptr(), workspace.numel(), L.stream_ptr(dev))
+    if status == L.PDM_ERR_WORKSPACE:
+        raise ValueError(f"workspace must be a uint8 tensor of >= {ws_bytes} bytes on {dev}")
     L.check(status, "pdm_onetrans_stack_fwd")
     return out
 

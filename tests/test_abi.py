@@ -123,7 +123,7 @@ def test_stack_workspace_size(pdm):
     assert size(B, kv, D, Fd, ns, [384, 256, 128, 64]) == a(block0) + 2 * inner
     assert size(B, kv, D, Fd, ns, [384, 256]) == a(block0) + inner
     assert size(B, kv, D, Fd, ns, [384]) == a(block0)
-    # the tiled path (d_model 384) holds h and g too: still layer 0's block workspace
+    # d_model 384 holds h and g too: still layer 0's block workspace
     blk384 = pdm.ops.onetrans_workspace_layout(4, 60, 40 + 3, 384, 1536)["total"][0]
     assert size(4, 60, 384, 1536, 3, [40, 20]) == a(blk384) + a(4 * 43 * 384 * 4)
     assert size(B, kv, D, Fd, ns, [384, 390]) == L.PDM_ERR_INVALID  # layer 1 keeps more than its kv

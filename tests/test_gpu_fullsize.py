@@ -113,6 +113,6 @@ def test_onetrans_stack_b1024_sampled_samples(pdm, dev):
 
 
 def test_onetransl_stack_b1024_sampled_samples(pdm, dev):
-    """The reference's OneTransL shape at B = 1024: d_model 384 (tiled path), 1516 tokens, the 8-layer pyramid
+    """The reference's OneTransL shape at B = 1024: d_model 384 (separate FFN kernels), 1516 tokens, the 8-layer pyramid
     1500 -> 16; layers 0-5 run the streaming attention (kv 1516 .. 668)."""
     _stack_sampled(pdm, dev, 384, 1536, 16, 1024, [1500, 1288, 1076, 864, 652, 440, 228, 16], 4, 700)

@@ -82,7 +82,7 @@ def _check_layer(pdm, dev, x, w, q_len, label="", v_sums=False):
         h_max = (x * x.square().mean(-1, keepdim=True).rsqrt() * w["norm1"]).abs().max().item()
         o_terms = o_terms + (terms["v"].max().item() * D * 2.0 ** -24 + 2 * 2.0 ** -8 * h_max * w_max) / ELEM_TOL
     _close("attention out", o, parts["o"], o_terms)
-    if "g" in layout:  # the tiled path keeps RMSNorm2 rows and GELU activations in the workspace
+    if "g" in layout:  # the separate FFN kernels keep RMSNorm2 rows and GELU activations in the workspace
         g = _ws_view(ws, layout, "g", (B, q_len, F))
         h2 = _ws_view(ws, layout, "h", (B, q_len, D))
         _close("rmsnorm2", h2, parts["h2"].to(torch.bfloat16), terms["h2"])
@@ -119,12 +119,12 @@ def test_block_d128_ffn384_and_norm_weights(pdm, dev):
 
 
 def test_block_d384_tiled_path(pdm, dev):
-    """d_model 384 (the reference's OneTransL width) runs the tiled GEMM path."""
+    """d_model 384 (the reference's OneTransL width) runs the FFN as separate kernels."""
     _run_case(pdm, dev, 5, 45, 21, 3, D=384, F=1536, seed=8, norm_std=0.2)
 
 
 def test_block_d512_tiled_path(pdm, dev):
-    """d_model 512 (8 heads) on the tiled GEMM path."""
+    """d_model 512 (8 heads), the FFN as separate kernels."""
     _run_case(pdm, dev, 3, 40, 20, 3, D=512, F=2048, seed=9, norm_std=0.2)
 
 
@@ -199,6 +199,36 @@ def test_block_stores_norm2_rows_only_on_request(pdm, dev, D):
         kept.append(bool((ws[off:off + size] == 0xAB).all()))
     assert kept == [True, False]
     assert torch.equal(outs[0], outs[1])
+
+
+def test_block_and_stack_workspace_without_room_for_the_split_ffn(pdm, dev):
+    """d_model 256: a workspace of Q, K and V^T alone runs the fused FFN on a small batch (checked against the oracle),
+    one byte less is refused, and so for a stack, whose guard bytes behind the workspace stay untouched."""
+    B, kv, q_len, n_ns, D, F = 5, 70, 37, 4, 256, 512
+    w = ot.random_weights(D, F, n_ns, std=0.02, seed=24, norm_std=0.1)
+    wd = _gpu_weights(w, dev)
+    x = torch.randn(B, kv, D, generator=torch.Generator().manual_seed(24))
+    least = pdm.ops.onetrans_workspace_layout(B, kv, q_len, D, F)["h"][0]
+    full = torch.full((least + 4096,), 0xAB, dtype=torch.uint8, device=dev)
+    got = pdm.ops.onetrans_block_raw(x.to(dev), wd, D // 64, q_len, workspace=full[:least]).cpu()
+    assert bool((full[least:] == 0xAB).all())
+    want, parts = ot.block_forward(x, w, q_len, D // 64, mode="autocast", return_parts=True)
+    tail = x[:, kv - q_len:]
+    _close("block update y - x_tail", got - tail, want - tail,
+           ot.term_magnitudes(x, w, q_len, D // 64, parts)["y"])
+    with pytest.raises(ValueError, match="workspace"):
+        pdm.ops.onetrans_block_raw(x.to(dev), wd, D // 64, q_len, workspace=full[:least - 1])
+    # a stack: the largest layer's Q, K, V^T, then two buffers of the largest inner output
+    q_s = [60, 33, 20]
+    least = pdm.ops.onetrans_workspace_layout(B, kv, 64, D, F)["h"][0] + 2 * ((B * 64 * D * 4 + 255) // 256 * 256)
+    full = torch.full((least + 4096,), 0xAB, dtype=torch.uint8, device=dev)
+    got = pdm.ops.onetrans_stack_raw(x.to(dev), [wd] * 3, D // 64, q_s, workspace=full[:least]).cpu()
+    assert bool((full[least:] == 0xAB).all())
+    want = ot.stack_forward(x, [w] * 3, q_s, D // 64)
+    tail = x[:, kv - 24:].double()
+    assert ((got.double() - want.double()).norm() / (want.double() - tail).norm()).item() <= 1e-2
+    with pytest.raises(ValueError, match="workspace"):
+        pdm.ops.onetrans_stack_raw(x.to(dev), [wd] * 3, D // 64, q_s, workspace=full[:least - 1])
 
 
 def test_block_wide_ffn(pdm, dev):
@@ -303,7 +333,7 @@ def test_block_residual_192_row_tiles(pdm, dev, B, kv, q_len, n_ns, D, F):
     (2, 720, 300, 256),    # above the LDS-resident attention's 608 keys: the streaming attention kernel
     (1, 1516, 1516, 256),  # the reference OneTransL's first layer (L_S = 1500 + 16 NS, full causal)
     (3, 1000, 700, 384),   # 6 heads: 18 (sample, head) pairs x 3 query blocks of 256, the last partial
-    (2, 650, 650, 384),    # just above 608 keys, full causal, tiled d_model 384 path
+    (2, 650, 650, 384),    # just above 608 keys, full causal, d_model 384
 ])
 def test_block_long_sequence_streaming_attention(pdm, dev, B, kv, q_len, D):
     _run_case(pdm, dev, B, kv, q_len, 16, D=D, F=4 * D, seed=kv, norm_std=0.1)
