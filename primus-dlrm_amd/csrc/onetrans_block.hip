@@ -1083,9 +1083,11 @@ static int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 // d_model 128, and 256 above kFusedMinRows kept rows, run the out-projection, RMSNorm2 and the FFN in one kernel, whose
 // tiles of 128 rows walk the whole hidden dimension one after another: 50 us at d_model 256 however few rows there are,
 // 53 us for 17,408 rows, 81 us for 34,816.  Below, and at d_model 384 / 512 (whose rows do not fit its registers), three
-// kernels split that work over the chip: 30 us for 4,352 rows, 57 us for 17,408, 112 us for 34,816.  (At d_model 128 the
-// one kernel is the faster at every size: 1 sample 43 against 49 us per block.)  The three keep the GELU activations (g)
-// in the workspace, and RMSNorm2's rows (h) for a caller that asks for them.
+// kernels split that work over the chip: 30 us for 4,352 rows, 57 us for 17,408, 112 us for 34,816.  (Those are for a
+// hidden dimension of 1,024; from 128 to 4,096 hidden units and 0 to 64 NS tokens, blocks of 256 to 13,952 rows took at
+// most 0.98 of their time with the one kernel and the weight-stationary projection.  At d_model 128 the one kernel is the
+// faster at every size: 1 sample 43 against 49 us per block.)  The three keep the GELU activations (g) in the workspace,
+// and RMSNorm2's rows (h) for a caller that asks for them.
 // The residual GEMM reaches the rows of g within 2^32 bytes, so d_model 256 takes the three only where all of g lies in them.
 constexpr int64_t kFusedMinRows = 14000;
 static int64_t split_max_rows(const pdm_block_desc& d) {  // kept rows up to which the three kernels run

@@ -14,12 +14,13 @@
 // rows (the last block of a sample, samples past the batch) read the block's last row again and store nothing.
 //
 // What bounds it, at OneTransL's second layer (d 384, B = 1024, 1,552,384 rows in, 1,335,296 kept): the fp32 rows in and
-// the bf16 outputs out (5.8 GB for Q/K/V, about 1.2 ms at a device copy's rate; 1.37 TFLOP, 0.55 ms of MFMA), behind
-// them the vector instructions between the MFMAs.  Q/K/V 1.72 ms against 0.63 (RMSNorm kernel) + 2.52 ms (128 x 256
-// LDS-tiled GEMM); FFN-up + GELU 2.0 ms against 0.53 + 2.61 ms.  What that took: addresses kept in registers and the
-// GELU table reached by one shift (231 -> 144 vector instructions per chunk: 2.20 -> 2.00 ms), whole 64-byte segments
-// per store, the NS tiles spread over the XCDs (2.14 -> 1.86 ms for Q/K/V).  64 rows per wave (half the LDS reads and
-// weight traffic) need 192 operand registers and leave none to overlap the stores: 1.88 ms without the norm.
+// the bf16 outputs out (6.5 GB at the L2 for Q/K/V, 7.2 GB for FFN-up, 1.4 and 1.5 ms at a device copy's rate; 1.37 TFLOP,
+// 0.55 ms of MFMA), behind them the vector instructions between the MFMAs (matrix units busy 43 and 44 %).  Q/K/V 1.70 ms
+// against 0.63 (RMSNorm kernel) + 2.52 ms (128 x 256 LDS-tiled GEMM); FFN-up + GELU 1.97 ms against 0.53 + 2.61 ms.  What
+// that took: addresses kept in registers and the GELU table reached by one shift (231 -> 144 vector instructions per
+// chunk: 2.20 -> 2.00 ms), whole 64-byte segments per store, the NS tiles spread over the XCDs (2.14 -> 1.86 ms for
+// Q/K/V), the normalised rows not stored (2.19 -> 1.97 ms for FFN-up).  64 rows per wave (half the LDS reads and weight
+// traffic) need 192 operand registers and leave none to overlap the stores: 1.88 ms without the norm.
 //
 // Workgroups split the N columns of one row tile when there are few row tiles, so that a small batch fills the chip;
 // the splits of a tile are neighbours on one XCD, whose L2 then serves the rows to all of them (4 layers of d 128 at

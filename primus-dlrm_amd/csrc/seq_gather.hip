@@ -243,13 +243,12 @@ SeqShape seq_shape(int vb, int pieces, int64_t num_tokens, int64_t table_bytes) 
     if (pieces > 16 && pieces <= 32 && num_tokens >= kSome) return {32, 8};
     if (pieces > 48 && pieces <= 64 && num_tokens >= kMany) return {32, 8};
     if (pieces > 128 && pieces <= 256 && num_tokens >= kSome) return {64, 4};
-  } else if (table_bytes > kInfinityCache) {
-    // rows from memory instead of the caches have a longer way: 64 pieces 16x4x2 88 / 131, 32x2x8 97 / 114; 256 pieces
-    // 64x4x2 345 / 475, 64x4x8 370 / 449 (98,304 tokens 93 / 123 and 97 / 110); 48 pieces, 768,000 tokens 16x3x2 220,
-    // 16x3x8 176 (from memory; 262,144 tokens 48 and 53)
-    if (pieces >= 40 && pieces <= 48 && num_tokens >= 2 * kMost) return {16, 8};
-    if (pieces > 48 && pieces <= 64 && num_tokens >= kMost / 2 * 3) return {32, 8};
-    if (pieces == 256 && num_tokens >= kMany) return {64, 8};
+  } else if (pieces > 192 && pieces <= 256 && num_tokens >= 2 * kMost && table_bytes > kInfinityCache) {
+    // 16-byte pieces: more tokens per group help rows that come from memory and cost those from the caches, and ids are
+    // skewed.  Zipf(1.1) / uniform ids, 786,432 tokens: 48 pieces (bf16 256 + 64 + 64 of 10,000,000 rows) 16x3x2 124 /
+    // 222, 16x3x4 133 / 206, 16x3x8 141 / 198; 64 pieces of 4,000,000 rows 16x4x2 147 / 246, 32x2x4 156 / 244, 16x4x8
+    // 185 / 251.  Only the widest rows gain with both: 256 pieces of 1,500,000 rows 64x4x2 978 / 909, 64x4x4 923 / 894.
+    return {64, 4};
   }
   return {lanes, per_lane == 1 ? 8 : (per_lane == 2 ? 4 : 2)};
 }
@@ -259,14 +258,13 @@ SeqFn pick_seq(int nch, int tpg) {
   switch (nch * 10 + tpg) {
     case 18: return seq_gather_kernel<VB, 1, 8>;
     case 24: return seq_gather_kernel<VB, 2, 4>;
-    case 28: return seq_gather_kernel<VB, 2, 8>;
+    case 28: if constexpr (VB == 4) return seq_gather_kernel<VB, 2, 8>; else return nullptr;
     case 32: return seq_gather_kernel<VB, 3, 2>;
-    case 38: return seq_gather_kernel<VB, 3, 8>;
-    case 42: return seq_gather_kernel<VB, 4, 2>;
-    case 82: return seq_gather_kernel<VB, 8, 2>;
     case 34: if constexpr (VB == 4) return seq_gather_kernel<VB, 3, 4>; else return nullptr;
-    case 44: if constexpr (VB == 4) return seq_gather_kernel<VB, 4, 4>; else return nullptr;
-    case 48: if constexpr (VB == 16) return seq_gather_kernel<VB, 4, 8>; else return nullptr;
+    case 38: if constexpr (VB == 4) return seq_gather_kernel<VB, 3, 8>; else return nullptr;
+    case 42: return seq_gather_kernel<VB, 4, 2>;
+    case 44: return seq_gather_kernel<VB, 4, 4>;
+    case 82: return seq_gather_kernel<VB, 8, 2>;
     default: return nullptr;
   }
 }

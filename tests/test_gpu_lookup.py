@@ -373,8 +373,7 @@ def test_seq_gather_lane_group_edges(pdm, dev, dims):
     ((31, 1), 2100, 50), ((47, 1), 2100, 50), ((33,), 9, 50),  # 32, 48: 16 lanes, eight tokens each in large calls
     ((49,), 600, 50), ((63, 1), 600, 50),                     # 49, 64: 32 lanes
     ((129,), 300, 50), ((255, 1), 300, 50),                   # 129, 256: 64 lanes, four tokens each
-    ((196,), 3100, 400_000), ((256,), 3100, 300_000),         # 49, 64 pieces of 16 bytes of tables past 256 MB
-    ((160,), 4100, 450_000), ((1024,), 600, 70_000),          # 40, 256 of them
+    ((772,), 4100, 100_000), ((1024,), 600, 70_000),          # 193, 256 pieces of 16 bytes of tables past 256 MB
 ])
 def test_seq_gather_group_shapes_by_size(pdm, dev, dims, B, rows):
     """The lane groups that depend on the number of tokens and the size of the tables, with a token count that no
