@@ -10,6 +10,11 @@
 namespace pdm {
 
 constexpr int kNsK = 64;  // column granularity of the GEMMs
+// Samples from which a wave walks every part of its sample.  Whole calls in us, four waves per sample / one: 8 tables and 8
+// dense parts (K 152, N 128) 1,024 samples 14.2 / 18.3, 4,096 20.1 / 21.2, 6,000 24.2 / 24.3, 30,000 74 / 69, 262,144 643 /
+// 559; one dense part (K 513, N 128) 15.3 / 15.4, 20.3 / 19.4,
+// 25.0 / 22.4, 56 / 44, 551 / 405; the 4 + 4 parts of K 396, N 256 15.3 / 17.4, 23.1 / 23.8, 28.5 / 28.2, 77 / 70, 676 / 600.
+constexpr int64_t kNsSplitSamples = 5000;
 
 struct NsArgs {
   const char* tables[PDM_NS_MAX_PARTS];
@@ -25,18 +30,20 @@ struct NsArgs {
   uint16_t* w1p;       // [N, K64]
   int32_t N;
   int64_t w1p_elems;  // 0: W1 is read where it is
+  int64_t row_blocks;  // blocks that write rows of raw
+  int32_t split;       // waves per sample: 4 or 1
   int32_t* err;
 };
 
-// Rows of raw and the columns that pad W1, in one launch.  Blocks 0 .. B - 1: one sample each, the parts dealt to the
-// four waves, lanes over a part's columns, bf16 (round to nearest even) out; the samples' id -> row chains run beside
-// each other (1,024 samples of 8 parts: a wave per sample walking every part took 8 us, W1's padding in a launch of its
-// own another 5; together 5 us).  The blocks after them: W1 [N, K] -> [N, K64] with zero columns K .. K64, 4 columns a
-// thread.
+// Rows of raw and the columns that pad W1, in one launch.  The first row_blocks blocks: a sample per `split` waves, which
+// share out its parts, lanes over a part's columns, bf16 (round to nearest even) out.  The blocks after them: W1 [N, K] ->
+// [N, K64] with zero columns K .. K64, 4 columns a thread.  Four waves per sample while the samples leave the card room:
+// the parts' id -> row chains run beside each other (1,024 samples of 8 parts: a wave per sample walking every part took
+// 8 us, W1's padding in a launch of its own another 5; together 5 us).
 __global__ __launch_bounds__(256) void ns_prep_kernel(NsArgs a) {
   const int64_t block = linear_block();
-  if (block >= a.B) {
-    const int64_t i = ((block - a.B) * 256 + threadIdx.x) * 4;
+  if (block >= a.row_blocks) {
+    const int64_t i = ((block - a.row_blocks) * 256 + threadIdx.x) * 4;
     if (i >= a.w1p_elems) return;
     const int n = (int)(i / a.K64), k = (int)(i - (int64_t)n * a.K64);
     const uint16_t* src = a.w1 + (int64_t)n * a.K;
@@ -48,13 +55,16 @@ __global__ __launch_bounds__(256) void ns_prep_kernel(NsArgs a) {
     *reinterpret_cast<u32x2_t*>(a.w1p + i) = u32x2_t{v[0] | v[1] << 16, v[2] | v[3] << 16};
     return;
   }
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  uint16_t* dst = a.raw + block * a.K64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t b = a.split == 4 ? block : block * 4 + wave;
+  const int part0 = a.split == 4 ? wave : 0;
+  if (b >= a.B) return;
+  uint16_t* dst = a.raw + b * a.K64;
   bool bad = false;
-  for (int j = wave; j < a.n_parts; j += 4) {
+  for (int j = part0; j < a.n_parts; j += a.split) {
     const int c0 = a.col[j], w = a.col[j + 1] - c0;
     if (j < a.n_scalar) {
-      const int64_t id = a.ids[j][block];
+      const int64_t id = a.ids[j][b];
       const bool ok = id >= 0 && id < a.rows[j];
       bad |= !ok;
       if (!ok) {
@@ -68,11 +78,11 @@ __global__ __launch_bounds__(256) void ns_prep_kernel(NsArgs a) {
       }
     } else {
       const int d = j - a.n_scalar;
-      const float* row = a.dense[d] + block * a.dense_stride[d];
+      const float* row = a.dense[d] + b * a.dense_stride[d];
       for (int c = lane; c < w; c += 64) dst[c0 + c] = (uint16_t)f32_to_bf16_bits(row[c]);
     }
   }
-  if (wave == 3)
+  if (part0 == a.split - 1)
     for (int c = a.K + lane; c < a.K64; c += 64) dst[c] = 0;
   if (bad && a.err) a.err[0] = 1;
 }
@@ -419,7 +429,9 @@ extern "C" int pdm_ns_tokenize_fwd(const pdm_ns_desc* desc, const void* const* t
   a.w1p = w1p;
   a.N = N;
   a.w1p_elems = pad ? (int64_t)N * K64 : 0;
-  hipLaunchKernelGGL(ns_prep_kernel, linear_grid(d.batch_size + (a.w1p_elems / 4 + 255) / 256), dim3(256), 0, s, a);
+  a.split = d.batch_size < kNsSplitSamples ? 4 : 1;
+  a.row_blocks = a.split == 4 ? d.batch_size : (d.batch_size + 3) / 4;
+  hipLaunchKernelGGL(ns_prep_kernel, linear_grid(a.row_blocks + (a.w1p_elems / 4 + 255) / 256), dim3(256), 0, s, a);
   PDM_CHECK_LAUNCH();
   NsGemmArgs g{};
   g.M = (int)d.batch_size;

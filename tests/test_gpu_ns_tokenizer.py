@@ -94,6 +94,24 @@ def test_ns_tokenize_tile_edges(pdm, dev, B, dense_dims, d, n_ns):
     _check(out.cpu(), tabs, ids, dense, w, n_ns)
 
 
+@pytest.mark.parametrize("B,dtype", [(4999, "bf16"), (5000, "fp32"), (5003, "bf16")])
+def test_ns_tokenize_waves_per_sample(pdm, dev, B, dtype):
+    """Four waves per sample below 5,000 samples, one from there on (the last workgroup partial): narrow and wide parts,
+    one bad id, W1 padded from 175 to 192 columns behind the rows."""
+    scalar, dense_dims, d, n_ns = [(300, 16), (50, 70), (700, 4)], [3, 81, 1], 64, 1
+    g = np.random.default_rng(B)
+    tabs, ids, dense = _parts(g, B, scalar, dense_dims, dtype, bad=True)
+    K = sum(dm for _, dm in scalar) + sum(dense_dims)
+    w = ot.random_autosplit_weights(K, d * n_ns, seed=K)
+    wb = {k: v.to(torch.bfloat16).contiguous().to(dev) for k, v in w.items()}
+    err = torch.zeros(1, dtype=torch.int32, device=dev)
+    out = pdm.ops.ns_tokenize_raw(*_dev(tabs, ids, dense, dev), wb["w1"], wb["b1"], wb["w2"], wb["b2"], n_ns,
+                                  err_flag=err)
+    torch.cuda.synchronize()
+    assert err.item() == 1
+    _check(out.cpu(), tabs, ids, dense, w, n_ns)
+
+
 def test_ns_tokenize_more_samples_than_one_grid_dimension(pdm, dev):
     """2^24 + 5 samples: one block each is more threads than a dimension of a launch holds.  The first and last samples
     and those around each multiple of 2^23 are compared."""
