@@ -418,13 +418,14 @@ static int launch_one(RowProjArgs a, hipStream_t s) {
   PDM_CHECK_HIP(err[dev]);
   // The S tokens behind a sample's last whole block: a block of their own, mostly padding when they are few, or tiles of
   // one token of 128 samples, like the NS tokens, without padding but with 2-byte V^T stores.  Tiles where they are few
-  // enough workgroups: up to 16 tokens of many samples for the FFN-up, 4 for Q/K/V.  Whole blocks of 4,096 samples in
+  // enough workgroups: up to 16 tokens of many samples for the FFN-up, 6 for Q/K/V.  Whole blocks of 4,096 samples in
   // us, blocks / tiles for the FFN-up / tiles for both: d 512, 1 S token 769 / 561 / 464, 4 829 / 648 / 542, 8 925 / 788
-  // / 768, 16 1,764 / 1,659 / 1,674, 28 1,453 / 1,430 / 1,504; Q/K/V alone at d 128: 1 87 / 77, 4 92 / 88, 8 94 / 104.
+  // / 768, 16 1,764 / 1,659 / 1,674, 28 1,453 / 1,430 / 1,504; Q/K/V alone (no NS tokens): d 128, 5 S tokens 73 / 71, 8
+  // 70 / 82; d 384, 5 275 / 233, 8 312 / 303; d 256, 5 158 / 140, 8 155 / 163.
   const int tail = a.n_s % 32, whole = a.n_s - tail;
   a.tiles_b = (a.B + 127) / 128;
   auto blocks = [&](int n) { return ((int64_t)a.B * ((n + 31) / 32) + 3) / 4; };
-  a.n_blk = (int64_t)tail * a.tiles_b * (EPI == ROWPROJ_QKV ? 8 : 2) <= blocks(a.n_s) - blocks(whole) ? whole : a.n_s;
+  a.n_blk = (int64_t)tail * a.tiles_b * (EPI == ROWPROJ_QKV ? 5 : 2) <= blocks(a.n_s) - blocks(whole) ? whole : a.n_s;
   a.blocks_per_sample = (a.n_blk + 31) / 32;
   a.n_tok = a.n_s - a.n_blk + a.n_ns;
   const int64_t wgs_s = blocks(a.n_blk), wgs_tok = (int64_t)a.n_tok * a.tiles_b;

@@ -163,6 +163,8 @@ def test_block_row_projection_edges(pdm, dev, B, kv, q_len, n_ns, D):
     (130, 35, 2, 2, 128),   # one S token behind a whole block, run token by token and not kept as a query
     (130, 36, 3, 2, 256),   # two of them, one kept; the FFN-up's only S token
     (512, 1, 1, 0, 512),    # one S token and no whole block, no NS tokens
+    (512, 40, 8, 2, 128),   # 38 S tokens: the six behind a whole block token by token, all kept
+    (512, 9, 9, 2, 256),    # seven S tokens: a block for Q/K/V, token by token for the FFN-up
     (256, 18, 18, 2, 384),  # 16 S tokens: token by token for the FFN-up, a block for Q/K/V
     (260, 52, 50, 3, 512),  # 49 and 47 S tokens: a whole block and 17 or 15 behind it
 ])
